@@ -7,9 +7,10 @@
 // inference/moe_block.py:704-740: each active expert's projections on its
 // gathered tokens).
 //
-// pf_gemm_kernel<BITS, TM, RT, MODE, SYM, ZF, DEEP>: a workgroup of 4 waves
-// owns TM token rows x (4 * 16 RT) weight rows (MODE gate/up: 4 * 8 RT row
-// indices of the gate AND the up matrix) and a range of K.
+// The MoE block's projections run in the tile form of glq_pf_tile.h.
+// pf_gemm_kernel<BITS, TM, RT, MODE, SYM, ZF, DEEP> takes the dense projection:
+// a workgroup of 4 waves owns TM token rows x (4 * 16 RT) weight rows and a
+// range of K.
 //  * Per 128-code group one LDS slot receives, by direct global->LDS loads,
 //    the TM rows of A (16-byte piece c of slot row r at c ^ (r % 16), so 16
 //    lanes reading one piece of 16 rows hit 16 distinct bank groups), each
@@ -663,6 +664,12 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
   }
 }
 
+}  // namespace glq
+
+#include "glq_pf_tile.h"
+
+namespace glq {
+
 // ---------------------------------------------------------------------------
 // Low-rank a = x U.  A job owns 16 rows of one tile of the list (one expert)
 // and K split sp; its 4 waves take the (matrix, 16-column) tiles of a.  U
@@ -866,29 +873,6 @@ static int pf_launch_k(const PfArgs& g, hipStream_t s) {
   return GLQ_OK;
 }
 
-// Row tiles per wave for a token tile: the accumulators (2 x TM/16 x RT
-// f32x4) and the codes must fit 256 VGPRs (two waves per SIMD).  The dense
-// form (non-integer zero-point path compiled in) takes RT = 2 from 64
-// tokens; the MoE forms RT = 4 below 128.
-constexpr int pf_rt(int mode, int tm) {
-  return tm == 128 ? 2 : (mode == kPfDense && tm == 64 ? 2 : 4);
-}
-
-// The dense form takes any symmetry and non-integer zero-points; the MoE
-// forms asymmetric codes with integer zero-points.
-template <int MODE, bool SYM, bool ZF>
-static int pf_launch_shape(const PfArgs& g, int bits, int tm, hipStream_t s) {
-  constexpr int R64 = pf_rt(MODE, 64);
-  if (bits == 2) {
-    if (tm == 128) return pf_launch_k<2, 128, 2, MODE, SYM, ZF>(g, s);
-    if (tm == 64) return pf_launch_k<2, 64, R64, MODE, SYM, ZF>(g, s);
-    return pf_launch_k<2, 32, 4, MODE, SYM, ZF>(g, s);
-  }
-  if (tm == 128) return pf_launch_k<4, 128, 2, MODE, SYM, ZF>(g, s);
-  if (tm == 64) return pf_launch_k<4, 64, R64, MODE, SYM, ZF>(g, s);
-  return pf_launch_k<4, 32, 4, MODE, SYM, ZF>(g, s);
-}
-
 // Tile of a dense launch: TM token rows x 64 RT weight rows, ring depth.
 struct PfTile {
   int tm, rt;
@@ -922,10 +906,23 @@ static int pf_launch_dense(const PfArgs& g, int bits, PfTile t, bool sym, hipStr
              : pf_launch_dense_bits<4, false, true>(g, t, s);
 }
 
-// Weight rows per workgroup for a token tile.
-static int pf_wg_rows_rt(int mode, int tm) {
-  const int rt = pf_rt(mode, tm);
-  return mode == kPfGateUp ? 4 * 8 * rt : 4 * 16 * rt;
+// Weight rows of a workgroup of the tile form (glq_pf_tile.h) of tm = 32, 64
+// (x 256 rows) or 128 (x 128 rows) tokens; a gate/up tile holds half as many
+// rows of each matrix.
+static int pt_wg_rows(int mode, int tm) {
+  const int r = tm == 128 ? 128 : 256;
+  return mode == kPfGateUp ? r / 2 : r;
+}
+static int pt_tiles_n(int64_t N, int mode, int tm) {
+  const int r = pt_wg_rows(mode, tm);
+  return (int)((N + r - 1) / r);
+}
+
+template <int MODE, bool SYM, bool ZF>
+static int pt_launch_tm(const PfArgs& g, int bits, int tm, hipStream_t s) {
+  if (tm == 128) return pt_launch<2, 2, 2, MODE, SYM, ZF>(g, bits, s);
+  if (tm == 64) return pt_launch<1, 4, 2, MODE, SYM, ZF>(g, bits, s);
+  return pt_launch<1, 4, 1, MODE, SYM, ZF>(g, bits, s);
 }
 
 static size_t pf_lowrank_lds(int nmat, int rank) {
@@ -1388,7 +1385,12 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
   PfMoePlan P;
   const int64_t Pn = T * k;
   const int64_t avg = Pn / std::max<int64_t>(E, 1);
-  P.tm = avg >= 96 ? 128 : (avg >= 32 ? 64 : 32);
+  // Token tile by the mean tokens an expert gets: 128 tokens where most experts
+  // fill one such tile and overflow a 64-token one, 64 above, 32 where most
+  // of a 64-token tile would be empty.  Whole blocks at 32 / 64 / 128: 19
+  // tokens an expert 293 / 336 / 458 us, 47: 382 / 363 / 421, 50: 361 / 385 /
+  // 393, 94: 594 / 577 / 566, 128: 716 / 649 / 671, 250: 1183 / 1036 / 1053.
+  P.tm = avg < 46 ? 32 : (avg >= 80 && avg < 112 ? 128 : 64);
   if (const char* e = getenv("GLQ_PF_MOE_TM")) {
     const int v = atoi(e);
     P.tm = v >= 128 ? 128 : (v >= 64 ? 64 : 32);
@@ -1396,7 +1398,7 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
   P.max_tiles = (int)((Pn + P.tm - 1) / P.tm + E);
   pf_lowrank_split(H, P.ks_gu, P.kps_gu);
   pf_lowrank_split(I, P.ks_d, P.kps_d);
-  P.stm = T >= 512 ? 128 : (T > 32 ? 64 : 32);
+  P.stm = T > 32 ? 64 : 32;
   int64_t o = 0;
   auto take = [&](int64_t bytes) {
     const int64_t at = o;
@@ -1577,11 +1579,11 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     g.ntiles = a.ntiles;
     g.M = (int)Pn; g.K = (int)H; g.N = (int)I; g.G = (int)(H / 128);
     g.kw = (int)kw_gu; g.rank = r;
-    g.ntn = (int)((I + pf_wg_rows_rt(kPfGateUp, P.tm) - 1) / pf_wg_rows_rt(kPfGateUp, P.tm));
+    g.ntn = pt_tiles_n(I, kPfGateUp, P.tm);
     g.ks = 1; g.gps = g.G;
     g.out_bits = p->bits;
     g.max_tiles = P.max_tiles;
-    rc = pf_launch_shape<kPfGateUp, false, false>(g, p->bits, P.tm, s);
+    rc = pt_launch_tm<kPfGateUp, false, false>(g, p->bits, P.tm, s);
     if (rc) return rc;
   }
   // 5. a = inter U_down per pair
@@ -1625,10 +1627,10 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     g.ntiles = a.ntiles;
     g.M = (int)Pn; g.K = (int)I; g.N = (int)H; g.G = (int)(I / 128);
     g.kw = (int)kw_d; g.rank = r;
-    g.ntn = (int)((H + pf_wg_rows_rt(kPfDown, P.tm) - 1) / pf_wg_rows_rt(kPfDown, P.tm));
+    g.ntn = pt_tiles_n(H, kPfDown, P.tm);
     g.ks = 1; g.gps = g.G;
     g.max_tiles = P.max_tiles;
-    rc = pf_launch_shape<kPfDown, false, false>(g, p->bits, P.tm, s);
+    rc = pt_launch_tm<kPfDown, false, false>(g, p->bits, P.tm, s);
     if (rc) return rc;
   }
   // 7. shared expert over every token
@@ -1647,11 +1649,11 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     g.y_ld = SI;
     g.M = (int)T; g.K = (int)H; g.N = (int)SI; g.G = (int)(H / 128);
     g.kw = (int)(H * sb / 32);
-    g.ntn = (int)((SI + pf_wg_rows_rt(kPfGateUp, P.stm) - 1) / pf_wg_rows_rt(kPfGateUp, P.stm));
+    g.ntn = pt_tiles_n(SI, kPfGateUp, P.stm);
     g.ks = 1; g.gps = g.G;
     g.out_bits = sb;
     g.max_tiles = ntm;
-    rc = pf_launch_shape<kPfGateUp, false, false>(g, sb, P.stm, s);
+    rc = pt_launch_tm<kPfGateUp, false, false>(g, sb, P.stm, s);
     if (rc) return rc;
     PfArgs d = {};
     d.xp = sinter;
@@ -1662,10 +1664,10 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     d.yf_ld = H;
     d.M = (int)T; d.K = (int)SI; d.N = (int)H; d.G = (int)(SI / 128);
     d.kw = (int)(SI * sb / 32);
-    d.ntn = (int)((H + pf_wg_rows_rt(kPfDown, P.stm) - 1) / pf_wg_rows_rt(kPfDown, P.stm));
+    d.ntn = pt_tiles_n(H, kPfDown, P.stm);
     d.ks = 1; d.gps = d.G;
     d.max_tiles = ntm;
-    rc = pf_launch_shape<kPfDown, false, false>(d, sb, P.stm, s);
+    rc = pt_launch_tm<kPfDown, false, false>(d, sb, P.stm, s);
     if (rc) return rc;
   }
   // 8. combine

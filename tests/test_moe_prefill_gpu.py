@@ -141,3 +141,24 @@ def test_non_integer_shared_zeros_use_decode_steps(gpu):
     out, logits = blk(p.h.reshape(1, 100, p.H).to(gpu))
     torch.cuda.synchronize()
     check(p, out.reshape(100, p.H).cpu(), logits.cpu(), "non-integer shared zeros")
+
+
+@pytest.mark.parametrize("T,E,top_k,H,inter,bits", [
+    (65, 8, 2, 512, 1024, 2),    # 16 tokens an expert: 32-token tiles, scale quads
+    (65, 1, 1, 128, 128, 2),     # one expert, one group, one row block
+    (129, 4, 2, 512, 640, 4),    # 64 an expert (64-token tiles), 8 and 5 groups, 4-bit
+    (160, 4, 2, 1280, 512, 2),   # 80 an expert (128-token tiles), 10 and 4 groups
+    (257, 2, 2, 640, 1024, 2),   # 257 rows on every expert: five 64-token tiles, one row over
+], ids=str)
+def test_prefill_tile_edges(gpu, T, E, top_k, H, inter, bits):
+    """The tile form's token tiles (by the mean tokens an expert gets) at their
+    edges: ragged last tiles, groups loaded one and four at a time, row blocks
+    past the projection's rows."""
+    args = dict(H=H, E=E, inter=inter, top_k=top_k, n_clusters=2, rank=24, shared_inter=256,
+                bits=bits)
+    seed = 10
+    if E > top_k:  # the first seed whose routing has no near-tie
+        seed = next(s for s in range(10, 60) if margin(fmt.make_moe(B=T, seed=s, **args)) >= 2)
+    p = lora_heavy(fmt.make_moe(B=T, seed=seed, **args))
+    _, out, logits = run(p, gpu)
+    check(p, out, logits, str((T, E, top_k, H, inter, bits)))
