@@ -48,6 +48,7 @@
 #include <cstdio>
 
 #include "glq_handoff.h"
+#include "glq_moe_route.h"
 #include "glq_stream.h"
 
 namespace glq {
@@ -671,16 +672,21 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
 namespace glq {
 
 // ---------------------------------------------------------------------------
-// Low-rank a = x U.  A job owns 16 rows of one tile of the list (one expert)
-// and K split sp; its 4 waves take the (matrix, 16-column) tiles of a.  U
-// chunks of 128 k (every matrix m) are staged in LDS in their natural (k,
-// rank) layout by 16-byte pieces; a lane forms its B operand (8 consecutive k
-// of one rank column, in A's order: natural, or the decode order of aperm
-// bits) from 8 two-byte LDS reads.  The fp32 partial sums of each split go to
-// part (ks, rows, nmat * rank); the GEMM epilogue sums them in split order and
-// rounds a to fp16 once.  The dense launch also runs, in its first
-// workgroups, the prep of the GEMM's A: x in decode order and its per-group
-// sums (one thread per (row, group)).
+// Low-rank a = x U over a tile list (one expert's rows a tile) or all rows.
+// Workgroup (64-row block, K slice, block of four 32-column tiles of the
+// matrices' a): per 128 codes, the rows of x come to LDS by buffer loads (two
+// slots, 16-byte piece c of row r at c ^ (r % 16)) and U's rows through
+// registers (the next chunk's are loaded while this one's are multiplied),
+// written transposed and in A's code order as pairs (two rows' halves of a
+// column in one word), so both MFMA operands are one 16-byte LDS read.  Row
+// col of the transposed U is 16 pieces of 8 codes, piece c at c ^ pf_ut_sw(col):
+// the reads' 16 columns and the writes' 8 columns x 8 pairs fall on distinct
+// banks.  The four waves take the column tiles, and the block's two 32-row
+// halves where there are fewer.
+//
+// A 16-row block with U in its natural layout (two-byte LDS reads of every B
+// operand, U read again for every 16 rows) took 100 us a launch for 12000
+// rows x (2048 -> 2 x 64) and 43 us for 1024 rows x (4096 -> 2 x 64).
 // ---------------------------------------------------------------------------
 struct PfLowrank {
   const __half* x;         // A rows, K halves each
@@ -692,7 +698,7 @@ struct PfLowrank {
   const int32_t* uslot[2];    // cluster -> row of U[m] (a cross-layer pool), or null
   const int32_t* tiles;    // tile list of the GEMM (null: dense)
   const int32_t* ntiles;
-  int tile_rows;           // rows per tile of the list (dense: 16)
+  int tile_rows;           // rows per tile of the list
   int nmat, rows_total, K, rank, ks, kps;
   float* part;             // (ks, rows_total, nmat * rank) fp32 partial sums of a (ks > 1)
   __half* a_out;           // (rows_total, nmat * rank) a = fp16(x U) (ks == 1, or finalized)
@@ -700,22 +706,23 @@ struct PfLowrank {
   int n_cnt;
 };
 
-constexpr int kLrRows = 16;  // rows per lowrank workgroup (one 16-row MFMA tile)
+constexpr int kLrRows = 64;  // rows per low-rank workgroup
+constexpr int kLrLds = 128 * 256 + 2 * kLrRows * 256;
 
+__device__ __forceinline__ int pf_ut_sw(int col) { return (col ^ (col >> 3)) & 15; }
 
-// One (16 rows, K split) job of a = x U: fp32 partial sums into
-// part[sp][row][m * rank + j].  A rows (16 x 128 codes) and U (128 x rank of
-// every matrix) reach LDS by direct global->LDS loads in a ring of two
-// slots, 16-byte pieces swizzled so the operand reads spread over the banks:
-// A piece p of row i at p ^ i, U piece j8 of row k at j8 ^ ((k / 8) % (rank / 8))
-// (power-of-two ranks; others unswizzled).
-__device__ void pf_lowrank_job(const PfLowrank& L, int job, int sp, unsigned char* smem) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, kb = lane >> 4;
-  const int sub = L.tile_rows / kLrRows;  // lowrank jobs per tile
-  const int ti = job / sub, part = job % sub;
+__device__ __forceinline__ void pf_lowrank_body(const PfLowrank& L, unsigned char* smem) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, h = lane >> 5;
+  if (L.zero_cnt && blockIdx.x + blockIdx.y + blockIdx.z == 0)
+    for (int i = tid; i < L.n_cnt; i += kPfThreads) L.zero_cnt[i] = 0u;
+  if (L.nmat == 0) return;  // the counters were all there was to do
+  const int job = blockIdx.x, sp = blockIdx.y, cb = blockIdx.z;
   int e = 0, p0, rows;
   if (L.tiles) {
+    const int sub = (L.tile_rows + kLrRows - 1) / kLrRows;  // row blocks per tile
+    const int ti = job / sub, part = job % sub;
     if (ti >= *L.ntiles) return;  // uniform over the workgroup
     e = L.tiles[3 * ti];
     p0 = L.tiles[3 * ti + 1] + part * kLrRows;
@@ -726,90 +733,125 @@ __device__ void pf_lowrank_job(const PfLowrank& L, int job, int sp, unsigned cha
   }
   if (rows <= 0) return;
   const int k0 = sp * L.kps, k1 = min(L.K, k0 + L.kps);
-  const int r = L.rank, r8 = r / 8, nct = (r + 15) / 16;
-  const int sw = (r8 & (r8 - 1)) == 0 ? r8 - 1 : 0;  // piece swizzle mask (power-of-two ranks)
-  const int jobs = L.nmat * nct;  // (matrix, column tile)
-  const int ub = 128 * r * 2;     // bytes of one matrix's U chunk
-  const int slot_bytes = 4096 + L.nmat * ub;
+  const int r = L.rank, ctm = (r + 31) / 32;        // column tiles per matrix
+  const int nct = min(4, L.nmat * ctm - 4 * cb);    // this block's
+  const int wct = nct <= 2 ? nct : 4, ct = wave % wct, mg = wave / wct, mw = 4 / wct;
+  unsigned char* ut = smem;
+  unsigned char* as = smem + 128 * 256;
   const __half* U[2];
+#pragma unroll
   for (int m = 0; m < 2; ++m) {
     int c = (m < L.nmat && L.cluster[m]) ? L.cluster[m][e] : 0;
     if (m < L.nmat && L.uslot[m]) c = L.uslot[m][c];
     U[m] = m < L.nmat ? L.U[m] + (int64_t)c * L.u_cs : nullptr;
   }
-  // A: wave w loads rows 4w..4w+3 (one instruction), lane -> (row, piece)
-  const int arr = 4 * wave + (lane >> 4);
-  const int apr = p0 + min(arr, rows - 1);
-  const __half* asrc = L.x + (int64_t)(L.arow ? L.arow[apr] : apr) * L.K + 8 * ((lane & 15) ^ arr);
-  const int nu = L.nmat * 128 * r8 / 64;  // U load instructions per workgroup
-  auto issue = [&](int kc, unsigned char* slot) {
-    __builtin_amdgcn_global_load_lds((const void*)(asrc + kc), (lds_void*)(slot + wave * 1024), 16,
-                                     0, 0);
-    for (int q = wave; q < nu; q += 4) {  // uniform over the wave
-      const int pidx = q * 64 + lane;     // piece index over [m][k][pos]
-      const int m = pidx / (128 * r8), rem = pidx - m * 128 * r8;
-      const int k = rem / r8, pos = rem - k * r8;
-      const int j8 = pos ^ ((k >> 3) & sw);
-      const int kk = min(kc + k, L.K - 1);
-      __builtin_amdgcn_global_load_lds((const void*)(U[m] + (int64_t)kk * r + 8 * j8),
-                                       (lds_void*)(slot + 4096 + q * 1024), 16, 0, 0);
+  // A: instruction q of the wave loads rows 4 (4 wave + q) .. + 3
+  unsigned aoff[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int ar = (4 * wave + q) * 4 + (lane >> 4);
+    const int p = p0 + min(ar, rows - 1);
+    const unsigned src = L.arow ? L.arow[p] : p;
+    aoff[q] = 2u * (src * (unsigned)L.K + 8 * ((lane & 15) ^ (ar & 15)));
+  }
+  const auto ars = pt_rsrc(L.x);
+  auto issue_a = [&](int kc, unsigned char* slot) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (lds_void*)(slot + (4 * wave + q) * 1024), 16,
+                                               aoff[q], kc * 2, 0, 0);
+  };
+  // U: item q of the thread is the pair of rows at A positions (2 pk, 2 pk + 1)
+  // of the chunk x 8 columns
+  const __half* us[4];
+  int dk[4], wpos[4], wcol[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int idx = tid + kPfThreads * q;
+    const int c8 = (idx & 7) + 8 * (idx >> 9), pk = (idx >> 3) & 63;
+    const int gt = 4 * cb + (c8 >> 2);
+    const int m = gt >= ctm ? 1 : 0, j0 = (gt - m * ctm) * 32 + (c8 & 3) * 8;
+    int k;  // natural code of position 2 pk; position 2 pk + 1 is dk further
+    if (L.aperm == 2) { k = 16 * (pk >> 3) + (pk & 7); dk[q] = 8; }
+    else if (L.aperm == 4) { k = 8 * (pk >> 2) + (pk & 3); dk[q] = 4; }
+    else { k = 2 * pk; dk[q] = 1; }
+    us[q] = c8 < 4 * nct && j0 < r ? (m ? U[1] : U[0]) + (int64_t)k * r + j0 : nullptr;
+    wcol[q] = c8 < 4 * nct ? 8 * c8 : -1;
+    wpos[q] = pk;
+  }
+  u32x4 ua[4], ub[4];
+  auto load_u = [&](int kc) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      ua[q] = ub[q] = u32x4{0u, 0u, 0u, 0u};
+      if (us[q]) {
+        ua[q] = *(const u32x4*)(us[q] + (int64_t)kc * r);
+        ub[q] = *(const u32x4*)(us[q] + (int64_t)(kc + dk[q]) * r);
+      }
     }
   };
-  constexpr int MJ = 8;  // jobs per wave (nmat * rank / 16 <= 32)
-  f32x4 acc[MJ];
-#pragma unroll
-  for (int q = 0; q < MJ; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-  issue(k0, smem);
+  f32x16 acc[2] = {};
+  issue_a(k0, as);
+  load_u(k0);
   int s = 0;
   for (int kc = k0; kc < k1; kc += 128) {
-    wait_vmcnt<0>();
-    asm volatile("s_barrier" ::: "memory");
-    if (kc + 128 < k1) issue(kc + 128, smem + (s ^ 1) * slot_bytes);
-    const unsigned char* sl = smem + s * slot_bytes;
-    const int kl = min(128, k1 - kc);
-    for (int ks = 0; ks < kl; ks += 32) {
-      const f16x8 av = *(const f16x8*)(sl + li * 256 + 16 * (((ks >> 3) + kb) ^ li));
+    __syncthreads();  // the chunk before has been read
 #pragma unroll
-      for (int q = 0; q < MJ; ++q) {
-        const int jb = wave + 4 * q;
-        if (jb >= jobs) break;  // uniform over the wave
-        const int m = jb / nct, ct = jb - m * nct;
-        const int j = min(ct * 16 + li, r - 1);
-        const __half* um = (const __half*)(sl + 4096 + m * ub);
-        f16x8 bv;
+    for (int q = 0; q < 4; ++q) {
+      if (wcol[q] < 0) continue;
+      const uint32_t a[4] = {ua[q].x, ua[q].y, ua[q].z, ua[q].w};
+      const uint32_t b[4] = {ub[q].x, ub[q].y, ub[q].z, ub[q].w};
 #pragma unroll
-        for (int q8 = 0; q8 < 8; ++q8) {
-          int k = ks + 8 * kb + q8;
-          if (L.aperm) {  // position k of A holds natural index perm_src(k)
-            const int p = k & 15;
-            k = (k & ~15) + (L.aperm == 2 ? perm_src<2>(p) : perm_src<4>(p));
+      for (int c = 0; c < 8; ++c) {
+        const int col = wcol[q] + c;
+        const uint32_t v = __builtin_amdgcn_perm(b[c >> 1], a[c >> 1],
+                                                 c & 1 ? 0x07060302u : 0x05040100u);
+        *(uint32_t*)(ut + col * 256 + (((wpos[q] >> 2) ^ pf_ut_sw(col)) << 4) +
+                     4 * (wpos[q] & 3)) = v;
+      }
+    }
+    wait_vmcnt<0>();  // this chunk's A
+    __syncthreads();
+    if (kc + 128 < k1) {  // uniform
+      issue_a(kc + 128, as + (s ^ 1) * kLrRows * 256);
+      load_u(kc + 128);
+    }
+    const unsigned char* sl = as + s * kLrRows * 256;
+    const int col = ct * 32 + li;
+    if (ct < nct) {  // uniform over the wave
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const f16x8 bv = *(const f16x8*)(ut + col * 256 + (((8 * h + t) ^ pf_ut_sw(col)) << 4));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int mb = mg + i * mw;  // 32-row half
+          if (mb < 2) {                // uniform over the wave
+            const int row = 32 * mb + li;
+            const f16x8 av = *(const f16x8*)(sl + row * 256 + (((8 * h + t) ^ (row & 15)) << 4));
+            acc[i] = mfma_32x32x16(av, bv, acc[i]);
           }
-          const int pos = (j >> 3) ^ ((k >> 3) & sw);
-          const __half hv = um[k * r + 8 * pos + (j & 7)];
-          bv[q8] = (_Float16)__half2float(hv);
         }
-        acc[q] = mfma_16x16x32(av, bv, acc[q]);
       }
     }
     s ^= 1;
   }
-  // acc[q][i]: row 4kb + i of the tile, rank column ct*16 + li
+  // acc[i][q]: row 8 (q / 4) + 4 h + q % 4 of 32-row half mg + i mw, column li
+  if (ct >= nct) return;
+  const int gt = 4 * cb + ct, m = gt >= ctm ? 1 : 0, j = (gt - m * ctm) * 32 + li;
+  if (j >= r) return;
   const int ld = L.nmat * r;
   float* out = L.part + (int64_t)sp * L.rows_total * ld;
 #pragma unroll
-  for (int q = 0; q < MJ; ++q) {
-    const int jb = wave + 4 * q;
-    if (jb >= jobs) break;
-    const int m = jb / nct, ct = jb - m * nct;
-    const int j = ct * 16 + li;
-    if (j >= r) continue;
+  for (int i = 0; i < 2; ++i) {
+    const int mb = mg + i * mw;
+    if (mb >= 2) continue;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int rr = 4 * kb + i;
+    for (int q = 0; q < 16; ++q) {
+      const int rr = 32 * mb + 8 * (q >> 2) + 4 * h + (q & 3);
       if (rr < rows) {
         const int64_t o = (int64_t)(p0 + rr) * ld + m * r + j;
-        if (L.ks == 1) L.a_out[o] = __float2half(acc[q][i]);
-        else out[o] = acc[q][i];
+        if (L.ks == 1) L.a_out[o] = __float2half(acc[i][q]);
+        else out[o] = acc[i][q];
       }
     }
   }
@@ -845,14 +887,10 @@ __global__ __launch_bounds__(256) void pf_xu_kernel(const __half* __restrict__ x
   if (tid == 0) handoff_reset(cnt + rb);
 }
 
-// Grid: n_jobs * ks lowrank jobs.
+// Grid: (row blocks, K splits, column blocks).
 __global__ __launch_bounds__(kPfThreads) void pf_lowrank_kernel(PfLowrank L) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if (L.zero_cnt && blockIdx.x == 0)
-    for (int i = threadIdx.x; i < L.n_cnt; i += kPfThreads) L.zero_cnt[i] = 0u;
-  if (L.nmat == 0) return;  // the counters were all there was to do
-  const int j = blockIdx.x;
-  pf_lowrank_job(L, j / L.ks, j % L.ks, smem);
+  pf_lowrank_body(L, smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -925,47 +963,59 @@ static int pt_launch_tm(const PfArgs& g, int bits, int tm, hipStream_t s) {
   return pt_launch<1, 4, 1, MODE, SYM, ZF>(g, bits, s);
 }
 
-static size_t pf_lowrank_lds(int nmat, int rank) {
-  return 2 * (4096 + (size_t)nmat * 128 * rank * 2);
-}
-
-// a = fp16(sum of the K-split partials in split order): one thread per element.
+// a = fp16(sum of the K-split partials in split order): four elements a thread
+// (n is a multiple of 8).
 __global__ __launch_bounds__(256) void pf_lowrank_finalize_kernel(const float* part, int ks,
                                                                   int64_t n, __half* a) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
   if (i >= n) return;
-  float s = 0.f;
-  for (int q = 0; q < ks; ++q) s += part[q * n + i];
-  a[i] = __float2half(s);
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int q0 = 0; q0 < ks; q0 += 4) {
+    float4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = *(const float4*)(part + min(q0 + u, ks - 1) * n + i);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (q0 + u < ks) {
+        s[0] += v[u].x;
+        s[1] += v[u].y;
+        s[2] += v[u].z;
+        s[3] += v[u].w;
+      }
+  }
+  uint16_t o[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) o[u] = __half_as_ushort(__float2half(s[u]));
+  *(u32x2*)(a + i) = u32x2{o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16};
 }
 
-// n_jobs: 16-row lowrank jobs (times L.ks splits); with none, one workgroup
-// still clears L.zero_cnt.
+// n_jobs: 64-row blocks; with no matrix, one workgroup still clears L.zero_cnt.
 static int pf_lowrank_launch(const PfLowrank& L, int n_jobs, hipStream_t s) {
+  if (L.nmat == 0) n_jobs = L.zero_cnt ? 1 : 0;
+  if (n_jobs == 0) return GLQ_OK;
+  const int ctm = (L.rank + 31) / 32;
+  const dim3 grid((unsigned)n_jobs, (unsigned)(L.nmat ? L.ks : 1),
+                  (unsigned)(L.nmat ? (L.nmat * ctm + 3) / 4 : 1));
   static size_t attr = 64 * 1024;
-  const size_t lds = L.nmat > 0 ? pf_lowrank_lds(L.nmat, L.rank) : 0;
-  int rc = set_lds_limit(pf_lowrank_kernel, lds, attr);
+  int rc = set_lds_limit(pf_lowrank_kernel, (size_t)kLrLds, attr);
   if (rc) return rc;
-  int64_t grid = L.nmat > 0 ? (int64_t)n_jobs * L.ks : 0;
-  if (grid == 0 && L.zero_cnt) grid = 1;  // the job index is past the list: no job
-  if (grid == 0) return GLQ_OK;
-  GLQ_CHECK(grid < (1ll << 31), "too many workgroups");
-  pf_lowrank_kernel<<<dim3((unsigned)grid), dim3(kPfThreads), lds, s>>>(L);
+  pf_lowrank_kernel<<<grid, dim3(kPfThreads), kLrLds, s>>>(L);
   GLQ_LAUNCH_CHECK("pf_lowrank_kernel");
   if (L.nmat > 0 && L.ks > 1) {
     const int64_t n = (int64_t)L.rows_total * L.nmat * L.rank;
-    pf_lowrank_finalize_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(
+    pf_lowrank_finalize_kernel<<<dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s>>>(
         L.part, L.ks, n, L.a_out);
     GLQ_LAUNCH_CHECK("pf_lowrank_finalize_kernel");
   }
   return GLQ_OK;
 }
 
-// K split of a = x U: splits of 512 codes (more for K > 8192: at most 16
-// splits), summed by pf_lowrank_finalize_kernel.
-static void pf_lowrank_split(int64_t K, int& ks, int& kps) {
-  int64_t per = std::max<int64_t>(512, (K + 15) / 16);
-  per = (per + 127) / 128 * 128;
+// K split of a = x U for `blocks` workgroups a split: enough splits for about
+// 512 workgroups (two on each CU), at most 16, each of at least 256 codes.
+static void pf_lowrank_split(int64_t K, int64_t blocks, int& ks, int& kps) {
+  int64_t n = std::max<int64_t>(1, std::min<int64_t>(16, 512 / std::max<int64_t>(blocks, 1)));
+  n = std::max<int64_t>(1, std::min<int64_t>(n, K / 256));
+  const int64_t per = ((K + n - 1) / n + 127) / 128 * 128;
   kps = (int)per;
   ks = (int)((K + per - 1) / per);
 }
@@ -1029,7 +1079,7 @@ static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, 
   if (const char* e = getenv("GLQ_PF_KS")) ks = std::max(1, std::min(G, atoi(e)));
   P.gps = (G + ks - 1) / ks;
   P.ks = (G + P.gps - 1) / P.gps;
-  pf_lowrank_split(K, P.lr_ks, P.lr_kps);
+  pf_lowrank_split(K, (M + kLrRows - 1) / kLrRows, P.lr_ks, P.lr_kps);
   P.a_bytes = rank > 0 ? align_up(M * rank * 2, 256) : 0;
   // a = x U in one launch (16-row blocks x K slices, last arrivers sum) when
   // the GEMM needs no split-K counters (those are cleared by the two-launch
@@ -1206,99 +1256,161 @@ struct PfMoe {
   __half* out;             // (T, H)
 };
 
+// Largest of the wave's 64 unsigned values, on every lane.
+__device__ __forceinline__ uint32_t pf_wave_max(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, false));
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = max(r[0], r[1]);
+  const auto q = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return max(q[0], q[1]);
+}
+
+// 16 halves of a code block in the decode order of bits (perm_src): pairs
+// (c, c + 8) at 2 bits, (c, c + 4) of each 8 at 4.
+__device__ __forceinline__ void pf_permute16(int bits, u32x4 lo, u32x4 hi, u32x4& o0, u32x4& o1) {
+  const uint32_t l[4] = {lo.x, lo.y, lo.z, lo.w}, g[4] = {hi.x, hi.y, hi.z, hi.w};
+  uint32_t o[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t sel = i & 1 ? 0x07060302u : 0x05040100u;
+    if (bits == 2) o[i] = __builtin_amdgcn_perm(g[i >> 1], l[i >> 1], sel);
+    else o[i] = i < 4 ? __builtin_amdgcn_perm(l[2 + (i >> 1)], l[i >> 1], sel)
+                      : __builtin_amdgcn_perm(g[2 + ((i - 4) >> 1)], g[(i - 4) >> 1], sel);
+  }
+  o0 = u32x4{o[0], o[1], o[2], o[3]};
+  o1 = u32x4{o[4], o[5], o[6], o[7]};
+}
+
+// Rows t0 .. t0 + 15 of x in the routed experts' decode order (and in the
+// shared expert's when it differs), by 512 threads, four blocks in flight.
+__device__ __forceinline__ void pf_permute_rows(const PfMoe& a, int t0, int tid) {
+  const int nb = a.H / 16, n = min(16, a.T - t0) * nb;  // 16-half blocks
+  const __half* src = a.h + (int64_t)t0 * a.H;
+  for (int i0 = tid; i0 < n; i0 += 4 * 512) {
+    u32x4 v[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const __half* p = src + 16 * (int64_t)min(i0 + 512 * u, n - 1);
+      v[u][0] = *(const u32x4*)p;
+      v[u][1] = *(const u32x4*)(p + 8);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + 512 * u;
+      if (i >= n) continue;
+      u32x4 o0, o1;
+      const int64_t at = (int64_t)t0 * a.H + 16 * (int64_t)i;
+      pf_permute16(a.bits, v[u][0], v[u][1], o0, o1);
+      *(u32x4*)(a.xp + at) = o0;
+      *(u32x4*)(a.xp + at + 8) = o1;
+      if (a.xps && a.xps != a.xp) {
+        pf_permute16(a.sbits, v[u][0], v[u][1], o0, o1);
+        *(u32x4*)(a.xps + at) = o0;
+        *(u32x4*)(a.xps + at + 8) = o1;
+      }
+    }
+  }
+}
+
 // One workgroup per 16 tokens: logits of every router row (MFMA tiles of 16
-// rows, K split over the waves, partial tiles summed in LDS in wave order),
-// then per token (one wave) softmax, top-k with ties to the lower index,
-// weights, and the rows of x in decode order.
-__global__ __launch_bounds__(256) void pf_moe_route_kernel(PfMoe a) {
-  __shared__ float red[4][16][17];  // per wave partial logits of one 16-row tile
-  __shared__ float lg[16][257];     // fp16-rounded logits (as float) of the 16 tokens
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// rows, K split over four of the eight waves, partial tiles summed in LDS in
+// wave order), then per token (one wave) softmax, top-k with ties to the
+// lower index and weights.  A second workgroup a block writes the rows of x
+// in decode order meanwhile.
+//
+// It is a chain of memory round trips and of cross-lane steps: each wave
+// holds every other router tile (NT of them) and loads two to eight K steps
+// of them and of x at once, and an argmax is one key (moe_key) through DPP and
+// permlane steps.  A tile at a time, a K step at a time and value and index
+// through LDS shuffles, it took 107 us at 1500 tokens x 128 experts, 51 us at
+// 512 x 8 over 4096 columns.
+template <int NT>
+__global__ __launch_bounds__(512) void pf_moe_route_kernel(PfMoe a) {
+  __shared__ float red[2][4][16][17];  // per wave partial logits of one 16-row tile
+  __shared__ float lg[16][257];        // fp16-rounded logits (as float) of the 16 tokens
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, kb = lane >> 4;
+  const int kw = wave & 3, par = wave >> 2;  // K quarter, tile parity
   const int t0 = blockIdx.x * 16;
-  const int nrow = a.E + (a.sgw ? 1 : 0), ntile = (nrow + 15) / 16;
+  if (blockIdx.y) {  // uniform: the rows of x in decode order
+    pf_permute_rows(a, t0, tid);
+    return;
+  }
+  const int nrow = a.E + (a.sgw ? 1 : 0);
   const int ta = min(t0 + li, a.T - 1);
   const int nks = a.H / 32;
-  for (int tile = 0; tile < ntile; ++tile) {
-    const int row = tile * 16 + li;
-    const __half* wr = row < a.E ? a.router_w + (int64_t)row * a.H
-                                 : (row == a.E && a.sgw ? a.sgw : nullptr);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int ks = wave; ks < nks; ks += 4) {
-      const f16x8 av = *(const f16x8*)(a.h + (int64_t)ta * a.H + 32 * ks + 8 * kb);
-      const f16x8 bv = wr ? *(const f16x8*)(wr + 32 * ks + 8 * kb) : f16x8{};
-      acc = mfma_16x16x32(av, bv, acc);
-    }
-    // acc[i]: token 4kb + i, router row li of the tile
+  {
+    const __half* xr = a.h + (int64_t)ta * a.H + 8 * kb;
+    const __half* wr[NT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][4 * kb + i][li] = acc[i];
-    __syncthreads();
-    {
-      const int t = tid >> 4, c = tid & 15;
-      const float s = red[0][t][c] + red[1][t][c] + red[2][t][c] + red[3][t][c];
-      if (tile * 16 + c < nrow) lg[t][tile * 16 + c] = __half2float(__float2half(s));
+    for (int i = 0; i < NT; ++i) {
+      const int row = (2 * i + par) * 16 + li;
+      wr[i] = row < a.E ? a.router_w + (int64_t)row * a.H + 8 * kb
+                        : (row == a.E && a.sgw ? a.sgw + 8 * kb : nullptr);
     }
-    __syncthreads();
-  }
-  // x rows in decode order (and in the shared expert's when it differs)
-  for (int idx = tid; idx < 16 * (a.H / 16); idx += 256) {
-    const int t = idx / (a.H / 16), blk = idx - t * (a.H / 16);
-    if (t0 + t >= a.T) continue;
-    const __half* src = a.h + (int64_t)(t0 + t) * a.H + 16 * blk;
-    const f16x8 a0 = *(const f16x8*)src, a1 = *(const f16x8*)(src + 8);
-    _Float16 in[16];
+    f32x4 acc[NT] = {};
+    constexpr int U = NT <= 2 ? 8 : NT <= 4 ? 4 : 2;  // K steps loaded at once
+    for (int k0 = kw; k0 < nks; k0 += 4 * U) {
+      f16x8 av[U], bv[U][NT];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      in[c] = a0[c];
-      in[8 + c] = a1[c];
-    }
-    for (int which = 0; which < 2; ++which) {
-      const int bits = which == 0 ? a.bits : a.sbits;
-      __half* dstb = which == 0 ? a.xp : a.xps;
-      if (which == 1 && (dstb == nullptr || dstb == a.xp)) break;
-      f16x8 o0, o1;
+      for (int u = 0; u < U; ++u) {
+        const int ks = 32 * min(k0 + 4 * u, nks - 1);
+        av[u] = *(const f16x8*)(xr + ks);
 #pragma unroll
-      for (int pos = 0; pos < 8; ++pos) {
-        o0[pos] = in[bits == 2 ? perm_src<2>(pos) : perm_src<4>(pos)];
-        o1[pos] = in[bits == 2 ? perm_src<2>(pos + 8) : perm_src<4>(pos + 8)];
+        for (int i = 0; i < NT; ++i) bv[u][i] = wr[i] ? *(const f16x8*)(wr[i] + ks) : f16x8{};
       }
-      __half* dst = dstb + (int64_t)(t0 + t) * a.H + 16 * blk;
-      *(f16x8*)dst = o0;
-      *(f16x8*)(dst + 8) = o1;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k0 + 4 * u < nks) {  // uniform over the wave
+#pragma unroll
+          for (int i = 0; i < NT; ++i) acc[i] = mfma_16x16x32(av[u], bv[u][i], acc[i]);
+        }
+    }
+    // acc[i][j]: token 4kb + j, router row li of tile 2 i + par
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) red[par][kw][4 * kb + j][li] = acc[i][j];
+      __syncthreads();
+      {
+        const int pr = tid >> 8, t = (tid >> 4) & 15, c = tid & 15;
+        const float s = red[pr][0][t][c] + red[pr][1][t][c] + red[pr][2][t][c] + red[pr][3][t][c];
+        const int row = (2 * i + pr) * 16 + c;
+        if (row < nrow) lg[t][row] = __half2float(__float2half(s));
+      }
+      __syncthreads();
     }
   }
   // routing, one wave per token
-  for (int t = wave; t < 16; t += 4) {
+  for (int t = wave; t < 16; t += 8) {
     const int tok = t0 + t;
     if (tok >= a.T) continue;
     if (a.logits_out)
       for (int e = lane; e < a.E; e += 64)
         a.logits_out[(int64_t)tok * a.E + e] = __float2half(lg[t][e]);
     if (a.sgw && lane == 0) a.sg[tok] = __float2half(1.f / (1.f + expf(-lg[t][a.E])));
-    // top-k: k rounds of the largest (logit, then lower index) not yet taken
-    uint32_t taken[4] = {0u, 0u, 0u, 0u};  // experts lane + 64 q taken
+    // top-k: k rounds of the largest key (logit, then lower index) not yet
+    // taken; key 0 is no expert
+    uint32_t key[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = lane + 64 * q;
+      key[q] = e < a.E ? moe_key(__half_as_ushort(__float2half(lg[t][e])), e) : 0u;
+    }
     float mx = 0.f, wsel = 0.f;
     int esel = 0;
     for (int j = 0; j < a.topk; ++j) {
-      float bv = -__builtin_inff();
-      int be = 0x7fffffff;
-      for (int q = 0; q < 4; ++q) {
-        const int e = lane + 64 * q;
-        if (e < a.E && !taken[q]) {
-          const float v = lg[t][e];
-          if (v > bv) { bv = v; be = e; }  // e ascending within a lane
-        }
-      }
-      // wave argmax: larger value, then lower index
+      const uint32_t best = pf_wave_max(max(max(key[0], key[1]), max(key[2], key[3])));
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) {
-        const float ov = __shfl_xor(bv, o);
-        const int oe = __shfl_xor(be, o);
-        if (ov > bv || (ov == bv && oe < be)) { bv = ov; be = oe; }
-      }
-      if ((be & 63) == lane) taken[be >> 6] = 1u;
+      for (int q = 0; q < 4; ++q)
+        if (key[q] == best) key[q] = 0u;
+      const float bv = moe_key_logit(best);
       if (j == 0) mx = bv;
-      if (lane == j) { esel = be; wsel = bv; }
+      if (lane == j) { esel = 0xFFFF - (int)(best & 0xFFFFu); wsel = bv; }
     }
     float sum = 0.f;
     for (int e = lane; e < a.E; e += 64) sum += expf(lg[t][e] - mx);
@@ -1316,32 +1428,70 @@ __global__ __launch_bounds__(256) void pf_moe_route_kernel(PfMoe a) {
 }
 
 // One workgroup: per-expert counts, offsets, each pick's sorted row, the token
-// of each sorted row, and the tile list.
+// of each sorted row, and the tile list.  A chain of memory round trips, so
+// eight picks a thread are loaded at once and the offsets are one wave's scan
+// (one load a pick and a serial walk over the experts took 18.7 us for 12000
+// picks of 128 experts).
 __global__ __launch_bounds__(1024) void pf_moe_dispatch_kernel(PfMoe a) {
-  __shared__ int cnt[256], off[256], cur[256], tb[257];
+  __shared__ int cnt[256], off[256], cur[256], tb[256];
   const int tid = threadIdx.x, P = a.T * a.topk;
-  for (int e = tid; e < a.E; e += 1024) cnt[e] = 0;
+  if (tid < 256) cnt[tid] = 0;
   __syncthreads();
-  for (int p = tid; p < P; p += 1024) atomicAdd(&cnt[a.sel[p]], 1);
-  __syncthreads();
-  if (tid == 0) {
-    int o = 0, tt = 0;
-    for (int e = 0; e < a.E; ++e) {
-      off[e] = o;
-      cur[e] = o;
-      tb[e] = tt;
-      o += cnt[e];
-      tt += (cnt[e] + a.tm - 1) / a.tm;
+  constexpr int U = 8;
+  for (int p0 = 0; p0 < P; p0 += 1024 * U) {
+    int e[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + 1024 * u + tid;
+      e[u] = p < P ? a.sel[p] : -1;
     }
-    tb[a.E] = tt;
-    *a.ntiles = tt;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e[u] >= 0) atomicAdd(&cnt[e[u]], 1);
   }
   __syncthreads();
-  for (int p = tid; p < P; p += 1024) {
-    const int e = a.sel[p];
-    const int r = atomicAdd(&cur[e], 1);
-    a.pos[p] = r;
-    a.stok[r] = p / a.topk;
+  if (tid < 64) {  // lane l: experts 4 l .. 4 l + 3
+    int c[4], rs = 0, ts = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      c[u] = cnt[4 * tid + u];
+      rs += c[u];
+      ts += (c[u] + a.tm - 1) / a.tm;
+    }
+    int ri = rs, ti = ts;  // inclusive sums over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int rv = __shfl_up(ri, o), tv = __shfl_up(ti, o);
+      if (tid >= o) {
+        ri += rv;
+        ti += tv;
+      }
+    }
+    if (tid == 63) *a.ntiles = ti;
+    int ro = ri - rs, to = ti - ts;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      off[4 * tid + u] = cur[4 * tid + u] = ro;
+      tb[4 * tid + u] = to;
+      ro += c[u];
+      to += (c[u] + a.tm - 1) / a.tm;
+    }
+  }
+  __syncthreads();
+  for (int p0 = 0; p0 < P; p0 += 1024 * U) {
+    int e[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + 1024 * u + tid;
+      e[u] = p < P ? a.sel[p] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (e[u] < 0) continue;
+      const int p = p0 + 1024 * u + tid, r = atomicAdd(&cur[e[u]], 1);
+      a.pos[p] = r;
+      a.stok[r] = p / a.topk;
+    }
   }
   for (int e = tid; e < a.E; e += 1024) {
     const int n = (cnt[e] + a.tm - 1) / a.tm;
@@ -1355,20 +1505,41 @@ __global__ __launch_bounds__(1024) void pf_moe_dispatch_kernel(PfMoe a) {
 }
 
 // out[t][n] = fp16(sum_k w_k y[pos(t, k)][n] + sg[t] fp16(shared[t][n])),
-// then fp16(residual + out): the decode step's combine (glq_moe.hip).
+// then fp16(residual + out): the decode step's combine (glq_moe.hip).  Four
+// columns a thread, the picks' rows loaded four at a time.  (top_k fp32 rows
+// read a token: 98 MB for 1500 tokens x 8 picks x 2048, 36.5 us at one column
+// a thread.)
 __global__ __launch_bounds__(256) void pf_moe_combine_kernel(PfMoe a) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
   if (i >= (int64_t)a.T * a.H) return;
   const int t = (int)(i / a.H), n = (int)(i - (int64_t)t * a.H);
-  float acc = 0.f;
-  for (int k = 0; k < a.topk; ++k) {
-    const int p = t * a.topk + k;
-    acc = fmaf(__half2float(a.wts[p]), a.ybuf[(int64_t)a.pos[p] * a.H + n], acc);
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < a.topk; k0 += 4) {
+    float4 v[4];
+    float w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int p = t * a.topk + min(k0 + u, a.topk - 1);
+      v[u] = *(const float4*)(a.ybuf + (int64_t)a.pos[p] * a.H + n);
+      w[u] = __half2float(a.wts[p]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (k0 + u < a.topk) {
+        acc[0] = fmaf(w[u], v[u].x, acc[0]);
+        acc[1] = fmaf(w[u], v[u].y, acc[1]);
+        acc[2] = fmaf(w[u], v[u].z, acc[2]);
+        acc[3] = fmaf(w[u], v[u].w, acc[3]);
+      }
   }
-  if (a.sy) acc = fmaf(__half2float(a.sg[t]), __half2float(__float2half(a.sy[i])), acc);
-  float o = __half2float(__float2half(acc));
-  if (a.res) o += __half2float(a.res[i]);
-  a.out[i] = __float2half(o);
+  const float sg = a.sy ? __half2float(a.sg[t]) : 0.f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    if (a.sy) acc[c] = fmaf(sg, __half2float(__float2half(a.sy[i + c])), acc[c]);
+    float o = __half2float(__float2half(acc[c]));
+    if (a.res) o += __half2float(a.res[i + c]);
+    a.out[i + c] = __float2half(o);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1396,8 +1567,10 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
     P.tm = v >= 128 ? 128 : (v >= 64 ? 64 : 32);
   }
   P.max_tiles = (int)((Pn + P.tm - 1) / P.tm + E);
-  pf_lowrank_split(H, P.ks_gu, P.kps_gu);
-  pf_lowrank_split(I, P.ks_d, P.kps_d);
+  // (about as many row blocks as experts' full blocks and one ragged each)
+  const int64_t lrb = (Pn + kLrRows - 1) / kLrRows + std::min<int64_t>(E, Pn) / 2;
+  pf_lowrank_split(H, lrb, P.ks_gu, P.kps_gu);
+  pf_lowrank_split(I, lrb, P.ks_d, P.kps_d);
   P.stm = T > 32 ? 64 : 32;
   int64_t o = 0;
   auto take = [&](int64_t bytes) {
@@ -1524,7 +1697,14 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
   float* lp = (float*)(w + P.off_lp);
 
   // 1-2. routing and dispatch
-  pf_moe_route_kernel<<<dim3((unsigned)((T + 15) / 16)), dim3(256), 0, s>>>(a);
+  {
+    const int nt = (int)((E + (a.sgw ? 1 : 0) + 31) / 32);  // pairs of 16-row router tiles
+    const auto kern = nt <= 1   ? pf_moe_route_kernel<1>
+                      : nt <= 2 ? pf_moe_route_kernel<2>
+                      : nt <= 4 ? pf_moe_route_kernel<4>
+                                : pf_moe_route_kernel<9>;
+    kern<<<dim3((unsigned)((T + 15) / 16), 2), dim3(512), 0, s>>>(a);
+  }
   GLQ_LAUNCH_CHECK("pf_moe_route_kernel");
   pf_moe_dispatch_kernel<<<dim3(1), dim3(1024), 0, s>>>(a);
   GLQ_LAUNCH_CHECK("pf_moe_dispatch_kernel");
@@ -1554,7 +1734,7 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     L.kps = P.kps_gu;
     L.part = lp;
     L.a_out = agu;
-    rc = pf_lowrank_launch(L, P.max_tiles * (P.tm / kLrRows), s);
+    rc = pf_lowrank_launch(L, P.max_tiles * ((P.tm + kLrRows - 1) / kLrRows), s);
     if (rc) return rc;
   }
   // 4. gate/up + SwiGLU -> inter (rows sorted by expert, down's decode order)
@@ -1605,7 +1785,7 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     L.kps = P.kps_d;
     L.part = lp;
     L.a_out = ad;
-    rc = pf_lowrank_launch(L, P.max_tiles * (P.tm / kLrRows), s);
+    rc = pf_lowrank_launch(L, P.max_tiles * ((P.tm + kLrRows - 1) / kLrRows), s);
     if (rc) return rc;
   }
   // 6. down -> y per sorted row (fp32)
@@ -1671,7 +1851,7 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     if (rc) return rc;
   }
   // 8. combine
-  pf_moe_combine_kernel<<<dim3((unsigned)((T * H + 255) / 256)), dim3(256), 0, s>>>(a);
+  pf_moe_combine_kernel<<<dim3((unsigned)((T * H / 4 + 255) / 256)), dim3(256), 0, s>>>(a);
   GLQ_LAUNCH_CHECK("pf_moe_combine_kernel");
   return GLQ_OK;
 }
