@@ -8,6 +8,8 @@
 
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+
 #include "glq_gemv_core.h"
 #include "glq_handoff.h"
 #include "glq_internal.h"
@@ -315,21 +317,36 @@ __global__ __launch_bounds__(kDecThreads) void qk_norm_rope_kernel(QkArgs a) {
 
 // ---------------------------------------------------------------------------
 // Single-query attention of token b's q heads of KV group g over cache
-// positions [0, L), L = *len (clamped to [1, max_len]), split over blocks of
-// kAttnChunk positions (flash-decoding):
+// positions [0, L), L = *len (clamped to [1, max_len]), flash-decoding:
 //   out = sum_p softmax_p(scale * q . k_p) v_p        (fp32, fp16 result)
-// Block (split, g, b) stages its K and V rows and the group's rep <= 8 q rows
-// in LDS (every load in flight at once), scores (position, head) pairs with
-// v_dot2 on fp16 pairs, forms per-head max m, sum l and l-weighted V rows o,
-// and writes (m, l, o) to the workspace.  The last block of (b, g) to arrive
-// (an arrival counter, incremented after a device-scope fence) merges the
-// splits -- M = max m_s, out = sum o_s e^(m_s - M) / sum l_s e^(m_s - M) --
-// and zeroes the counter for the next call; the last block of (0, 0) also
-// advances *advance (the cache's fill counter) by one.
+// K and V rows are read once and used by the group's rep <= 8 heads, so the
+// bound is their bytes; the work per byte has to stay below the vector rate:
+//  * Scores by v_mfma_f32_16x16x32_f16 with A = the heads' q rows (16, zero
+//    past rep) and B = 16 positions' K rows straight from memory (lane (pos,
+//    kb) holds 16-byte piece 4 t + kb of its row at k-step t): no LDS.
+//  * The weighted V sum in fp32 on v_fma_mix: lane (r, c) holds columns
+//    8 c .. + 8 of the positions = r mod 4 (16-byte loads of four whole rows)
+//    and the sums of RH heads; a weight reaches its lanes through 1 KB of LDS
+//    a wave.  16 fmas a position and lane at 8 heads: about 10 TB/s of V for
+//    the chip.
+//  * A wave takes 32-position blocks w, w + 4, ... of its workgroup's range
+//    with the next block's 16 KB in flight; online softmax a block.
+//  * The L positions are split evenly on the device over at most nsplit
+//    workgroups a group (whole 128-position steps), so every L uses them all;
+//    the ones past L leave at once and are not counted.  nsplit gives about
+//    two workgroups a CU (the kernel's occupancy): one round of them.
+// The last workgroup of (b, g) to arrive (an arrival counter, data handed
+// over coherently) merges the splits in order -- M = max m_s, out = sum o_s
+// e^(m_s - M) / sum l_s e^(m_s - M) -- and zeroes the counter for the next
+// call; the one of (0, 0) also advances *advance (the cache's fill counter).
+//
+// 16 sequences x 4000 positions, 32 / 4 heads (131 MB): with 128 positions a
+// workgroup staged in LDS and each head's scores and sums read from there,
+// 85 us (1.5 TB/s).
 // ---------------------------------------------------------------------------
-constexpr int kAttnChunk = 128;
+constexpr int kAttnChunk = 128;   // positions of a workgroup's step
 constexpr int kAttnMaxRep = 8;
-constexpr int kKStride = kHeadDim + 8;  // LDS row of K (halves), 16-byte aligned
+constexpr int kAttnMaxSplit = 64;
 constexpr int kPartStride = kHeadDim + 4;  // m, l, 2 pad, o: rows 16-byte aligned
 
 struct AttnArgs {
@@ -349,161 +366,265 @@ struct AttnArgs {
   int rank, rpad;
 };
 
-constexpr size_t kAttnLds = 2 * kAttnMaxRep * kHeadDim          // q rows
-                            + 2 * kAttnChunk * kKStride          // K rows
-                            + 2 * kAttnChunk * kHeadDim          // V rows
-                            + 4 * kAttnMaxRep * kAttnChunk + 16;  // weights, flag
+// LDS: per wave 32 x 8 weights; then the waves' (m, l) and sums; then, in the
+// XU form, the merged rows and URows::dot's sums.
+constexpr int kAttnWts = 4 * 32 * 8;                              // floats
+constexpr int kAttnOut = 4 * kAttnMaxRep * (kHeadDim + 2);        // floats
+constexpr size_t kAttnLds = 4 * (kAttnWts + kAttnOut) + 16;
+static_assert(kAttnOut >= kAttnMaxRep * kHeadDim / 2 + kURowsRed, "XU area");
 
-template <bool XU>
-__global__ __launch_bounds__(kDecThreads) void decode_attention_kernel(AttnArgs a) {
+// Largest of a DPP row's 16 lanes, on each of them.
+__device__ __forceinline__ float row16_max(float v) {
+  auto m = [&](int y) { v = fmaxf(v, __int_as_float(y)); };
+  m(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
+  m(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
+  m(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false));
+  m(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));
+  return v;
+}
+
+__device__ __forceinline__ float row16_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));
+  return v;
+}
+
+// RH: heads of a lane's sums (4 or 8, at least rep).
+template <bool XU, int RH>
+__global__ __launch_bounds__(kDecThreads, 2) void decode_attention_kernel(AttnArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __half* qs = (__half*)smem;
-  __half* ks = qs + kAttnMaxRep * kHeadDim;
-  __half* vs = ks + kAttnChunk * kKStride;
-  float* ps = (float*)(vs + kAttnChunk * kHeadDim);
-  int* flag = (int*)(ps + kAttnMaxRep * kAttnChunk);
+  float* obuf = (float*)smem + kAttnWts;  // [wave][head][m, l, o[128]]
+  int* flag = (int*)(obuf + kAttnOut);
   const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rep = a.Hq / a.Hk;
   const int L = min(max(*a.len, 1), a.max_len);
-  const int c0 = split * kAttnChunk, n = max(0, min(kAttnChunk, L - c0));
-  const int64_t base = ((int64_t)b * a.Hk + g) * a.max_len * kHeadDim + (int64_t)c0 * kHeadDim;
-  // stage: 16-byte pieces, 16 per row; K and V rows [0, n), q rows [0, rep).
-  // Every load is unconditional (rows past n re-read row n - 1, the rows past
-  // n in LDS are never read), so all 16 go out before the first wait.
-  if (n > 0) {
-    constexpr int NJ = kAttnChunk * 16 / kDecThreads;  // 16-byte pieces per thread
-    f16x8 kb[NJ], vb[NJ];
+  // positions of a split: L over nsplit, whole steps; splits with positions
+  const int steps = (L + kAttnChunk - 1) / kAttnChunk;
+  const int chunk = (steps + a.nsplit - 1) / a.nsplit * kAttnChunk;
+  const int nact = (L + chunk - 1) / chunk;
+  if (split >= nact) return;  // uniform
+  const int c0 = split * chunk, c1 = min(c0 + chunk, L);
+  const int64_t base = ((int64_t)b * a.Hk + g) * a.max_len * kHeadDim;
+  const f16x8* kp = (const f16x8*)(a.k_cache + base);
+  const f16x8* vp = (const f16x8*)(a.v_cache + base);
+  const int li = lane & 15, kb = lane >> 4;
+  f16x8 q[4];  // A rows: heads (zero past rep)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int idx = j * kDecThreads + tid, r = min(idx >> 4, n - 1), c = idx & 15;
-      kb[j] = ((const f16x8*)(a.k_cache + base))[r * 16 + c];
-      vb[j] = ((const f16x8*)(a.v_cache + base))[r * 16 + c];
-    }
-    if (tid < rep * 16)
-      ((f16x8*)qs)[tid] = ((const f16x8*)(a.q + ((int64_t)b * a.Hq + g * rep) * kHeadDim))[tid];
+  for (int t = 0; t < 4; ++t)
+    q[t] = li < rep ? ((const f16x8*)(a.q + ((int64_t)b * a.Hq + g * rep + li) * kHeadDim))[4 * t + kb]
+                    : f16x8{};
+  float* pw = (float*)smem + wave * 32 * 8;  // this wave's weights [position][head]
+  // m, l: heads 4 kb + j (kb < 2); l a lane's own positions'.  o: columns
+  // 8 li .. + 8 of the positions = kb mod 4
+  float m[4], l[4], o[RH][8];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int idx = j * kDecThreads + tid, r = idx >> 4, c = idx & 15;
-      *(f16x8*)(ks + r * kKStride + 8 * c) = kb[j];
-      ((f16x8*)vs)[idx] = vb[j];
-    }
+  for (int j = 0; j < 4; ++j) {
+    m[j] = -__builtin_inff();
+    l[j] = 0.f;
   }
-  __syncthreads();
-  // scores: position p = tid % chunk, heads h = tid / chunk, + 256 / chunk, ...
-  {
-    const int p = tid & (kAttnChunk - 1);
-    for (int h = tid / kAttnChunk; h < rep; h += kDecThreads / kAttnChunk) {
-      float s = -__builtin_inff();
-      if (p < n) {
-        float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const f16x8 kv = *(const f16x8*)(ks + p * kKStride + 8 * j);
-          const f16x8 qv = *(const f16x8*)(qs + h * kHeadDim + 8 * j);
+  for (int h = 0; h < RH; ++h)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const f16x2 k2 = {kv[2 * e], kv[2 * e + 1]}, q2 = {qv[2 * e], qv[2 * e + 1]};
-            if (e & 1)
-              s1 = __builtin_amdgcn_fdot2(q2, k2, s1, false);
-            else
-              s0 = __builtin_amdgcn_fdot2(q2, k2, s0, false);
-          }
-        }
-        s = (s0 + s1) * a.scale;
+    for (int e = 0; e < 8; ++e) o[h][e] = 0.f;
+  struct Block {
+    f16x8 k[2][4], v[8];
+  };
+  auto load = [&](Block& x, int p0) {  // rows past L re-read row L - 1
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f16x8* row = kp + (int64_t)min(p0 + 16 * i + li, L - 1) * 16;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x.k[i][t] = row[4 * t + kb];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x.v[i] = vp[(int64_t)min(p0 + 4 * i + kb, L - 1) * 16 + li];
+  };
+  auto step = [&](Block& x, int p0) {
+    float s[2][4], mx[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc = mfma_16x16x32(q[t], x.k[i][t], acc);
+      const bool in = p0 + 16 * i + li < c1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[i][j] = in ? acc[j] * a.scale : -__builtin_inff();
+    }
+    bool grow = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      mx[j] = fmaxf(m[j], row16_max(fmaxf(s[0][j], s[1][j])));
+      grow |= mx[j] > m[j];
+    }
+    if (__builtin_amdgcn_ballot_w64(grow) != 0) {  // uniform: rescale the sums
+      float f[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f[j] = mx[j] > m[j] ? expf(m[j] - mx[j]) : 1.f;
+        l[j] *= f[j];
+        m[j] = mx[j];
       }
-      ps[h * kAttnChunk + p] = s;
-    }
-  }
-  __syncthreads();
-  // per head (32 lanes each): chunk max and sum, weights in place
-  const int h = tid >> 5, l32 = tid & 31;
-  float m = -__builtin_inff(), l = 0.f;
-  if (h < rep) {
-    float* row = ps + h * kAttnChunk;
 #pragma unroll
-    for (int i = 0; i < kAttnChunk / 32; ++i) m = fmaxf(m, row[l32 + 32 * i]);
+      for (int h = 0; h < RH; ++h) {
+        const float fh = __int_as_float(
+            __builtin_amdgcn_readlane(__float_as_int(f[h & 3]), 16 * (h >> 2)));
 #pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if (n > 0) {
-#pragma unroll
-      for (int i = 0; i < kAttnChunk / 32; ++i) {
-        const int p = l32 + 32 * i;
-        const float e = p < n ? expf(row[p] - m) : 0.f;
-        row[p] = e;
-        l += e;
+        for (int e = 0; e < 8; ++e) o[h][e] *= fh;
       }
     }
 #pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) l += __shfl_xor(l, o);
-  }
-  __syncthreads();
-  // o_h[4 l32 .. +4] = sum_p w[h][p] v[p][..]
-  float* my = a.part + (((int64_t)b * a.Hq + g * rep + h) * a.nsplit + split) * kPartStride;
-  if (h < rep) {
-    float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
-    const float* row = ps + h * kAttnChunk;
-#pragma unroll 8
-    for (int p = 0; p < n; ++p) {
-      const float w = row[p];
-      const uint2 vv = *(const uint2*)(vs + p * kHeadDim + 4 * l32);
-      const f16x2 va = __builtin_bit_cast(f16x2, vv.x), vb2 = __builtin_bit_cast(f16x2, vv.y);
-      o0 += w * (float)va[0];
-      o1 += w * (float)va[1];
-      o2 += w * (float)vb2[0];
-      o3 += w * (float)vb2[1];
-    }
-    if (l32 == 0) {
-      handoff_put(my, m);
-      handoff_put(my + 1, l);
-    }
-    handoff_put(my + 4 + 4 * l32, o0);
-    handoff_put(my + 5 + 4 * l32, o1);
-    handoff_put(my + 6 + 4 * l32, o2);
-    handoff_put(my + 7 + 4 * l32, o3);
-  }
-  // arrival (glq_handoff.h); the last block of (b, g) merges the splits
-  if (!handoff_arrive(a.count + b * a.Hk + g, (unsigned)a.nsplit, flag)) return;
-  // The other blocks' partials through coherent loads, up to 8 splits' worth
-  // in flight at once, merged online (running max M, sums rescaled when M
-  // grows).  Every thread loads (threads past rep read head rep - 1's and
-  // drop them), so that in the XU form the group's rows of U -- rows
-  // [g R, g R + R) -- go out right after the first 8 splits' loads: the merge
-  // waits for its own loads only and the U rows arrive behind it.
-  const int R = rep * kHeadDim;
-  URows<kAttnMaxRep * kHeadDim / 32> ur;
-  const float* ph =
-      a.part + ((int64_t)b * a.Hq + g * rep + min(h, rep - 1)) * a.nsplit * kPartStride;
-  float M = -__builtin_inff(), den = 0.f, r0 = 0.f, r1 = 0.f, r2 = 0.f, r3 = 0.f;
-  auto merge8 = [&](int s0, bool first) {
-    float ms[8], ls[8];
-    float4 os[8];
+    for (int i = 0; i < 2; ++i) {
+      const bool in = p0 + 16 * i + li < c1;
+      float4 w;
+      float* wv = (float*)&w;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int s2 = min(s0 + j, a.nsplit - 1);
-      const float* pp = ph + s2 * kPartStride;
-      ms[j] = handoff_get(pp);
-      ls[j] = handoff_get(pp + 1);
-      os[j] = float4{handoff_get(pp + 4 + 4 * l32), handoff_get(pp + 5 + 4 * l32),
-                     handoff_get(pp + 6 + 4 * l32), handoff_get(pp + 7 + 4 * l32)};
-    }
-    if constexpr (XU) {
-      if (first) ur.issue(a.U + (int64_t)g * R * a.rank, a.rank, R, 0);
+      for (int j = 0; j < 4; ++j) {
+        // (a head whose scores are all -inf so far has m = -inf: no weight)
+        wv[j] = in && m[j] != -__builtin_inff() ? expf(s[i][j] - m[j]) : 0.f;
+        l[j] += wv[j];
+      }
+      if (kb < 2) *(float4*)(pw + (16 * i + li) * 8 + 4 * kb) = w;
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (s0 + j >= a.nsplit || ms[j] == -__builtin_inff()) continue;  // none / empty split
-      const float Mn = fmaxf(M, ms[j]);
-      const float fo = expf(M - Mn), fn = expf(ms[j] - Mn);  // M = -inf: fo = 0
-      den = den * fo + ls[j] * fn;
-      r0 = r0 * fo + os[j].x * fn;
-      r1 = r1 * fo + os[j].y * fn;
-      r2 = r2 * fo + os[j].z * fn;
-      r3 = r3 * fo + os[j].w * fn;
-      M = Mn;
+    for (int i = 0; i < 8; ++i) {
+      const int p = 4 * i + kb;
+      const float4 w0 = *(const float4*)(pw + p * 8);
+      const float4 w1 = RH > 4 ? *(const float4*)(pw + p * 8 + 4) : w0;
+      const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+      f16x8 v = x.v[i];
+      if (p0 + 32 > c1 && p0 + p >= c1) v = f16x8{};  // weight 0 times a row that is no position's
+#pragma unroll
+      for (int h = 0; h < RH; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[h][e] = fmaf(w[h], (float)v[e], o[h][e]);
     }
   };
-  merge8(0, true);
-  for (int s0 = 8; s0 < a.nsplit; s0 += 8) merge8(s0, false);
+  {
+    Block x, y;
+    int p0 = c0 + 32 * wave;
+    if (p0 < c1) load(x, p0);
+    if (chunk == kAttnChunk && p0 < c1) {  // one step: nothing to load ahead
+      step(x, p0);
+      p0 = c1;
+    }
+    while (p0 < c1) {  // (loads past the range re-read rows of it)
+      load(y, min(p0 + kAttnChunk, c1 - 1));
+      step(x, p0);
+      p0 += kAttnChunk;
+      if (p0 >= c1) break;
+      load(x, min(p0 + kAttnChunk, c1 - 1));
+      step(y, p0);
+      p0 += kAttnChunk;
+    }
+  }
+  // the wave's sums: l over the 16 lanes of a head's row, o over the four kb
+  // by lane swaps that leave each kb a quarter of the heads (two values in,
+  // their two sums out on different lanes)
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    l[j] = row16_sum(l[j]);
+    if (li == 0 && 4 * kb + j < RH) {
+      float* ow = obuf + (wave * kAttnMaxRep + 4 * kb + j) * (kHeadDim + 2);
+      ow[0] = m[j];
+      ow[1] = l[j];
+    }
+  }
+  auto swap32 = [](float x, float y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false,
+                                                    false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  auto swap16 = [](float x, float y) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false,
+                                                    false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+#pragma unroll
+  for (int h = 0; h < RH / 4; ++h) {
+    // heads h + RH / 4 (kb & 1) + RH / 2 (kb / 2) on lane group kb
+    float* ow = obuf + (wave * kAttnMaxRep + h + RH / 4 * (kb & 1) + RH / 2 * (kb >> 1)) *
+                           (kHeadDim + 2) + 2 + 8 * li;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      ow[e] = swap16(swap32(o[h][e], o[h + RH / 2][e]),
+                     swap32(o[h + RH / 4][e], o[h + RH / 4 + RH / 2][e]));
+  }
+  __syncthreads();
+  // the four waves merged in order: thread (head h, columns 4 l32 .. + 4)
+  const int h = tid >> 5, l32 = tid & 31;
+  float M = -__builtin_inff(), den = 0.f, r0 = 0.f, r1 = 0.f, r2 = 0.f, r3 = 0.f;
+  auto merge = [&](float ms, float ls, float4 os) {
+    if (ms == -__builtin_inff()) return;  // no position, or none with a weight
+    const float Mn = fmaxf(M, ms);
+    const float fo = expf(M - Mn), fn = expf(ms - Mn);  // M = -inf: fo = 0
+    den = den * fo + ls * fn;
+    r0 = r0 * fo + os.x * fn;
+    r1 = r1 * fo + os.y * fn;
+    r2 = r2 * fo + os.z * fn;
+    r3 = r3 * fo + os.w * fn;
+    M = Mn;
+  };
+  if (h < rep) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float* ow = obuf + (w * kAttnMaxRep + h) * (kHeadDim + 2);
+      const float* oc = ow + 2 + 4 * l32;
+      merge(ow[0], ow[1], float4{oc[0], oc[1], oc[2], oc[3]});
+    }
+  }
+  const int R = rep * kHeadDim;
+  URows<kAttnMaxRep * kHeadDim / 32> ur;
+  if (nact == 1) {
+    if constexpr (XU) ur.issue(a.U + (int64_t)g * R * a.rank, a.rank, R, 0);
+    __syncthreads();  // obuf has been read
+  } else {
+    float* my = a.part + (((int64_t)b * a.Hq + g * rep + h) * a.nsplit + split) * kPartStride;
+    if (h < rep) {
+      if (l32 == 0) {
+        handoff_put(my, M);
+        handoff_put(my + 1, den);
+      }
+      handoff_put(my + 4 + 4 * l32, r0);
+      handoff_put(my + 5 + 4 * l32, r1);
+      handoff_put(my + 6 + 4 * l32, r2);
+      handoff_put(my + 7 + 4 * l32, r3);
+    }
+    // arrival (glq_handoff.h); the last workgroup of (b, g) merges the splits
+    if (!handoff_arrive(a.count + b * a.Hk + g, (unsigned)nact, flag)) return;
+    // The other workgroups' partials through coherent loads, up to 8 splits'
+    // worth in flight at once, merged online in split order.  Every thread
+    // loads (threads past rep read head rep - 1's and drop them), so that in
+    // the XU form the group's rows of U -- rows [g R, g R + R) -- go out right
+    // after the first 8 splits' loads: the merge waits for its own loads only
+    // and the U rows arrive behind it.
+    const float* ph =
+        a.part + ((int64_t)b * a.Hq + g * rep + min(h, rep - 1)) * a.nsplit * kPartStride;
+    M = -__builtin_inff();
+    den = r0 = r1 = r2 = r3 = 0.f;
+    auto merge8 = [&](int s0, bool first) {
+      float ms[8], ls[8];
+      float4 os[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float* pp = ph + min(s0 + j, nact - 1) * kPartStride;
+        ms[j] = handoff_get(pp);
+        ls[j] = handoff_get(pp + 1);
+        os[j] = float4{handoff_get(pp + 4 + 4 * l32), handoff_get(pp + 5 + 4 * l32),
+                       handoff_get(pp + 6 + 4 * l32), handoff_get(pp + 7 + 4 * l32)};
+      }
+      if constexpr (XU) {
+        if (first) ur.issue(a.U + (int64_t)g * R * a.rank, a.rank, R, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (s0 + j < nact) merge(ms[j], ls[j], os[j]);
+    };
+    merge8(0, true);
+    for (int s0 = 8; s0 < nact; s0 += 8) merge8(s0, false);
+  }
   if (h < rep) {
     const float inv = 1.f / den;
     f16x2 oa = {(_Float16)(r0 * inv), (_Float16)(r1 * inv)};
@@ -511,12 +632,12 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_kernel(AttnArgs 
     __half* dst = a.out + (int64_t)b * a.Hq * kHeadDim + (int64_t)(g * rep + h) * kHeadDim;
     const uint2 o4 = uint2{__builtin_bit_cast(uint32_t, oa), __builtin_bit_cast(uint32_t, ob)};
     *(uint2*)(dst + 4 * l32) = o4;
-    if constexpr (XU) *(uint2*)((__half*)ks + h * kHeadDim + 4 * l32) = o4;  // K rows are dead
+    if constexpr (XU) *(uint2*)((__half*)obuf + h * kHeadDim + 4 * l32) = o4;  // the sums are dead
   }
   if constexpr (XU) {
     // the group's partial of out U (fp32), read by the next launch
-    const __half* xo = (const __half*)ks;
-    float* red = (float*)((__half*)ks + kAttnMaxRep * kHeadDim);  // kURowsRed floats
+    const __half* xo = (const __half*)obuf;
+    float* red = obuf + kAttnMaxRep * kHeadDim / 2;  // kURowsRed floats
     float* mine = a.xpart + ((int64_t)g * a.B + b) * a.rpad;
     __syncthreads();  // the merged rows are in xo
     for (int jb = 0; jb < a.rpad; jb += 64) {
@@ -526,7 +647,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_kernel(AttnArgs 
     }
   }
   if (tid == 0) {
-    handoff_reset(a.count + b * a.Hk + g);
+    if (nact > 1) handoff_reset(a.count + b * a.Hk + g);
     if (a.advance && b == 0 && g == 0) *a.advance += 1;
   }
 }
@@ -696,7 +817,6 @@ static int attention_launch(const void* q, const void* k_cache, const void* v_ca
                             void* out, const void* U, int64_t rank, float* parts,
                             void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace glq;
-  static size_t attr = 64 * 1024, attr_xu = 64 * 1024;
   GLQ_CHECK(head_dim == kHeadDim, "head_dim must be %d (got %lld)", kHeadDim,
             (long long)head_dim);
   GLQ_CHECK(tokens >= 0 && tokens <= 65535, "tokens must be in [0, 65535]");
@@ -719,25 +839,24 @@ static int attention_launch(const void* q, const void* k_cache, const void* v_ca
   a.q = (const __half*)q; a.k_cache = (const __half*)k_cache; a.v_cache = (const __half*)v_cache;
   a.len = len; a.advance = advance; a.out = (__half*)out;
   a.B = (int)tokens; a.Hq = (int)q_heads; a.Hk = (int)kv_heads; a.max_len = (int)max_len;
-  a.nsplit = (int)((max_len + kAttnChunk - 1) / kAttnChunk);
+  // about two workgroups a CU, whole steps, a bounded merge (the workspace
+  // holds a partial for every step of the cache)
+  const int64_t steps = (max_len + kAttnChunk - 1) / kAttnChunk;
+  a.nsplit = (int)std::max<int64_t>(
+      1, std::min({steps, (int64_t)kAttnMaxSplit, 512 / (tokens * kv_heads)}));
   a.scale = scale;
   a.part = (float*)workspace;
   a.count = (unsigned*)((char*)workspace +
-                        align_up(4 * tokens * q_heads * (int64_t)a.nsplit * kPartStride, 256));
+                        align_up(4 * tokens * q_heads * steps * kPartStride, 256));
   a.U = (const __half*)U;
   a.xpart = parts;
   a.rank = (int)rank;
   a.rpad = (int)align_up(rank, 32);
   const dim3 grid((unsigned)a.nsplit, (unsigned)kv_heads, (unsigned)tokens);
-  if (U) {
-    int rc = set_lds_limit(decode_attention_kernel<true>, kAttnLds, attr_xu);
-    if (rc) return rc;
-    decode_attention_kernel<true><<<grid, dim3(kDecThreads), kAttnLds, (hipStream_t)stream>>>(a);
-  } else {
-    int rc = set_lds_limit(decode_attention_kernel<false>, kAttnLds, attr);
-    if (rc) return rc;
-    decode_attention_kernel<false><<<grid, dim3(kDecThreads), kAttnLds, (hipStream_t)stream>>>(a);
-  }
+  const bool few = q_heads / kv_heads <= 4;
+  auto kern = U ? (few ? decode_attention_kernel<true, 4> : decode_attention_kernel<true, 8>)
+                : (few ? decode_attention_kernel<false, 4> : decode_attention_kernel<false, 8>);
+  kern<<<grid, dim3(kDecThreads), kAttnLds, (hipStream_t)stream>>>(a);
   GLQ_LAUNCH_CHECK("decode_attention_kernel");
   return GLQ_OK;
 }

@@ -301,3 +301,35 @@ def test_fused_layers_match_framework_layers(gpu, monkeypatch, B, producer):
         kd = (la.keys[:, :, :n].float() - lb.keys[:, :, :n].float()).abs().max()
         assert float(kd) <= 0.02 * float(lb.keys[:, :, :n].float().abs().max())
         assert torch.equal(la.keys[:, :, n:], lb.keys[:, :, n:])
+
+
+@pytest.mark.parametrize("B,Hq,Hk,L,maxlen", [
+    (130, 32, 4, 300, 320),   # one workgroup a group: three steps, the last ragged
+    (64, 32, 4, 257, 600),    # two splits of two steps, the second of one position
+    (8, 16, 4, 1000, 1032),   # 4 heads a group, one step a split
+    (16, 64, 8, 1153, 2000),  # 4 splits of three steps, one position over
+    (2, 6, 1, 127, 9000),     # one split of a long cache
+])
+def test_decode_attention_splits(gpu, B, Hq, Hk, L, maxlen):
+    """Position splits made on the device from the length: steps of 128, one to
+    several a workgroup, with infinities past the length (not read into the
+    sums, also where a block's rows are clamped)."""
+    hd = 128
+    g = torch.Generator(device=gpu).manual_seed(L)
+    q = torch.randn(B, Hq, hd, generator=g, device=gpu).half()
+    kc = torch.randn(B, Hk, maxlen, hd, generator=g, device=gpu).half()
+    vc = torch.randn(B, Hk, maxlen, hd, generator=g, device=gpu).half()
+    kc[:, :, L:] = float("inf")
+    vc[:, :, L:] = float("inf")
+    ln = torch.tensor([L], dtype=torch.int32, device=gpu)
+    ws = kernels.decode_attention_workspace(q, kc)
+    out = kernels.decode_attention(q, kc, vc, ln, hd ** -0.5, workspace=ws)
+    again = kernels.decode_attention(q, kc, vc, ln, hd ** -0.5, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    for b in (0, B - 1):
+        K, V = kc[b, :, :L].double(), vc[b, :, :L].double()
+        s = q[b].double().reshape(Hk, Hq // Hk, hd) @ K.transpose(1, 2).contiguous() * hd ** -0.5
+        ref = (torch.softmax(s, dim=-1) @ V).reshape(-1)
+        err = (out[b].double() - ref).abs()
+        assert bool((err <= 1e-3 + 2e-3 * ref.abs()).all()), float(err.max())  # fp16 rounding
