@@ -53,6 +53,20 @@ class TurboMat(ctypes.Structure):
     ]
 
 
+class TurboPrefillParams(ctypes.Structure):
+    """glq_turbo_prefill_params (include/glorcq_hip.h), field for field."""
+    _fields_ = [
+        *[(n, _i64) for n in ("tokens", "hidden", "experts", "inter", "top_k", "rank",
+                              "shared_inter")],
+        ("norm_topk_prob", ctypes.c_int32), ("shared_bits", ctypes.c_int32),
+        ("h", _vp), ("router_w", _vp), ("shared_gate_w", _vp),
+        *[(n, _vp * 3) for n in ("codes", "norms", "centroids", "U", "cluster_of", "SV")],
+        ("signs", _vp * 2), ("Pi", _vp * 2),
+        *[(n, _vp * 3) for n in ("shared_codes", "shared_scales", "shared_zeros")],
+        *[(n, _vp) for n in ("shared_y", "residual", "out", "router_logits")],
+    ]
+
+
 # name -> (restype, argtypes); must match include/glorcq_hip.h exactly.
 SIGNATURES = {
     "glq_version": (_c_int, []),
@@ -66,6 +80,8 @@ SIGNATURES = {
         _vp, _vp,                       # bias, y
         _vp, _i64, _vp,                 # workspace, bytes, stream
     ]),
+    "glq_turbo_moe_prefill_workspace_bytes": (_i64, [ctypes.POINTER(TurboPrefillParams)]),
+    "glq_turbo_moe_prefill": (_c_int, [ctypes.POINTER(TurboPrefillParams), _vp, _i64, _vp]),
     "glq_gemv_noalloc_max_scratch_bytes": (_i64, []),
     "glq_gemv_lora_noalloc": (_c_int, [
         _vp, _i64, _i64, _i64,          # x, M, K, N

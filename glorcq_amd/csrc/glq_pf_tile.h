@@ -39,18 +39,41 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(f16x8 a, f16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
+// What B is made of (template argument BITS): 2 or 4, group-quantized codes;
+// kPtTurbo, 2-bit indices of a codebook with a norm per row (no groups: the
+// products of all K run into y, the codebook in fp16 hi + lo parts, an MFMA
+// each, the norm at the end; A in the 4-bit decode order, turbo_decode's);
+// kPtHalf, fp16 rows (n, K), both operands in natural order.
+constexpr int kPtTurbo = 3, kPtHalf = 16;
+
+// fp16 codebook in v_perm_b32 form (low bytes of C0..C3, high bytes): hi part,
+// or the residual of it.
+__device__ __forceinline__ void pt_lut(const float* c, bool residual, uint32_t& lb, uint32_t& hb) {
+  lb = hb = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const __half hi = __float2half(c[i]);
+    const __half v = residual ? __float2half(c[i] - __half2float(hi)) : hi;
+    const uint32_t u = __half_as_ushort(v);
+    lb |= (u & 0xffu) << (8 * i);
+    hb |= (u >> 8) << (8 * i);
+  }
+}
+
 template <int BITS, int WM, int WN, int MT>
 struct PtSlot {
   static constexpr int TM = 32 * MT * WM;           // tokens of a tile
   static constexpr int NB = 2 * WN;                 // 32-row blocks of a tile
-  static constexpr int CB = BITS == 2 ? 32 : 64;    // code bytes per row per group
+  static constexpr int CB = BITS == 4 ? 64 : BITS == kPtHalf ? 256 : 32;  // B bytes per row per group
   static constexpr int C = TM * 256;                // A rows, then the codes
   static constexpr int BYTES = C + NB * 32 * CB;
   static constexpr int NIA = TM / 16;               // A load instructions per wave
   static constexpr int NIC = NB * CB / 128;         // code load instructions per wave
   static constexpr int NI = NIA + NIC;
   // ring depth: as many slots as let two workgroups share a CU, at most 4
-  static constexpr int D = 4 * BYTES <= 80 * 1024 ? 4 : (3 * BYTES <= 80 * 1024 ? 3 : 2);
+  // (fp16 rows: three for one workgroup)
+  static constexpr int D = BITS == kPtHalf ? 3
+                                           : 4 * BYTES <= 80 * 1024 ? 4 : (3 * BYTES <= 80 * 1024 ? 3 : 2);
 };
 
 // Weight row of row li of 32-row block b (may be >= N: clamp for loads).
@@ -61,6 +84,11 @@ __device__ __forceinline__ int pt_row(int n0, int b, int li) {
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pt_rsrc(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0xFFFFFFFFu, 0x00027000);
+}
+
+// Column n in the decode order of out_bits (0: natural).
+__device__ __forceinline__ int pt_col(int out_bits, int n) {
+  return out_bits ? (n & ~15) + perm_pos_rt(out_bits, n & 15) : n;
 }
 
 // Both halves' value of a pair loaded as (scale | zero-point) by lane half.
@@ -111,7 +139,9 @@ __device__ __forceinline__ PfK<BITS> pt_consts(__half sh, __half zh, float zoff)
 
 template <int BITS, int WM, int WN, int MT, int MODE, bool SYM, bool ZF, bool SZQ>
 __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
-  static_assert(WM * WN == 4 && (BITS == 2 || BITS == 4), "4 waves");
+  constexpr bool SCALED = BITS == 2 || BITS == 4;
+  static_assert(WM * WN == 4 && (SCALED || BITS == kPtTurbo || BITS == kPtHalf), "4 waves");
+  static_assert(BITS != kPtHalf || MODE == kPfDense, "one matrix");
   using SL = PtSlot<BITS, WM, WN, MT>;
   constexpr bool TWO = MODE == kPfGateUp;
   constexpr int D = SL::D;
@@ -131,6 +161,9 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
     rows = min(SL::TM, g.M - p0);
   }
   const int n0 = blockIdx.x * (TWO ? 32 : 64) * WN;
+  // K split z (DOWN: fp32 results of their own, summed by the combine; split 0
+  // has the low-rank term)
+  const int g0 = MODE == kPfDown ? (int)blockIdx.z * g.gps : 0;
 
   // ---- load addresses: element offsets from uniform bases ----
   // (buffer loads: one constant offset a lane, the group's in a scalar; they
@@ -149,32 +182,41 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
 #pragma unroll
   for (int q = 0; q < SL::NIC; ++q) {
     const int i = wave * SL::NIC + q;  // 1 KB of the slot's code region
-    const int b = BITS == 2 ? i : i >> 1;
-    const int piece = (BITS == 2 ? 0 : 2 * (i & 1)) + h;
-    crsrc[q] = pt_rsrc((TWO && (b & 1) ? g.codes[1] : g.codes[0]) + e * g.codes_es);
-    coff[q] = 4u * ((unsigned)min(pt_row<MODE>(n0, b, li), g.N - 1) * g.kw + 4 * piece);
+    if constexpr (BITS == kPtHalf) {
+      const int r = 4 * i + (lane >> 4);
+      crsrc[q] = pt_rsrc(g.codes[0]);
+      coff[q] = 2u * ((unsigned)min(pt_row<MODE>(n0, r >> 5, r & 31), g.N - 1) * (unsigned)g.K +
+                      (((lane & 15) ^ (r & 15)) << 3));
+    } else {
+      const int b = BITS == 4 ? i >> 1 : i;
+      const int piece = (BITS == 4 ? 2 * (i & 1) : 0) + h;
+      crsrc[q] = pt_rsrc((TWO && (b & 1) ? g.codes[1] : g.codes[0]) + e * g.codes_es);
+      coff[q] = 4u * ((unsigned)min(pt_row<MODE>(n0, b, li), g.N - 1) * g.kw + 4 * piece);
+    }
   }
   // scale (half 0) or zero-point (half 1) of this lane's row in each of the
   // wave's two 32-row blocks
-  const uint16_t* szp[2];
+  const uint16_t* szp[2] = {};
+  if constexpr (SCALED)
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {
     const int n = min(pt_row<MODE>(n0, 2 * wn + nt, li), g.N - 1);
     const int m = TWO ? nt : 0;
     const __half* base = (SYM || h == 0) ? g.scales[m] : g.zeros[m];
-    szp[nt] = (const uint16_t*)base + e * g.sz_es + (int64_t)n * g.G;
+    szp[nt] = (const uint16_t*)base + e * g.sz_es + (int64_t)n * g.G + g0;
   }
-  const int ng = g.G;
+  const int ng = MODE == kPfDown ? min(g.gps, g.G - g0) : g.G;
   auto issue = [&](int grp, unsigned char* slot) {
 #pragma unroll
     for (int q = 0; q < SL::NIA; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          arsrc, (lds_void*)(slot + (wave * SL::NIA + q) * 1024), 16, aoff[q], grp * 256, 0, 0);
+          arsrc, (lds_void*)(slot + (wave * SL::NIA + q) * 1024), 16, aoff[q],
+          (g0 + grp) * 256, 0, 0);
 #pragma unroll
     for (int q = 0; q < SL::NIC; ++q) {
       const int i = wave * SL::NIC + q;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(crsrc[q], (lds_void*)(slot + SL::C + i * 1024), 16,
-                                               coff[q], grp * SL::CB, 0, 0);
+                                               coff[q], (g0 + grp) * SL::CB, 0, 0);
     }
   };
 
@@ -190,10 +232,86 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
   // 32 (i WM + wm))
   const int nact = max(0, min(MT, ((rows + 31) / 32 - wm + WM - 1) / WM));
 
+  uint32_t lut[TWO ? 2 : 1][4] = {};  // codebook: hi's low and high bytes, lo's
+  if constexpr (BITS == kPtTurbo)
+#pragma unroll
+    for (int m = 0; m < (TWO ? 2 : 1); ++m) {
+      pt_lut(g.cent[m], false, lut[m][0], lut[m][1]);
+      pt_lut(g.cent[m], true, lut[m][2], lut[m][3]);
+    }
+
   // one group's products of NM token blocks
   auto group = [&](auto nm, int grp, const unsigned char* sl, const __half (&sh)[2],
                    const __half (&zh)[2]) {
     constexpr int NM = decltype(nm)::value;
+    auto arow = [&](int i) { return sl + (32 * (i * WM + wm) + li) * 256; };
+    auto piece = [&](int i, int p) { return *(const u32x4*)(arow(i) + ((p ^ (li & 15)) << 4)); };
+    auto a_op = [&](int i, int t) { return __builtin_bit_cast(f16x8, piece(i, 8 * h + t)); };
+    if constexpr (BITS == kPtHalf) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        f16x8 bv[2];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+          bv[nt] = *(const f16x8*)(sl + SL::C + ((2 * wn + nt) * 32 + li) * 256 +
+                                   (((8 * h + t) ^ (li & 15)) << 4));
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+          const f16x8 av = a_op(i, t);
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt) y[i][nt] = mfma_32x32x16(av, bv[nt], y[i][nt]);
+        }
+      }
+      return;
+    } else if constexpr (BITS == kPtTurbo) {
+      uint32_t tw[2][4];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        const u32x4 v = *(const u32x4*)(sl + SL::C + (2 * wn + nt) * 32 * SL::CB + li * 16 + h * 512);
+        tw[nt][0] = v.x; tw[nt][1] = v.y; tw[nt][2] = v.z; tw[nt][3] = v.w;
+      }
+      f16x8 av[2][2][NM];  // [word parity][slice][block], a word ahead of its use
+      auto load_a = [&](int i4) {
+#pragma unroll
+        for (int sl2 = 0; sl2 < 2; ++sl2)
+#pragma unroll
+          for (int i = 0; i < NM; ++i) av[i4 & 1][sl2][i] = a_op(i, 2 * i4 + sl2);
+      };
+      load_a(0);
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        if (i4 < 3) load_a(i4 + 1);
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          const int m = TWO ? nt : 0;
+          uint32_t bh[2][4], bl[2][4];  // slices 0,4,1,5,.. and 8,12,9,13,.. of the word
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t X = (tw[nt][i4] >> (2 * q)) & 0x03030303u, X4 = X | 0x04040404u;
+            const uint32_t sa = __builtin_amdgcn_perm(X4, X, 0x05010400u);  // (q, q + 4)
+            const uint32_t sb = __builtin_amdgcn_perm(X4, X, 0x07030602u);  // (q + 8, q + 12)
+            bh[0][q] = __builtin_amdgcn_perm(lut[m][1], lut[m][0], sa);
+            bh[1][q] = __builtin_amdgcn_perm(lut[m][1], lut[m][0], sb);
+            bl[0][q] = __builtin_amdgcn_perm(lut[m][3], lut[m][2], sa);
+            bl[1][q] = __builtin_amdgcn_perm(lut[m][3], lut[m][2], sb);
+          }
+#pragma unroll
+          for (int sl2 = 0; sl2 < 2; ++sl2) {
+            const f16x8 vh = __builtin_bit_cast(
+                f16x8, u32x4{bh[sl2][0], bh[sl2][1], bh[sl2][2], bh[sl2][3]});
+            const f16x8 vl = __builtin_bit_cast(
+                f16x8, u32x4{bl[sl2][0], bl[sl2][1], bl[sl2][2], bl[sl2][3]});
+#pragma unroll
+            for (int i = 0; i < NM; ++i) {
+              y[i][nt] = mfma_32x32x16(av[i4 & 1][sl2][i], vh, y[i][nt]);
+              y[i][nt] = mfma_32x32x16(av[i4 & 1][sl2][i], vl, y[i][nt]);
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    } else {
     uint32_t w[2][BITS == 2 ? 4 : 8];
     PfK<BITS> kc[2];
 #pragma unroll
@@ -210,9 +328,6 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
       }
       kc[nt] = pt_consts<BITS, SYM, ZF>(sh[nt], zh[nt], g.zoff);
     }
-    auto arow = [&](int i) { return sl + (32 * (i * WM + wm) + li) * 256; };
-    auto piece = [&](int i, int p) { return *(const u32x4*)(arow(i) + ((p ^ (li & 15)) << 4)); };
-    auto a_op = [&](int i, int t) { return __builtin_bit_cast(f16x8, piece(i, 8 * h + t)); };
     // A operands two steps ahead of their use (an LDS read takes longer than
     // a step's four MFMAs); a scheduling barrier a step keeps them there
     f32x16 acc[NM][2];
@@ -264,6 +379,7 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
       for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
         for (int j = 0; j < 16; ++j) y[i][nt][j] = fmaf(kc[nt].s, acc[i][nt][j], y[i][nt][j]);
+    }
   };
 
   // ---- main loop: U groups an iteration share one load of scales.  One loop
@@ -271,6 +387,7 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
   constexpr int U = SZQ ? 4 : 1;
   u32x2 sz[2];
   auto load_sz = [&](int grp) {
+    if constexpr (!SCALED) return;
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
       if constexpr (SZQ) sz[nt] = *(const u32x2*)(szp[nt] + grp);
@@ -284,7 +401,8 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
   auto loop = [&](auto nm) {
     int in = D - 1, cur = 0;  // ring slots of the next issue and of the group
     for (int c = 0; c < ng; c += U) {
-      uint32_t s2[2][2], z2[2][2];  // [block][group pair]
+      uint32_t s2[2][2] = {}, z2[2][2] = {};  // [block][group pair]
+      if constexpr (SCALED)
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) {
         // (moved to registers of their own, so that the next load goes to
@@ -327,8 +445,20 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
   else loop(std::integral_constant<int, 0>{});
   wait_vmcnt<0>();  // the tail's loads land before the workgroup's LDS goes away
 
+  if constexpr (BITS == kPtTurbo) {  // the rows' norms
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const int n = min(pt_row<MODE>(n0, 2 * wn + nt, li), g.N - 1);
+      const float nr = g.norms[TWO ? nt : 0][e * g.n_es + n];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) y[i][nt][j] *= nr;
+    }
+  }
+
   // ---- low-rank term: y += a SV^T (a: token rows, SV: weight rows) ----
-  if (g.a != nullptr && g.rank > 0) {
+  if (g.a != nullptr && g.rank > 0 && g0 == 0) {
     for (int j0 = 0; j0 < g.rank; j0 += 16) {
       const int jk = j0 + 8 * h;
       const bool jv = jk < g.rank;
@@ -362,7 +492,7 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
     if constexpr (MODE == kPfGateUp) {
       const int n = pt_row<MODE>(n0, 2 * wn, li);
       if (n >= g.N) continue;
-      const int col = (n & ~15) + perm_pos_rt(g.out_bits, n & 15);
+      const int col = pt_col(g.out_bits, n);
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int r = t0 + 8 * (j >> 2) + (j & 3);
@@ -380,9 +510,10 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
           const int r = t0 + 8 * (j >> 2) + (j & 3);
           if (r >= rows) continue;
           if constexpr (MODE == kPfDense)
-            g.y[(int64_t)(p0 + r) * g.y_ld + n] = __float2half(y[i][nt][j] + bn);
+            g.y[(int64_t)(p0 + r) * g.y_ld + pt_col(g.out_bits, n)] =
+                __float2half(y[i][nt][j] + bn);
           else
-            g.yf[(int64_t)(p0 + r) * g.yf_ld + n] = y[i][nt][j];
+            g.yf[blockIdx.z * g.yf_ss + (int64_t)(p0 + r) * g.yf_ld + n] = y[i][nt][j];
         }
       }
     }
@@ -402,7 +533,7 @@ static int pt_launch_k(const PfArgs& g, hipStream_t s) {
   const size_t lds = (size_t)SL::D * SL::BYTES;
   int rc = set_lds_limit(pf_tile_kernel<BITS, WM, WN, MT, MODE, SYM, ZF, SZQ>, lds, attr);
   if (rc) return rc;
-  const dim3 grid((unsigned)g.ntn, (unsigned)g.max_tiles);
+  const dim3 grid((unsigned)g.ntn, (unsigned)g.max_tiles, (unsigned)(MODE == kPfDown ? g.ks : 1));
   pf_tile_kernel<BITS, WM, WN, MT, MODE, SYM, ZF, SZQ><<<grid, dim3(kPfThreads), lds, s>>>(g);
   GLQ_LAUNCH_CHECK("pf_tile_kernel");
   return GLQ_OK;

@@ -66,6 +66,9 @@ struct PfArgs {
   const __half* scales[2];   // (E, N, G)
   const __half* zeros[2];    // (E, N, G) (unused with SYM)
   int64_t codes_es, sz_es;   // expert strides (elements)
+  const float* norms[2];     // TurboQuant codes: (E, N) row norms,
+  int64_t n_es;
+  const float* cent[2];      // and the 4-entry codebook
   const __half* a;           // low-rank a (rows, a_ld) fp16: matrix m at column m*rank, or null
   int a_ld;
   const __half* sv[2];       // (E, N, rank)
@@ -74,7 +77,7 @@ struct PfArgs {
   __half* y;                 // DENSE: (M, N); GATE/UP: inter (rows, N) in decode order
   int64_t y_ld;
   float* yf;                 // DOWN: (rows, N) fp32
-  int64_t yf_ld;
+  int64_t yf_ld, yf_ss;      // and elements between its K splits (tile form)
   const float* c2;           // ZF: per (group, row) sum of x, (G, c2_ld) fp32
   int64_t c2_ld;
   float* part;               // split-K partial tiles (ks, tiles, TM, ntn*WGROWS) fp32, or null
@@ -84,7 +87,7 @@ struct PfArgs {
   int M, K, N, G, kw, rank;
   int ntn;                   // weight-row tiles of a workgroup along N
   int ks, gps;               // K splits, groups per split
-  int out_bits;              // GATE/UP: decode order of inter's consumer (2 or 4)
+  int out_bits;              // tile form: decode order of y's consumer (2, 4, or 0: natural)
   int max_tiles;             // token tiles in the grid (y dimension)
   float zoff;                // added to every zero-point (signed codes stored offset by 2^(b-1))
   // a = x U formed in the same launch (dense form, no K split; pf_xu_job):
@@ -956,6 +959,26 @@ static int pt_tiles_n(int64_t N, int mode, int tm) {
   return (int)((N + r - 1) / r);
 }
 
+// K splits of a DOWN launch of `wgs` workgroups over G groups: towards two
+// workgroups a CU, at least four groups each, at most 8 (whole quads of groups
+// where the rows' scales are).  Splits cost a fp32 pass over the results, so a
+// launch of 256 workgroups or more has none.  (256 tokens x 5632 -> 2048: 32
+// workgroups of 44 groups, 56 us unsplit.)
+static int pt_down_split(int64_t wgs, int G, int& gps) {
+  int ks = wgs >= 256 ? 1 : (int)std::min<int64_t>({8, 512 / wgs, std::max(1, G / 4)});
+  ks = std::max(ks, 1);
+  gps = (G + ks - 1) / ks;
+  if (G % 4 == 0) gps = (gps + 3) / 4 * 4;
+  return (G + gps - 1) / gps;
+}
+
+// fp32 elements pf_shared_launch may write to sy.
+static int64_t pf_shared_sy_elems(int64_t T, int64_t H, int64_t SI, int tm) {
+  int gps;
+  const int64_t wgs = (int64_t)pt_tiles_n(H, kPfDown, tm) * ((T + tm - 1) / tm);
+  return (int64_t)pt_down_split(wgs, (int)(SI / 128), gps) * T * H;
+}
+
 template <int MODE, bool SYM, bool ZF>
 static int pt_launch_tm(const PfArgs& g, int bits, int tm, hipStream_t s) {
   if (tm == 128) return pt_launch<2, 2, 2, MODE, SYM, ZF>(g, bits, s);
@@ -1251,7 +1274,10 @@ struct PfMoe {
   int32_t* tiles;          // (max_tiles, 3)
   int32_t* ntiles;
   const float* ybuf;       // (T * topk, H) routed outputs per sorted row
-  const float* sy;         // (T, H) shared expert output, or null
+  const float* sy;         // (sks, T, H) shared expert output in K splits, or null
+  int sks;
+  const __half* syh;       // or it as fp16
+  const __half* xsrc;      // rows that xp holds in decode order (null: h)
   const __half* res;       // (T, H) residual or null
   __half* out;             // (T, H)
 };
@@ -1288,30 +1314,44 @@ __device__ __forceinline__ void pf_permute16(int bits, u32x4 lo, u32x4 hi, u32x4
 // shared expert's when it differs), by 512 threads, four blocks in flight.
 __device__ __forceinline__ void pf_permute_rows(const PfMoe& a, int t0, int tid) {
   const int nb = a.H / 16, n = min(16, a.T - t0) * nb;  // 16-half blocks
-  const __half* src = a.h + (int64_t)t0 * a.H;
-  for (int i0 = tid; i0 < n; i0 += 4 * 512) {
-    u32x4 v[4][2];
+  for (int which = 0; which < 2; ++which) {
+    __half* dst = which ? a.xps : a.xp;
+    if (dst == nullptr || (which && dst == a.xp)) continue;
+    const __half* src = (which == 0 && a.xsrc ? a.xsrc : a.h) + (int64_t)t0 * a.H;
+    const int bits = which ? a.sbits : a.bits;
+    dst += (int64_t)t0 * a.H;
+    for (int i0 = tid; i0 < n; i0 += 4 * 512) {
+      u32x4 v[4][2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const __half* p = src + 16 * (int64_t)min(i0 + 512 * u, n - 1);
-      v[u][0] = *(const u32x4*)p;
-      v[u][1] = *(const u32x4*)(p + 8);
-    }
+      for (int u = 0; u < 4; ++u) {
+        const __half* p = src + 16 * (int64_t)min(i0 + 512 * u, n - 1);
+        v[u][0] = *(const u32x4*)p;
+        v[u][1] = *(const u32x4*)(p + 8);
+      }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = i0 + 512 * u;
-      if (i >= n) continue;
-      u32x4 o0, o1;
-      const int64_t at = (int64_t)t0 * a.H + 16 * (int64_t)i;
-      pf_permute16(a.bits, v[u][0], v[u][1], o0, o1);
-      *(u32x4*)(a.xp + at) = o0;
-      *(u32x4*)(a.xp + at + 8) = o1;
-      if (a.xps && a.xps != a.xp) {
-        pf_permute16(a.sbits, v[u][0], v[u][1], o0, o1);
-        *(u32x4*)(a.xps + at) = o0;
-        *(u32x4*)(a.xps + at + 8) = o1;
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + 512 * u;
+        if (i >= n) continue;
+        u32x4 o0, o1;
+        pf_permute16(bits, v[u][0], v[u][1], o0, o1);
+        *(u32x4*)(dst + 16 * (int64_t)i) = o0;
+        *(u32x4*)(dst + 16 * (int64_t)i + 8) = o1;
       }
     }
+  }
+}
+
+// n rows of 16-half blocks in the 4-bit decode order: two blocks a thread.
+__global__ __launch_bounds__(256) void pf_permute_kernel(const __half* src, int64_t blocks,
+                                                         __half* dst) {
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int64_t i = ((int64_t)blockIdx.x * 2 + u) * 256 + threadIdx.x;
+    if (i >= blocks) continue;
+    u32x4 o0, o1;
+    pf_permute16(4, *(const u32x4*)(src + 16 * i), *(const u32x4*)(src + 16 * i + 8), o0, o1);
+    *(u32x4*)(dst + 16 * i) = o0;
+    *(u32x4*)(dst + 16 * i + 8) = o1;
   }
 }
 
@@ -1392,7 +1432,8 @@ __global__ __launch_bounds__(512) void pf_moe_route_kernel(PfMoe a) {
     if (a.logits_out)
       for (int e = lane; e < a.E; e += 64)
         a.logits_out[(int64_t)tok * a.E + e] = __float2half(lg[t][e]);
-    if (a.sgw && lane == 0) a.sg[tok] = __float2half(1.f / (1.f + expf(-lg[t][a.E])));
+    if (lane == 0)
+      a.sg[tok] = __float2half(a.sgw ? 1.f / (1.f + expf(-lg[t][a.E])) : 1.f);
     // top-k: k rounds of the largest key (logit, then lower index) not yet
     // taken; key 0 is no expert
     uint32_t key[4];
@@ -1532,10 +1573,27 @@ __global__ __launch_bounds__(256) void pf_moe_combine_kernel(PfMoe a) {
         acc[3] = fmaf(w[u], v[u].w, acc[3]);
       }
   }
-  const float sg = a.sy ? __half2float(a.sg[t]) : 0.f;
+  const float sg = a.sy || a.syh ? __half2float(a.sg[t]) : 0.f;
+  float sh[4] = {0.f, 0.f, 0.f, 0.f};
+  if (a.sy)
+    for (int q0 = 0; q0 < a.sks; q0 += 4) {
+      float4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = *(const float4*)(a.sy + (int64_t)min(q0 + u, a.sks - 1) * a.T * a.H + i);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (q0 + u < a.sks) {
+          sh[0] += v[u].x;
+          sh[1] += v[u].y;
+          sh[2] += v[u].z;
+          sh[3] += v[u].w;
+        }
+    }
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    if (a.sy) acc[c] = fmaf(sg, __half2float(__float2half(a.sy[i + c])), acc[c]);
+    if (a.syh) acc[c] = fmaf(sg, __half2float(a.syh[i + c]), acc[c]);
+    else if (a.sy) acc[c] = fmaf(sg, __half2float(__float2half(sh[c])), acc[c]);
     float o = __half2float(__float2half(acc[c]));
     if (a.res) o += __half2float(a.res[i + c]);
     a.out[i + c] = __float2half(o);
@@ -1595,9 +1653,62 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
   P.off_inter = take(Pn * I * 2);
   P.off_y = take(Pn * H * 4);
   P.off_sinter = take(SI > 0 ? T * SI * 2 : 0);
-  P.off_sy = take(SI > 0 ? T * H * 4 : 0);
+  P.off_sy = take(SI > 0 ? pf_shared_sy_elems(T, H, SI, P.stm) * 4 : 0);
   P.total = o;
   return P;
+}
+
+// Launches 1-2 of a prompt: routing (and x in decode order), dispatch.
+static int pf_route_launch(const PfMoe& a, hipStream_t s) {
+  const int nt = (a.E + (a.sgw ? 1 : 0) + 31) / 32;  // pairs of 16-row router tiles
+  const auto kern = nt <= 1   ? pf_moe_route_kernel<1>
+                    : nt <= 2 ? pf_moe_route_kernel<2>
+                    : nt <= 4 ? pf_moe_route_kernel<4>
+                              : pf_moe_route_kernel<9>;
+  kern<<<dim3((unsigned)((a.T + 15) / 16), 2), dim3(512), 0, s>>>(a);
+  GLQ_LAUNCH_CHECK("pf_moe_route_kernel");
+  pf_moe_dispatch_kernel<<<dim3(1), dim3(1024), 0, s>>>(a);
+  GLQ_LAUNCH_CHECK("pf_moe_dispatch_kernel");
+  return GLQ_OK;
+}
+
+// The shared expert over every token: xps (T, H) in its decode order -> sy
+// (sks, T, H) fp32 in K splits, through sinter (T, SI).
+static int pf_shared_launch(int64_t T, int64_t H, int64_t SI, int bits, int tm, const __half* xps,
+                            const int32_t* const codes[3], const void* const scales[3],
+                            const void* const zeros[3], __half* sinter, float* sy, int& sks,
+                            hipStream_t s) {
+  const int ntm = (int)((T + tm - 1) / tm);
+  PfArgs g = {};
+  g.xp = xps;
+  for (int m = 0; m < 2; ++m) {
+    g.codes[m] = (const uint32_t*)codes[m];
+    g.scales[m] = (const __half*)scales[m];
+    g.zeros[m] = (const __half*)zeros[m];
+  }
+  g.y = sinter;
+  g.y_ld = SI;
+  g.M = (int)T; g.K = (int)H; g.N = (int)SI; g.G = (int)(H / 128);
+  g.kw = (int)(H * bits / 32);
+  g.ntn = pt_tiles_n(SI, kPfGateUp, tm);
+  g.out_bits = bits;
+  g.max_tiles = ntm;
+  int rc = pt_launch_tm<kPfGateUp, false, false>(g, bits, tm, s);
+  if (rc) return rc;
+  PfArgs d = {};
+  d.xp = sinter;
+  d.codes[0] = (const uint32_t*)codes[2];
+  d.scales[0] = (const __half*)scales[2];
+  d.zeros[0] = (const __half*)zeros[2];
+  d.yf = sy;
+  d.yf_ld = H;
+  d.M = (int)T; d.K = (int)SI; d.N = (int)H; d.G = (int)(SI / 128);
+  d.kw = (int)(SI * bits / 32);
+  d.ntn = pt_tiles_n(H, kPfDown, tm);
+  d.max_tiles = ntm;
+  d.ks = sks = pt_down_split((int64_t)d.ntn * ntm, d.G, d.gps);
+  d.yf_ss = T * H;
+  return pt_launch_tm<kPfDown, false, false>(d, bits, tm, s);
 }
 
 static int pf_moe_check(const glq_moe_params* p) {
@@ -1697,17 +1808,8 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
   float* lp = (float*)(w + P.off_lp);
 
   // 1-2. routing and dispatch
-  {
-    const int nt = (int)((E + (a.sgw ? 1 : 0) + 31) / 32);  // pairs of 16-row router tiles
-    const auto kern = nt <= 1   ? pf_moe_route_kernel<1>
-                      : nt <= 2 ? pf_moe_route_kernel<2>
-                      : nt <= 4 ? pf_moe_route_kernel<4>
-                                : pf_moe_route_kernel<9>;
-    kern<<<dim3((unsigned)((T + 15) / 16), 2), dim3(512), 0, s>>>(a);
-  }
-  GLQ_LAUNCH_CHECK("pf_moe_route_kernel");
-  pf_moe_dispatch_kernel<<<dim3(1), dim3(1024), 0, s>>>(a);
-  GLQ_LAUNCH_CHECK("pf_moe_dispatch_kernel");
+  rc = pf_route_launch(a, s);
+  if (rc) return rc;
 
   // expert strides (elements)
   const int64_t kw_gu = H * p->bits / 32, kw_d = I * p->bits / 32;
@@ -1815,42 +1917,300 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
   }
   // 7. shared expert over every token
   if (SI > 0) {
-    const int sb = p->shared_bits;
-    __half* sinter = (__half*)(w + P.off_sinter);
-    const int ntm = (int)((T + P.stm - 1) / P.stm);
-    PfArgs g = {};
-    g.xp = a.xps;
-    for (int m = 0; m < 2; ++m) {
-      g.codes[m] = (const uint32_t*)p->shared_codes[m];
-      g.scales[m] = (const __half*)p->shared_scales[m];
-      g.zeros[m] = (const __half*)p->shared_zeros[m];
-    }
-    g.y = sinter;
-    g.y_ld = SI;
-    g.M = (int)T; g.K = (int)H; g.N = (int)SI; g.G = (int)(H / 128);
-    g.kw = (int)(H * sb / 32);
-    g.ntn = pt_tiles_n(SI, kPfGateUp, P.stm);
-    g.ks = 1; g.gps = g.G;
-    g.out_bits = sb;
-    g.max_tiles = ntm;
-    rc = pt_launch_tm<kPfGateUp, false, false>(g, sb, P.stm, s);
-    if (rc) return rc;
-    PfArgs d = {};
-    d.xp = sinter;
-    d.codes[0] = (const uint32_t*)p->shared_codes[2];
-    d.scales[0] = (const __half*)p->shared_scales[2];
-    d.zeros[0] = (const __half*)p->shared_zeros[2];
-    d.yf = (float*)(w + P.off_sy);
-    d.yf_ld = H;
-    d.M = (int)T; d.K = (int)SI; d.N = (int)H; d.G = (int)(SI / 128);
-    d.kw = (int)(SI * sb / 32);
-    d.ntn = pt_tiles_n(H, kPfDown, P.stm);
-    d.ks = 1; d.gps = d.G;
-    d.max_tiles = ntm;
-    rc = pt_launch_tm<kPfDown, false, false>(d, sb, P.stm, s);
+    rc = pf_shared_launch(T, H, SI, p->shared_bits, P.stm, a.xps, p->shared_codes,
+                          p->shared_scales, p->shared_zeros, (__half*)(w + P.off_sinter),
+                          (float*)(w + P.off_sy), a.sks, s);
     if (rc) return rc;
   }
   // 8. combine
+  pf_moe_combine_kernel<<<dim3((unsigned)((T * H / 4 + 255) / 256)), dim3(256), 0, s>>>(a);
+  GLQ_LAUNCH_CHECK("pf_moe_combine_kernel");
+  return GLQ_OK;
+}
+
+namespace glq {
+// ===========================================================================
+// A TurboQuant block over a prompt (glq_turbo_moe_prefill): the steps of
+// glq_moe_prefill with the experts' inputs rotated before their codebook
+// GEMMs (the reference's _forward_sparse on TurboQuant layers,
+// inference/moe_block.py:704-740, quantized_linear.py:315-349).  x U takes the
+// unrotated inputs.  As consecutive 16-token decode steps each read the picked
+// experts again: 256 tokens through the 60-expert block took 16 steps, 2.2 ms.
+// ===========================================================================
+struct TpPlan {
+  int tm, max_tiles, stm, ks_gu, kps_gu, ks_d, kps_d;
+  int64_t off_xr, off_xp, off_xps, off_sel, off_wts, off_sg, off_pos, off_stok, off_tiles, off_lp,
+      off_agu, off_ad, off_inter, off_tmp, off_xd, off_y, off_sinter, off_sy, total;
+};
+
+static TpPlan tp_plan(const glq_turbo_prefill_params* p) {
+  const int64_t T = p->tokens, H = p->hidden, E = p->experts, I = p->inter, k = p->top_k;
+  const int64_t r = p->rank, SI = p->shared_inter, Pn = T * k;
+  TpPlan P;
+  P.tm = Pn / std::max<int64_t>(E, 1) < 46 ? 32 : 64;  // as pf_moe_plan's tiles
+  P.max_tiles = (int)((Pn + P.tm - 1) / P.tm + E);
+  P.stm = T > 32 ? 64 : 32;
+  const int64_t lrb = (Pn + kLrRows - 1) / kLrRows + std::min<int64_t>(E, Pn) / 2;
+  pf_lowrank_split(H, lrb, P.ks_gu, P.kps_gu);
+  pf_lowrank_split(I, lrb, P.ks_d, P.kps_d);
+  int64_t o = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = o;
+    o = align_up(o + bytes, 256);
+    return at;
+  };
+  P.off_xr = take(T * H * 2);
+  P.off_xp = take(T * H * 2);
+  P.off_xps = take(SI > 0 ? T * H * 2 : 0);
+  P.off_sel = take(Pn * 4);
+  P.off_wts = take(Pn * 2);
+  P.off_sg = take(T * 2);
+  P.off_pos = take(Pn * 4);
+  P.off_stok = take(Pn * 4);
+  P.off_tiles = take((int64_t)P.max_tiles * 12 + 4);
+  const int64_t lp = r > 0 ? std::max<int64_t>(P.ks_gu > 1 ? P.ks_gu * Pn * 2 * r * 4 : 0,
+                                               P.ks_d > 1 ? P.ks_d * Pn * r * 4 : 0)
+                           : 0;
+  P.off_lp = take(lp);
+  P.off_agu = take(Pn * 2 * r * 2);
+  P.off_ad = take(Pn * r * 2);
+  P.off_inter = take(Pn * I * 2);
+  P.off_tmp = take(p->signs[1] ? Pn * I * 2 : 0);
+  P.off_xd = take(Pn * I * 2);
+  P.off_y = take(Pn * H * 4);
+  P.off_sinter = take(SI > 0 ? T * SI * 2 : 0);
+  P.off_sy = take(SI > 0 ? pf_shared_sy_elems(T, H, SI, P.stm) * 4 : 0);
+  P.total = o;
+  return P;
+}
+
+static int tp_check(const glq_turbo_prefill_params* p) {
+  GLQ_CHECK(p != nullptr, "null params");
+  const int64_t T = p->tokens, H = p->hidden, E = p->experts, I = p->inter, k = p->top_k;
+  GLQ_CHECK(T >= 1 && T <= (1 << 20), "tokens=%lld must be in 1..%d", (long long)T, 1 << 20);
+  GLQ_CHECK(E >= 1 && E <= 256, "experts=%lld must be in 1..256", (long long)E);
+  GLQ_CHECK(k >= 1 && k <= 16 && k <= E, "top_k=%lld out of range", (long long)k);
+  GLQ_CHECK(H >= 128 && H % 128 == 0 && H <= (1 << 16), "hidden=%lld must be a multiple of 128",
+            (long long)H);
+  GLQ_CHECK(I >= 128 && I % 128 == 0 && I <= (1 << 16), "inter=%lld must be a multiple of 128",
+            (long long)I);
+  GLQ_CHECK(T * H < (1ll << 31) && T * k * std::max(I, H) < (1ll << 31), "tokens x width too large");
+  GLQ_CHECK(p->rank >= 0 && p->rank % 8 == 0 && p->rank <= 128,
+            "rank=%lld must be a multiple of 8, <= 128", (long long)p->rank);
+  const int64_t SI = p->shared_inter;
+  GLQ_CHECK(SI >= 0 && SI % 128 == 0 && SI <= (1 << 17) && T * std::max<int64_t>(SI, 1) < (1ll << 31),
+            "shared_inter=%lld must be a multiple of 128", (long long)SI);
+  GLQ_CHECK(SI == 0 || p->shared_bits == 2 || p->shared_bits == 4, "shared_bits must be 2 or 4");
+  GLQ_CHECK(SI == 0 || p->shared_y == nullptr, "shared weights or a shared output, not both");
+  GLQ_CHECK(p->h && p->router_w && p->out, "null h, router_w or out");
+  auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
+  GLQ_CHECK(al16(p->h) && al16(p->router_w) && (!p->shared_gate_w || al16(p->shared_gate_w)),
+            "h, router_w and shared_gate_w must be 16-byte aligned");
+  for (int i = 0; i < 3; ++i) {
+    GLQ_CHECK(p->codes[i] && p->norms[i] && p->centroids[i] && al16(p->codes[i]),
+              "codes (16-byte aligned), norms and centroids are needed (proj %d)", i);
+    if (p->rank > 0)
+      GLQ_CHECK(p->U[i] && p->cluster_of[i] && p->SV[i] && al16(p->U[i]) && al16(p->SV[i]),
+                "U, cluster_of and SV (16-byte aligned) are needed with a rank");
+    if (SI > 0)
+      GLQ_CHECK(p->shared_codes[i] && p->shared_scales[i] && p->shared_zeros[i] &&
+                    al16(p->shared_codes[i]),
+                "null or misaligned shared-expert weights (proj %d)", i);
+  }
+  for (int i = 0; i < 2; ++i) {
+    GLQ_CHECK((p->signs[i] != nullptr) != (p->Pi[i] != nullptr),
+              "one rotation, signs or Pi, is needed for %s", i ? "down" : "gate and up");
+    const int64_t d = i ? I : H;
+    GLQ_CHECK(p->Pi[i] == nullptr || al16(p->Pi[i]), "Pi must be 16-byte aligned");
+    GLQ_CHECK(p->signs[i] == nullptr || ((d & (d - 1)) == 0 && d <= 32768),
+              "the Hadamard transform takes a power of two <= 32768 (got %lld)", (long long)d);
+  }
+  return GLQ_OK;
+}
+
+// out (rows, d) = fp16(x Pi^T) in the 4-bit decode order.
+static int tp_rotate(const __half* x, int64_t rows, int64_t d, const void* Pi, __half* out,
+                     hipStream_t s) {
+  PfArgs g = {};
+  g.xp = x;
+  g.codes[0] = (const uint32_t*)Pi;
+  g.y = out;
+  g.y_ld = d;
+  g.out_bits = 4;
+  g.M = (int)rows; g.K = (int)d; g.N = (int)d; g.G = (int)(d / 128);
+  g.ntn = (int)((d + 127) / 128);
+  g.max_tiles = (int)((rows + 63) / 64);
+  return pt_launch_k<kPtHalf, 2, 2, 1, kPfDense, false, false, false>(g, s);
+}
+
+template <int MODE>
+static int tp_gemm(const PfArgs& g, int tm, hipStream_t s) {
+  if (tm == 64) return pt_launch_k<kPtTurbo, 1, 4, 2, MODE, false, false, false>(g, s);
+  return pt_launch_k<kPtTurbo, 1, 4, 1, MODE, false, false, false>(g, s);
+}
+}  // namespace glq
+
+extern "C" int64_t glq_turbo_moe_prefill_workspace_bytes(const glq_turbo_prefill_params* p) {
+  using namespace glq;
+  clear_error();
+  return tp_check(p) == GLQ_OK ? tp_plan(p).total : -1;
+}
+
+extern "C" int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  using namespace glq;
+  clear_error();
+  int rc = tp_check(p);
+  if (rc) return rc;
+  const int64_t T = p->tokens, H = p->hidden, E = p->experts, I = p->inter, k = p->top_k;
+  const int64_t SI = p->shared_inter, Pn = T * k, r = p->rank;
+  const TpPlan P = tp_plan(p);
+  GLQ_CHECK(workspace != nullptr && workspace_bytes >= P.total && ((uintptr_t)workspace & 255) == 0,
+            "a 256-byte aligned workspace of %lld bytes is needed (got %lld)", (long long)P.total,
+            (long long)workspace_bytes);
+  hipStream_t s = (hipStream_t)stream;
+  char* w = (char*)workspace;
+  auto hp = [&](int64_t off) { return (__half*)(w + off); };
+  PfMoe a = {};
+  a.T = (int)T; a.H = (int)H; a.E = (int)E; a.I = (int)I; a.topk = (int)k;
+  a.norm = p->norm_topk_prob ? 1 : 0;
+  a.SI = (int)SI; a.bits = 4; a.sbits = SI > 0 ? p->shared_bits : 4;
+  a.tm = P.tm; a.max_tiles = P.max_tiles;
+  a.h = (const __half*)p->h;
+  a.router_w = (const __half*)p->router_w;
+  a.sgw = (const __half*)p->shared_gate_w;
+  a.logits_out = (__half*)p->router_logits;
+  a.xps = SI > 0 ? hp(P.off_xps) : nullptr;
+  a.sel = (int32_t*)(w + P.off_sel);
+  a.wts = hp(P.off_wts);
+  a.sg = hp(P.off_sg);
+  a.pos = (int32_t*)(w + P.off_pos);
+  a.stok = (int32_t*)(w + P.off_stok);
+  a.tiles = (int32_t*)(w + P.off_tiles);
+  a.ntiles = a.tiles + 3 * P.max_tiles;
+  a.ybuf = (const float*)(w + P.off_y);
+  a.sy = SI > 0 ? (const float*)(w + P.off_sy) : nullptr;
+  a.syh = (const __half*)p->shared_y;
+  a.res = (const __half*)p->residual;
+  a.out = (__half*)p->out;
+  // 1. gate/up's input: the transform of h (put in decode order by the routing
+  // launch), or h Pi^T
+  if (p->signs[0]) {
+    rc = glq_rht(p->h, 0, T, H, p->signs[0], 0, hp(P.off_xr), 0, stream);
+    a.xsrc = hp(P.off_xr);
+    a.xp = hp(P.off_xp);
+  } else {
+    rc = tp_rotate(a.h, T, H, p->Pi[0], hp(P.off_xp), s);
+  }
+  if (rc) return rc;
+  // 2-3. routing and dispatch
+  rc = pf_route_launch(a, s);
+  if (rc) return rc;
+  // 4. a = x U for gate and up per pair, 5. gate/up + SwiGLU -> inter
+  auto lowrank = [&](const __half* x, const int32_t* arow, int m0, int nmat, int64_t K, int ks,
+                     int kps, __half* out) {
+    PfLowrank L = {};
+    L.x = x;
+    L.arow = arow;
+    L.nmat = nmat;
+    for (int m = 0; m < nmat; ++m) {
+      L.U[m] = (const __half*)p->U[m0 + m];
+      L.cluster[m] = p->cluster_of[m0 + m];
+    }
+    L.u_cs = K * r;
+    L.tiles = a.tiles;
+    L.ntiles = a.ntiles;
+    L.tile_rows = P.tm;
+    L.rows_total = (int)Pn;
+    L.K = (int)K;
+    L.rank = (int)r;
+    L.ks = ks;
+    L.kps = kps;
+    L.part = (float*)(w + P.off_lp);
+    L.a_out = out;
+    return pf_lowrank_launch(L, P.max_tiles * ((P.tm + kLrRows - 1) / kLrRows), s);
+  };
+  if (r > 0) {
+    rc = lowrank(a.h, a.stok, 0, 2, H, P.ks_gu, P.kps_gu, hp(P.off_agu));
+    if (rc) return rc;
+  }
+  __half* inter = hp(P.off_inter);
+  {
+    PfArgs g = {};
+    g.xp = hp(P.off_xp);
+    g.arow = a.stok;
+    for (int m = 0; m < 2; ++m) {
+      g.codes[m] = (const uint32_t*)p->codes[m];
+      g.norms[m] = p->norms[m];
+      g.cent[m] = p->centroids[m];
+      g.sv[m] = r > 0 ? (const __half*)p->SV[m] : nullptr;
+    }
+    g.kw = (int)(H / 16);
+    g.codes_es = I * g.kw;
+    g.n_es = I;
+    g.a = r > 0 ? hp(P.off_agu) : nullptr;
+    g.a_ld = (int)(2 * r);
+    g.sv_es = I * r;
+    g.y = inter;
+    g.y_ld = I;
+    g.tiles = a.tiles;
+    g.ntiles = a.ntiles;
+    g.M = (int)Pn; g.K = (int)H; g.N = (int)I; g.G = (int)(H / 128);
+    g.rank = (int)r;
+    g.ntn = pt_tiles_n(I, kPfGateUp, P.tm);
+    g.max_tiles = P.max_tiles;
+    rc = tp_gemm<kPfGateUp>(g, P.tm, s);
+    if (rc) return rc;
+  }
+  // 6. a = inter U_down per pair, 7. the down's input rotated, in decode order
+  if (r > 0) {
+    rc = lowrank(inter, nullptr, 2, 1, I, P.ks_d, P.kps_d, hp(P.off_ad));
+    if (rc) return rc;
+  }
+  if (p->signs[1]) {
+    rc = glq_rht(inter, 0, Pn, I, p->signs[1], 0, hp(P.off_tmp), 0, stream);
+    if (rc) return rc;
+    const int64_t blocks = Pn * I / 16;
+    pf_permute_kernel<<<dim3((unsigned)((blocks + 511) / 512)), dim3(256), 0, s>>>(
+        hp(P.off_tmp), blocks, hp(P.off_xd));
+    GLQ_LAUNCH_CHECK("pf_permute_kernel");
+  } else {
+    rc = tp_rotate(inter, Pn, I, p->Pi[1], hp(P.off_xd), s);
+    if (rc) return rc;
+  }
+  // 8. down -> y per sorted row (fp32)
+  {
+    PfArgs g = {};
+    g.xp = hp(P.off_xd);
+    g.codes[0] = (const uint32_t*)p->codes[2];
+    g.norms[0] = p->norms[2];
+    g.cent[0] = p->centroids[2];
+    g.sv[0] = r > 0 ? (const __half*)p->SV[2] : nullptr;
+    g.kw = (int)(I / 16);
+    g.codes_es = H * g.kw;
+    g.n_es = H;
+    g.a = r > 0 ? hp(P.off_ad) : nullptr;
+    g.a_ld = (int)r;
+    g.sv_es = H * r;
+    g.yf = (float*)(w + P.off_y);
+    g.yf_ld = H;
+    g.tiles = a.tiles;
+    g.ntiles = a.ntiles;
+    g.M = (int)Pn; g.K = (int)I; g.N = (int)H; g.G = (int)(I / 128);
+    g.rank = (int)r;
+    g.ntn = pt_tiles_n(H, kPfDown, P.tm);
+    g.ks = 1; g.gps = g.G;
+    g.max_tiles = P.max_tiles;
+    rc = tp_gemm<kPfDown>(g, P.tm, s);
+    if (rc) return rc;
+  }
+  // 9. shared expert, 10. combine
+  if (SI > 0) {
+    rc = pf_shared_launch(T, H, SI, p->shared_bits, P.stm, a.xps, p->shared_codes,
+                          p->shared_scales, p->shared_zeros, hp(P.off_sinter),
+                          (float*)(w + P.off_sy), a.sks, s);
+    if (rc) return rc;
+  }
   pf_moe_combine_kernel<<<dim3((unsigned)((T * H / 4 + 255) / 256)), dim3(256), 0, s>>>(a);
   GLQ_LAUNCH_CHECK("pf_moe_combine_kernel");
   return GLQ_OK;

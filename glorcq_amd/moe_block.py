@@ -31,7 +31,8 @@ Differences:
   pick; the shared expert (its own GLoRCQLinear projections); and the
   weighted combine with the gated shared term (glq_moe_combine).  Each step
   reads only the picked experts' weights (the reference's graph mode runs
-  all E, :742-890).
+  all E, :742-890).  More than 16 tokens run as one glq_turbo_moe_prefill
+  (grouped codebook GEMMs over each expert's tokens).
 """
 
 from __future__ import annotations
@@ -276,6 +277,10 @@ class GraphCompatibleMoeBlock(nn.Module):
                 raise RuntimeError("residual must match hidden_states (fp16)")
             res = residual.reshape(-1, self.hidden).contiguous()
         t = self.t
+        if self.kind == "turbo" and _turbo_prefill_ok(self, h.shape[0]):
+            out, lg = turbo_prefill(self, h, res)
+            out = out.reshape(shape)
+            return (out, lg) if self.return_router_logits else out
         if self.kind == "turbo":
             outs, logits = [], []
             for t0 in range(0, h.shape[0], TURBO_MAX_TOKENS):
@@ -431,10 +436,16 @@ def _turbo_derived(t: dict) -> None:
     for proj in PROJS:
         Pi = t[f"Pi_{proj}"]
         t[f"PiT_{proj}"] = None if Pi is None else Pi.t().contiguous()
-    # Pi of down as fp16 rows (output n's weights contiguous), for
-    # glq_turbo_moe_down_prep
-    Pd = t["Pi_down"]
-    t["Pi_down_c"] = None if Pd is None else Pd.to(torch.float16).contiguous()
+    # Pi as fp16 rows (output n's weights contiguous): down's for
+    # glq_turbo_moe_down_prep, and gate/up's for glq_turbo_moe_prefill
+    for proj in ("gate", "down"):
+        Pi = t[f"Pi_{proj}"]
+        t[f"Pi_{proj}_c"] = None if Pi is None else Pi.to(torch.float16).contiguous()
+    # glq_turbo_moe_prefill's shared GEMMs take integer zero-points; checked
+    # once here
+    sw = _turbo_shared_weights(t)
+    t["shared_zeros_integral"] = sw is not None and all(
+        bool(torch.equal(z, z.round())) for z in sw[2])
     if t["rank"] > 0:
         t["U_gu"] = torch.cat([t["U_gate"], t["U_up"]]).contiguous()
 
@@ -728,6 +739,66 @@ def turbo_step(blk: GraphCompatibleMoeBlock, h: torch.Tensor, res: torch.Tensor 
     _lib.check(lib.glq_moe_combine(yd.data_ptr(), wts.data_ptr(), _lib.ptr(shared), sg.data_ptr(),
                                    _lib.ptr(res), B, H, k, out.data_ptr(), stream),
                "glq_moe_combine")
+    return out, logits
+
+
+def _turbo_prefill_ok(blk: GraphCompatibleMoeBlock, T: int) -> bool:
+    """More than one step's tokens go through glq_turbo_moe_prefill when it
+    takes the block: gate and up rotated alike, widths of whole 128-code
+    groups, a rank that is a multiple of 8 (at most 128)."""
+    t = blk.t
+    return (T > TURBO_MAX_TOKENS and not os.environ.get("GLQ_TURBO_SEQ") and t["same_rot_gu"]
+            and blk.hidden % 128 == 0 and blk.hidden <= 4096  # the decode router's limit
+            and blk.inter % 128 == 0 and blk.num_experts <= 256
+            and blk.top_k <= 16 and blk.rank % 8 == 0 and blk.rank <= 128
+            and blk.inter <= 1 << 16
+            and T * blk.top_k * max(blk.hidden, blk.inter, blk.shared_inter) < 1 << 31)
+
+
+def turbo_prefill(blk: GraphCompatibleMoeBlock, h: torch.Tensor, res: torch.Tensor | None):
+    """A prompt through a TurboQuant block (glq_turbo_moe_prefill): (out (T, H)
+    fp16, router logits (T, E) fp16).  A shared expert whose weights its
+    grouped GEMMs do not take runs as its own projections first."""
+    lib = _lib.load()
+    t = blk.t
+    T, H = h.shape
+    out = torch.empty_like(h)
+    logits = torch.empty(T, blk.num_experts, dtype=torch.float16, device=h.device)
+    p = _lib.TurboPrefillParams()
+    p.tokens, p.hidden, p.experts, p.inter = T, H, blk.num_experts, blk.inter
+    p.top_k, p.rank, p.norm_topk_prob = blk.top_k, blk.rank, int(blk.norm_topk_prob)
+    p.h, p.router_w = h.data_ptr(), t["router_w"].data_ptr()
+    p.shared_gate_w = _lib.ptr(t["shared_gate_w"])
+    for i, proj in enumerate(PROJS):
+        p.codes[i] = t[f"words_{proj}"].data_ptr()
+        p.norms[i] = t[f"norms_{proj}"].data_ptr()
+        p.centroids[i] = t[f"cent_{proj}"].data_ptr()
+        if blk.rank:
+            p.U[i] = t[f"U_{proj}"].data_ptr()
+            p.cluster_of[i] = t[f"cluster_{proj}"].data_ptr()
+            p.SV[i] = t[f"SV_{proj}"].data_ptr()
+    for i, proj in enumerate(("gate", "down")):
+        p.signs[i] = _lib.ptr(t[f"signs_{proj}"])
+        p.Pi[i] = None if t[f"signs_{proj}"] is not None else _lib.ptr(t[f"Pi_{proj}_c"])
+    shared = None
+    if blk.shared_inter > 0:
+        sw = _turbo_shared_weights(t)
+        if sw is not None and t["shared_zeros_integral"] and blk.shared_inter % 128 == 0:
+            p.shared_inter, p.shared_bits = blk.shared_inter, 4
+            for i in range(3):
+                p.shared_codes[i] = sw[0][i].data_ptr()
+                p.shared_scales[i], p.shared_zeros[i] = sw[1][i].data_ptr(), sw[2][i].data_ptr()
+        else:
+            shared = _turbo_shared_expert(t, h, lib)
+            p.shared_y = shared.data_ptr()
+    p.residual, p.out, p.router_logits = _lib.ptr(res), out.data_ptr(), logits.data_ptr()
+    n = lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(p))
+    if n < 0:
+        _lib.check(1, "glq_turbo_moe_prefill_workspace_bytes")
+    from .kernels import workspace
+    ws = workspace(h.device, max(int(n), 256))
+    _lib.check(lib.glq_turbo_moe_prefill(ctypes.byref(p), ws.data_ptr(), ws.numel(),
+                                         _lib.stream_handle(h.device)), "glq_turbo_moe_prefill")
     return out, logits
 
 

@@ -533,6 +533,47 @@ int glq_turbo_moe_gemv(int64_t picks, int64_t x_div, const void* x_rot, int64_t 
                        void* y, void* stream);
 
 /*
+ * A TurboQuant block over a prompt: routing, then every routed expert's
+ * codebook projections as grouped GEMMs over its tokens, the shared expert,
+ * the weighted sum (the reference's _forward_sparse, inference/moe_block.py:
+ * 704-740, on TurboQuant layers; the decode step's routing and combine).
+ * Projections in the order gate, up, down: codes (experts, N, K/16) words,
+ * norms (experts, N), centroids (4,), SV (experts, N, rank), U (rows, K,
+ * rank) at row cluster_of[expert].  Rotations [0] of gate and up's input,
+ * [1] of down's: signs (fp32, a power-of-two width) or Pi (width, width)
+ * fp16 rows, x_rot = fp16(x Pi^T).  The shared expert: 2- or 4-bit group-128
+ * weights with integer zero-points (shared_inter > 0), or its output
+ * shared_y (tokens, hidden), or none.  residual may be NULL.  hidden, inter
+ * and shared_inter are multiples of 128, rank of 8 (<= 128; 0: none).
+ */
+typedef struct glq_turbo_prefill_params {
+  int64_t tokens, hidden, experts, inter, top_k, rank, shared_inter;
+  int32_t norm_topk_prob, shared_bits;
+  const void* h;
+  const void* router_w;
+  const void* shared_gate_w;
+  const int32_t* codes[3];
+  const float* norms[3];
+  const float* centroids[3];
+  const void* U[3];
+  const int32_t* cluster_of[3];
+  const void* SV[3];
+  const float* signs[2];
+  const void* Pi[2];
+  const int32_t* shared_codes[3];
+  const void* shared_scales[3];
+  const void* shared_zeros[3];
+  const void* shared_y;
+  const void* residual;
+  void* out;
+  void* router_logits;
+} glq_turbo_prefill_params;
+
+int64_t glq_turbo_moe_prefill_workspace_bytes(const glq_turbo_prefill_params* p);
+int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
+/*
  * out[t] = fp16(sum_k weights[t][k] y[t top_k + k] + shared_gate[t] shared[t])
  * (+ residual[t]): the block's weighted sum (moe_block.py:470-476) and the
  * gated shared expert (:429-435) in fp32, rounded once (shared NULL: no

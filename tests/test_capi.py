@@ -280,3 +280,39 @@ def test_gptq_signature_refuses_unprepared_codes_under_capture(monkeypatch):
     q = torch.zeros(16, 128, dtype=torch.int32)
     with pytest.raises(RuntimeError, match="not prepared before graph capture"):
         kernels.gptq_dequant_matmul_fused(x, q, s, s, 128, False)
+
+
+def test_turbo_prefill_checks_arguments(lib):
+    """glq_turbo_moe_prefill rejects bad shapes and pointers on the host."""
+    import ctypes
+
+    from glorcq_amd import _lib
+
+    def params(**kw):
+        q = _lib.TurboPrefillParams()
+        base = dict(tokens=40, hidden=512, experts=8, inter=384, top_k=2, rank=16,
+                    h=1 << 12, router_w=1 << 12, out=1 << 12)
+        for k, v in {**base, **kw}.items():
+            setattr(q, k, v)
+        for i in range(3):
+            for f in ("codes", "norms", "centroids", "U", "cluster_of", "SV"):
+                getattr(q, f)[i] = 1 << 12
+        q.signs[0], q.Pi[1] = 1 << 12, 1 << 12
+        return q
+
+    need = lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(params()))
+    assert need > 0
+    assert lib.glq_turbo_moe_prefill(ctypes.byref(params()), 1 << 12, need - 1, None) == 1
+    assert b"workspace" in lib.glq_last_error()
+    for kw, word in ((dict(hidden=500), b"hidden"), (dict(inter=300), b"inter"),
+                     (dict(rank=12), b"rank"), (dict(rank=136), b"rank"),
+                     (dict(top_k=9), b"top_k"), (dict(experts=300), b"experts"),
+                     (dict(h=(1 << 12) + 2), b"aligned"), (dict(out=None), b"null"),
+                     (dict(shared_inter=128, shared_bits=4), b"shared")):
+        assert lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(params(**kw))) == -1
+        assert word in lib.glq_last_error(), (kw, lib.glq_last_error())
+    q = params()
+    q.signs[1] = 1 << 12  # two rotations of the down's input
+    assert lib.glq_turbo_moe_prefill(ctypes.byref(q), 1 << 12, 1 << 30, None) == 1
+    q = params(hidden=384, inter=512)  # the transform takes powers of two
+    assert lib.glq_turbo_moe_prefill(ctypes.byref(q), 1 << 12, 1 << 30, None) == 1

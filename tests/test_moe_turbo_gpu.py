@@ -253,3 +253,37 @@ def test_turbo_fused_step_matches_launch_sequence(gpu, B, seed, inter, rot_gu, r
     ref = O.moe_forward(p)
     for out in (out_f, out_s):
         assert bar(out.reshape(p.B, p.H).cpu(), ref)
+
+
+@pytest.mark.parametrize("T,H,inter,rot_gu,rot_down,rank,shared", [
+    (17, 512, 384, "rht", "qr", 64, 0),      # one token past a step, 32-token tiles
+    (65, 1024, 512, "qr", "rht", 24, 512),   # one over a 64-row block; both rotations swapped
+    (100, 256, 256, "rht", "rht", 0, 0),     # no low-rank term
+    (300, 512, 640, "rht", "qr", 128, 384),  # 64-token tiles; two column blocks of x U
+], ids=str)
+def test_turbo_prompt(gpu, T, H, inter, rot_gu, rot_down, rank, shared):
+    """More than a step's tokens as one prompt (glq_turbo_moe_prefill): edges of
+    the token tiles and row blocks, either rotation on either side, ranks of
+    one and two column blocks, the shared expert in the launches and, with
+    zero-points that are not integers, as its own projections."""
+    kw = dict(H=H, E=6, inter=inter, top_k=2, n_clusters=3, rank=rank, shared_inter=shared,
+              rot_gate_up=rot_gu, rot_down=rot_down)
+    seed = next(s for s in range(3, 60)
+                if margin(fmt.make_turbo_moe(B=T, seed=s, **kw)) >= 2)
+    p = fmt.make_turbo_moe(B=T, seed=seed, **kw)
+    if rank:
+        p = lora_heavy(p, 10.0)
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+    res = (torch.randn(1, T, H, generator=torch.Generator().manual_seed(T)) * 0.5).half()
+    out, logits = blk(p.h.reshape(1, T, H).to(gpu), residual=res.to(gpu))
+    torch.cuda.synchronize()
+    check_routing(p, logits.cpu())
+    ref = O.moe_forward(p).half().double() + res.reshape(T, H).double()
+    assert bar(out.reshape(T, H).cpu(), ref)
+    if shared:
+        for proj in fmt.PROJS:
+            p.shared[proj].zeros = (p.shared[proj].zeros.float() + 0.25).half()
+        blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+        assert not blk.t["shared_zeros_integral"]
+        out, _ = run(blk, p, gpu)
+        assert bar(out, O.moe_forward(p))
