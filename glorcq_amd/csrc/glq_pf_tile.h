@@ -26,8 +26,8 @@
 //    the words of its half of K, k-step t (0..7) uses slice t of them, and the
 //    A operand of step t is decode-order piece 8 h + t of a token's row.
 //  * Scales and zero-points: lanes of half 0 load the scale, of half 1 the
-//    zero-point, and one v_permlane32_swap gives both to both; four groups a
-//    load where the rows' scales are whole aligned quads (SZQ), else one.
+//    zero-point, and one v_permlane32_swap gives both to both; two groups a
+//    load where the rows' scales are whole aligned pairs (SZQ), else one.
 //  * y += s (acc - zf c2) as in pf_gemm_kernel.
 #pragma once
 
@@ -242,12 +242,13 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
 
   // one group's products of NM token blocks
   auto group = [&](auto nm, int grp, const unsigned char* sl, const __half (&sh)[2],
-                   const __half (&zh)[2]) {
+                   const __half (&zh)[2], const auto& after_reads) {
     constexpr int NM = decltype(nm)::value;
     auto arow = [&](int i) { return sl + (32 * (i * WM + wm) + li) * 256; };
     auto piece = [&](int i, int p) { return *(const u32x4*)(arow(i) + ((p ^ (li & 15)) << 4)); };
     auto a_op = [&](int i, int t) { return __builtin_bit_cast(f16x8, piece(i, 8 * h + t)); };
     if constexpr (BITS == kPtHalf) {
+      after_reads();
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
         f16x8 bv[2];
@@ -278,6 +279,7 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
           for (int i = 0; i < NM; ++i) av[i4 & 1][sl2][i] = a_op(i, 2 * i4 + sl2);
       };
       load_a(0);
+      after_reads();
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
         if (i4 < 3) load_a(i4 + 1);
@@ -329,25 +331,39 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
       kc[nt] = pt_consts<BITS, SYM, ZF>(sh[nt], zh[nt], g.zoff);
     }
     // A operands two steps ahead of their use (an LDS read takes longer than
-    // a step's four MFMAs); a scheduling barrier a step keeps them there
+    // a step's four MFMAs), B operands one: a step's region holds its MFMAs
+    // and the next step's decode, interleaved, so that a wave alone on its
+    // SIMD keeps the matrix core busy
     f32x16 acc[NM][2];
-    f16x8 av[3][NM];
+    f16x8 av[3][NM], bv[2][2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < NM; ++i) av[t][i] = a_op(i, t);
+    after_reads();
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) bv[0][nt] = pf_decode<BITS, SYM>(w[nt], kc[nt], 0, dk);
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       if (t + 2 < 8) {
 #pragma unroll
         for (int i = 0; i < NM; ++i) av[(t + 2) % 3][i] = a_op(i, t + 2);
       }
-      const f16x8 b0 = pf_decode<BITS, SYM>(w[0], kc[0], t, dk);
-      const f16x8 b1 = pf_decode<BITS, SYM>(w[1], kc[1], t, dk);
+      if (t < 7) {
 #pragma unroll
-      for (int i = 0; i < NM; ++i) {
-        acc[i][0] = mfma_32x32x16(av[t % 3][i], b0, t == 0 ? f32x16{} : acc[i][0]);
-        acc[i][1] = mfma_32x32x16(av[t % 3][i], b1, t == 0 ? f32x16{} : acc[i][1]);
+        for (int nt = 0; nt < 2; ++nt)
+          bv[(t + 1) & 1][nt] = pf_decode<BITS, SYM>(w[nt], kc[nt], t + 1, dk);
+      }
+#pragma unroll
+      for (int i = 0; i < NM; ++i)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+          acc[i][nt] = mfma_32x32x16(av[t % 3][i], bv[t & 1][nt], t == 0 ? f32x16{} : acc[i][nt]);
+#pragma unroll
+      for (int q = 0; q < 2 * NM; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                 // LDS read
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                 // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, NM == 2 ? 5 : 10, 0);  // vector work
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -384,14 +400,14 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
 
   // ---- main loop: U groups an iteration share one load of scales.  One loop
   // per count of token blocks (a branch in the loop costs copies of y) ----
-  constexpr int U = SZQ ? 4 : 1;
-  u32x2 sz[2];
+  constexpr int U = SZQ ? 2 : 1;
+  uint32_t sz[2];
   auto load_sz = [&](int grp) {
     if constexpr (!SCALED) return;
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
-      if constexpr (SZQ) sz[nt] = *(const u32x2*)(szp[nt] + grp);
-      else sz[nt].x = szp[nt][grp];
+      if constexpr (SZQ) sz[nt] = *(const uint32_t*)(szp[nt] + grp);
+      else sz[nt] = szp[nt][grp];
     }
     asm volatile("" ::: "memory");  // before the ring's next loads
   };
@@ -401,20 +417,15 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
   auto loop = [&](auto nm) {
     int in = D - 1, cur = 0;  // ring slots of the next issue and of the group
     for (int c = 0; c < ng; c += U) {
-      uint32_t s2[2][2] = {}, z2[2][2] = {};  // [block][group pair]
+      uint32_t s2[2] = {}, z2[2] = {};  // [block]
       if constexpr (SCALED)
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) {
         // (moved to registers of their own, so that the next load goes to
         // sz's and not through a copy that waits for it at the loop's end)
-        const uint32_t r0 = sz[nt].x, r1 = sz[nt].y;
-        uint32_t v0, v1;
-        asm volatile("v_mov_b32 %0, %1" : "=v"(v0) : "v"(r0));
-        pt_halves(v0, s2[nt][0], z2[nt][0]);
-        if constexpr (SZQ) {
-          asm volatile("v_mov_b32 %0, %1" : "=v"(v1) : "v"(r1));
-          pt_halves(v1, s2[nt][1], z2[nt][1]);
-        }
+        uint32_t v;
+        asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "v"(sz[nt]));
+        pt_halves(v, s2[nt], z2[nt]);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -424,18 +435,20 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
         wait_lgkm0();
         asm volatile("s_barrier" ::: "memory");
         if (u == 0) load_sz(min(c + U, ng - U));
-        issue(min(c + u + D - 1, ng - 1), smem + in * SL::BYTES);
+        unsigned char* const next = smem + in * SL::BYTES;
         const unsigned char* sl = smem + cur * SL::BYTES;
         in = in + 1 == D ? 0 : in + 1;
         cur = cur + 1 == D ? 0 : cur + 1;
-        if constexpr (decltype(nm)::value > 0) {
+        const auto load_next = [&] { issue(min(c + u + D - 1, ng - 1), next); };
+        if constexpr (decltype(nm)::value == 0) load_next();
+        else {
           __half sh[2], zh[2];
 #pragma unroll
           for (int nt = 0; nt < 2; ++nt) {
-            sh[nt] = pt_half(s2[nt][u >> 1], u & 1);
-            zh[nt] = pt_half(z2[nt][u >> 1], u & 1);
+            sh[nt] = pt_half(s2[nt], u);
+            zh[nt] = pt_half(z2[nt], u);
           }
-          group(nm, c + u, sl, sh, zh);
+          group(nm, c + u, sl, sh, zh, load_next);  // (the loads after its first LDS reads)
         }
       }
     }
@@ -539,20 +552,20 @@ static int pt_launch_k(const PfArgs& g, hipStream_t s) {
   return GLQ_OK;
 }
 
-// Scales and zero-points whose rows are whole 8-byte aligned quads.
-static bool pt_quads(const PfArgs& g, bool sym, int nmat) {
+// Scales and zero-points whose rows are whole 4-byte aligned pairs.
+static bool pt_pairs(const PfArgs& g, bool sym, int nmat) {
   uintptr_t m = 0;
   for (int i = 0; i < nmat; ++i)
     m |= (uintptr_t)g.scales[i] | (sym ? 0 : (uintptr_t)g.zeros[i]);
-  return g.G % 4 == 0 && m % 8 == 0;
+  return g.G % 2 == 0 && m % 4 == 0;
 }
 
 template <int WM, int WN, int MT, int MODE, bool SYM, bool ZF>
 static int pt_launch(const PfArgs& g, int bits, hipStream_t s) {
-  // (with the fractional zero-points' branch four groups an iteration would
+  // (with the fractional zero-points' branch two groups an iteration would
   // spill registers)
   if constexpr (!ZF)
-    if (pt_quads(g, SYM, MODE == kPfGateUp ? 2 : 1))
+    if (pt_pairs(g, SYM, MODE == kPfGateUp ? 2 : 1))
       return bits == 2 ? pt_launch_k<2, WM, WN, MT, MODE, SYM, ZF, true>(g, s)
                        : pt_launch_k<4, WM, WN, MT, MODE, SYM, ZF, true>(g, s);
   return bits == 2 ? pt_launch_k<2, WM, WN, MT, MODE, SYM, ZF, false>(g, s)

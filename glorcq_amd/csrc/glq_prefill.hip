@@ -44,8 +44,11 @@
 //
 // pf_lowrank_kernel: a = x U for the low-rank term (fp32 accumulation, one
 // fp16 rounding), 16 rows per workgroup with U staged in LDS.
+#include <unistd.h>
+
 #include <algorithm>
 #include <cstdio>
+#include <cstring>
 
 #include "glq_handoff.h"
 #include "glq_moe_route.h"
@@ -674,6 +677,22 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
 
 namespace glq {
 
+// 16 halves of a code block in the decode order of bits (perm_src): pairs
+// (c, c + 8) at 2 bits, (c, c + 4) of each 8 at 4.
+__device__ __forceinline__ void pf_permute16(int bits, u32x4 lo, u32x4 hi, u32x4& o0, u32x4& o1) {
+  const uint32_t l[4] = {lo.x, lo.y, lo.z, lo.w}, g[4] = {hi.x, hi.y, hi.z, hi.w};
+  uint32_t o[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t sel = i & 1 ? 0x07060302u : 0x05040100u;
+    if (bits == 2) o[i] = __builtin_amdgcn_perm(g[i >> 1], l[i >> 1], sel);
+    else o[i] = i < 4 ? __builtin_amdgcn_perm(l[2 + (i >> 1)], l[i >> 1], sel)
+                      : __builtin_amdgcn_perm(g[2 + ((i - 4) >> 1)], g[(i - 4) >> 1], sel);
+  }
+  o0 = u32x4{o[0], o[1], o[2], o[3]};
+  o1 = u32x4{o[4], o[5], o[6], o[7]};
+}
+
 // ---------------------------------------------------------------------------
 // Low-rank a = x U over a tile list (one expert's rows a tile) or all rows.
 // Workgroup (64-row block, K slice, block of four 32-column tiles of the
@@ -707,6 +726,9 @@ struct PfLowrank {
   __half* a_out;           // (rows_total, nmat * rank) a = fp16(x U) (ks == 1, or finalized)
   unsigned* zero_cnt;      // counters the following GEMM launch expects zero, or null
   int n_cnt;
+  // arrival counters (row block x column block), zero before and after: the
+  // splits' partials are summed by the last to arrive (null: by a launch)
+  unsigned* cnt;
 };
 
 constexpr int kLrRows = 64;  // rows per low-rank workgroup
@@ -714,14 +736,11 @@ constexpr int kLrLds = 128 * 256 + 2 * kLrRows * 256;
 
 __device__ __forceinline__ int pf_ut_sw(int col) { return (col ^ (col >> 3)) & 15; }
 
-__device__ __forceinline__ void pf_lowrank_body(const PfLowrank& L, unsigned char* smem) {
+__device__ __forceinline__ void pf_lowrank_body(const PfLowrank& L, int job, int sp, int cb,
+                                               unsigned char* smem) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, h = lane >> 5;
-  if (L.zero_cnt && blockIdx.x + blockIdx.y + blockIdx.z == 0)
-    for (int i = tid; i < L.n_cnt; i += kPfThreads) L.zero_cnt[i] = 0u;
-  if (L.nmat == 0) return;  // the counters were all there was to do
-  const int job = blockIdx.x, sp = blockIdx.y, cb = blockIdx.z;
   int e = 0, p0, rows;
   if (L.tiles) {
     const int sub = (L.tile_rows + kLrRows - 1) / kLrRows;  // row blocks per tile
@@ -839,25 +858,66 @@ __device__ __forceinline__ void pf_lowrank_body(const PfLowrank& L, unsigned cha
     s ^= 1;
   }
   // acc[i][q]: row 8 (q / 4) + 4 h + q % 4 of 32-row half mg + i mw, column li
-  if (ct >= nct) return;
   const int gt = 4 * cb + ct, m = gt >= ctm ? 1 : 0, j = (gt - m * ctm) * 32 + li;
-  if (j >= r) return;
   const int ld = L.nmat * r;
   float* out = L.part + (int64_t)sp * L.rows_total * ld;
+  if (ct < nct && j < r) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int mb = mg + i * mw;
-    if (mb >= 2) continue;
+    for (int i = 0; i < 2; ++i) {
+      const int mb = mg + i * mw;
+      if (mb >= 2) continue;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int rr = 32 * mb + 8 * (q >> 2) + 4 * h + (q & 3);
-      if (rr < rows) {
-        const int64_t o = (int64_t)(p0 + rr) * ld + m * r + j;
-        if (L.ks == 1) L.a_out[o] = __float2half(acc[i][q]);
-        else out[o] = acc[i][q];
+      for (int q = 0; q < 16; ++q) {
+        const int rr = 32 * mb + 8 * (q >> 2) + 4 * h + (q & 3);
+        if (rr < rows) {
+          const int64_t o = (int64_t)(p0 + rr) * ld + m * r + j;
+          if (L.ks == 1) L.a_out[o] = __float2half(acc[i][q]);
+          else if (L.cnt) handoff_put(out + o, acc[i][q]);
+          else out[o] = acc[i][q];
+        }
       }
     }
   }
+  if (L.cnt == nullptr || L.ks == 1) return;
+  // the block's last split sums them in split order (one matrix: columns
+  // [128 cb, 128 cb + nc) of its rows), pairs of columns a load
+  int* flag = (int*)smem;
+  __syncthreads();  // every wave is done with smem
+  if (!handoff_arrive(L.cnt + job * (int)((ctm + 3) / 4) + cb, (unsigned)L.ks, flag)) return;
+  const int nc2 = min(128, r - 128 * cb) / 2, n2 = rows * nc2;
+  for (int i0 = tid; i0 < n2; i0 += 4 * kPfThreads) {
+    float s0[4] = {0.f, 0.f, 0.f, 0.f}, s1[4] = {0.f, 0.f, 0.f, 0.f};
+    int64_t o[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = min(i0 + kPfThreads * u, n2 - 1);
+      o[u] = (int64_t)(p0 + i / nc2) * ld + 128 * cb + 2 * (i % nc2);
+    }
+    for (int q0 = 0; q0 < L.ks; q0 += 4) {
+      unsigned long long v[4][4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          v[q][u] = handoff_get((const unsigned long long*)(L.part + o[u] +
+                                (int64_t)min(q0 + q, L.ks - 1) * L.rows_total * ld));
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q0 + q < L.ks) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            s0[u] += __uint_as_float((uint32_t)v[q][u]);
+            s1[u] += __uint_as_float((uint32_t)(v[q][u] >> 32));
+          }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i0 + kPfThreads * u < n2)
+        *(uint32_t*)(L.a_out + o[u]) = __half_as_ushort(__float2half(s0[u])) |
+                                       (uint32_t)__half_as_ushort(__float2half(s1[u])) << 16;
+  }
+  if (tid == 0) handoff_reset(L.cnt + job * (int)((ctm + 3) / 4) + cb);
 }
 
 // a = fp16(x U) of the dense prefill in one launch: workgroup (row block
@@ -893,7 +953,74 @@ __global__ __launch_bounds__(256) void pf_xu_kernel(const __half* __restrict__ x
 // Grid: (row blocks, K splits, column blocks).
 __global__ __launch_bounds__(kPfThreads) void pf_lowrank_kernel(PfLowrank L) {
   extern __shared__ __align__(16) unsigned char smem[];
-  pf_lowrank_body(L, smem);
+  if (L.zero_cnt && blockIdx.x + blockIdx.y + blockIdx.z == 0)
+    for (int i = threadIdx.x; i < L.n_cnt; i += kPfThreads) L.zero_cnt[i] = 0u;
+  if (L.nmat == 0) return;  // the counters were all there was to do
+  pf_lowrank_body(L, blockIdx.x, blockIdx.y, blockIdx.z, smem);
+}
+
+// The launch before a dense GEMM in tile form: its first n_lr workgroups are
+// the jobs of a = x U (row blocks x K splits x column blocks); each of the
+// others puts kPrepGroups (row, 128-code group) units of x in decode order and
+// forms their sums c2 (group, row) for fractional zero-points (c2 may be
+// null), 8 threads a unit.
+struct PfPrep {
+  PfLowrank L;
+  int n_lr, ncb;
+  const __half* x;
+  __half* xp;
+  float* c2;
+  int64_t c2_ld;
+  int bits, G;
+  int64_t units;  // rows x groups
+};
+constexpr int kPrepGroups = 128;
+
+__global__ __launch_bounds__(kPfThreads) void pf_prep_kernel(PfPrep p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if ((int)blockIdx.x < p.n_lr) {
+    const int cb = blockIdx.x % p.ncb, rest = blockIdx.x / p.ncb;
+    pf_lowrank_body(p.L, rest / p.L.ks, rest % p.L.ks, cb, smem);
+    return;
+  }
+  const int64_t u0 = (int64_t)(blockIdx.x - p.n_lr) * kPrepGroups;
+  const int l8 = threadIdx.x & 7;
+  u32x4 v[4][2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int64_t u = min(u0 + 32 * q + (threadIdx.x >> 3), p.units - 1);
+    const u32x4* s = (const u32x4*)(p.x + u * 128 + 16 * l8);
+    v[q][0] = s[0];
+    v[q][1] = s[1];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int64_t u = u0 + 32 * q + (threadIdx.x >> 3);
+    const bool in = u < p.units;
+    if (in) {
+      u32x4 o0, o1;
+      pf_permute16(p.bits, v[q][0], v[q][1], o0, o1);
+      u32x4* d = (u32x4*)(p.xp + u * 128 + 16 * l8);
+      d[0] = o0;
+      d[1] = o1;
+    }
+    if (p.c2) {  // uniform
+      float c = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const f16x8 hv = __builtin_bit_cast(f16x8, v[q][i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c += (float)hv[e];
+      }
+      c += __shfl_xor(c, 1);
+      c += __shfl_xor(c, 2);
+      c += __shfl_xor(c, 4);
+      if (in && l8 == 0) {
+        const int64_t row = u / p.G;
+        p.c2[(u - row * p.G) * p.c2_ld + row] = c;
+      }
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -960,7 +1087,7 @@ static int pt_tiles_n(int64_t N, int mode, int tm) {
 }
 
 // K splits of a DOWN launch of `wgs` workgroups over G groups: towards two
-// workgroups a CU, at least four groups each, at most 8 (whole quads of groups
+// workgroups a CU, at least four groups each, at most 8 (whole pairs of groups
 // where the rows' scales are).  Splits cost a fp32 pass over the results, so a
 // launch of 256 workgroups or more has none.  (256 tokens x 5632 -> 2048: 32
 // workgroups of 44 groups, 56 us unsplit.)
@@ -968,7 +1095,7 @@ static int pt_down_split(int64_t wgs, int G, int& gps) {
   int ks = wgs >= 256 ? 1 : (int)std::min<int64_t>({8, 512 / wgs, std::max(1, G / 4)});
   ks = std::max(ks, 1);
   gps = (G + ks - 1) / ks;
-  if (G % 4 == 0) gps = (gps + 3) / 4 * 4;
+  if (G % 2 == 0) gps = (gps + 1) / 2 * 2;
   return (G + gps - 1) / gps;
 }
 
@@ -981,7 +1108,8 @@ static int64_t pf_shared_sy_elems(int64_t T, int64_t H, int64_t SI, int tm) {
 
 template <int MODE, bool SYM, bool ZF>
 static int pt_launch_tm(const PfArgs& g, int bits, int tm, hipStream_t s) {
-  if (tm == 128) return pt_launch<2, 2, 2, MODE, SYM, ZF>(g, bits, s);
+  if constexpr (MODE != kPfDense)
+    if (tm == 128) return pt_launch<2, 2, 2, MODE, SYM, ZF>(g, bits, s);
   if (tm == 64) return pt_launch<1, 4, 2, MODE, SYM, ZF>(g, bits, s);
   return pt_launch<1, 4, 1, MODE, SYM, ZF>(g, bits, s);
 }
@@ -1047,6 +1175,8 @@ static void pf_lowrank_split(int64_t K, int64_t blocks, int& ks, int& kps) {
 // Dense plan: token tile, K splits and workspace of one projection.
 // ---------------------------------------------------------------------------
 struct PfDensePlan {
+  int pt;            // token tile of the tile form (glq_pf_tile.h), or 0
+  int64_t xp_bytes, c2_bytes, c2_ld;
   int tm, rt, ntn, ntm, ks, gps, lr_ks, lr_kps;
   bool deep;
   bool xu1;          // a = x U by pf_xu_kernel (one launch)
@@ -1059,8 +1189,43 @@ struct PfDensePlan {
 // call, so the one-launch x U takes at most kPfSyncBytes / 4 row blocks.
 constexpr int64_t kPfSyncBytes = 4096;
 
+// Token tile of the tile form (64 or 32, x 256 rows) for a dense launch, or 0
+// where pf_gemm_kernel's smaller tiles are the better form: estimates of the
+// three in us, from measured calls with x U (rank 64).  A workgroup of the
+// tile form takes 1.42 us a group at 64 tokens, 1 us at 32 (a CU's workgroups
+// share its rate, so from 256 tiles on time grows with the tiles) after
+// 18-20 us of the x launch, first loads and stores; pf_gemm_kernel about 470
+// TF/s after 12 us and 0.85 (2-bit) or 0.55 (4-bit) us a group of its chain.
+//   (K, N, bits, M): tile form 32 / 64, pf_gemm_kernel (us)
+//   2048, 1408, 2,  512: 34.8 / 43.5, 25.1    2048:  47.7 / 46.7, 57.5
+//   2048, 4096, 4,  512: 37.6 / 44.7, 36.6    1024:  53.0 / 47.5, 66.6
+//   4096, 14336, 2, 256: 71.8 / 65.4, 76.9    2048: 380.6 / 287.8, 426.8
+//   5632, 2048, 4,  256: 62.5 / 81.1, 43.5    1024:  69.8 / 83.8, 103.5
+//   14336, 4096, 2, 150: 118.9 / 166.7, 157.7 2048: 449.5 / 324.7, 536.7
+//   768, 2048, 2,  1024: 26.6 / 31.3, 25.3    2048:  33.2 / 34.3, 38.9
+static int pt_dense_tile(int64_t M, int64_t K, int64_t N, int bits) {
+  const double G = (double)(K / 128), nt = (double)((N + 255) / 256);
+  const double t64 = 18 + 1.42 * G * std::max(1.0, (double)((M + 63) / 64) * nt / 256);
+  const double t32 = 20 + 1.0 * G * std::max(1.0, (double)((M + 31) / 32) * nt / 256);
+  const double old = 12 + (bits == 2 ? 0.85 : 0.55) * G + 2e-6 * (double)M * N * K / 470;
+  if (std::min(t32, t64) >= 0.95 * old) return 0;
+  return t64 <= t32 ? 64 : 32;
+}
+
+// The tests' GLQ_PF_* settings.  One pass over the environment a plan finds
+// that there is none (a call makes five plans).
+struct PfEnv {
+  bool any = false;
+  PfEnv() {
+    for (char** e = environ; e && *e; ++e)
+      if ((*e)[0] == 'G' && strncmp(*e, "GLQ_PF_", 7) == 0) any = true;
+  }
+  const char* get(const char* name) const { return any ? getenv(name) : nullptr; }
+};
+
 static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, int bits) {
   PfDensePlan P;
+  const PfEnv env;
   // Big launches (a 64 x 128 tile per CU or more): 64-token tiles, shallow
   // rings, two workgroups per CU.  Smaller ones: 32-token tiles of
   // 128 rows from 256 tokens, else 16-token tiles of 64 rows, with deep rings
@@ -1082,7 +1247,7 @@ static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, 
     P.rt = 1;
     P.deep = true;
   }
-  if (const char* e = getenv("GLQ_PF_CFG")) {  // "tm,rt,deep": a supported tile
+  if (const char* e = env.get("GLQ_PF_CFG")) {  // "tm,rt,deep": a supported tile
     int tm = 0, rt = 0, deep = 0;
     if (sscanf(e, "%d,%d,%d", &tm, &rt, &deep) == 3) {
       const bool ok = deep ? ((tm == 16 || tm == 32) && (rt == 1 || rt == 2)) || (tm == 64 && rt == 2)
@@ -1099,10 +1264,34 @@ static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, 
   P.ntm = (int)((M + P.tm - 1) / P.tm);
   const int G = (int)(K / 128);
   int ks = 1;
-  if (const char* e = getenv("GLQ_PF_KS")) ks = std::max(1, std::min(G, atoi(e)));
+  if (const char* e = env.get("GLQ_PF_KS")) ks = std::max(1, std::min(G, atoi(e)));
   P.gps = (G + ks - 1) / ks;
   P.ks = (G + P.gps - 1) / P.gps;
+  P.pt = 0;
+  P.xp_bytes = P.c2_bytes = P.c2_ld = 0;
+  if (ks == 1 && !env.get("GLQ_PF_CFG")) P.pt = pt_dense_tile(M, K, N, bits);
   pf_lowrank_split(K, (M + kLrRows - 1) / kLrRows, P.lr_ks, P.lr_kps);
+  if (P.pt) {
+    // x in decode order, its group sums (whole tiles of rows), a and its
+    // partials, summed in their launch (a counter word per 64-row block)
+    P.ntn = pt_tiles_n(N, kPfDense, P.pt);
+    P.ntm = (int)((M + P.pt - 1) / P.pt);
+    P.ks = 1;
+    P.gps = G;
+    if ((M + kLrRows - 1) / kLrRows > kPfSyncBytes / 4) {
+      P.lr_ks = 1;
+      P.lr_kps = (int)K;
+    }
+    P.xu1 = false;
+    P.xp_bytes = align_up(M * K * 2, 256);
+    P.c2_ld = align_up(M, 128);
+    P.c2_bytes = align_up((int64_t)G * P.c2_ld * 4, 256);
+    P.a_bytes = rank > 0 ? align_up(M * rank * 2, 256) : 0;
+    P.lp_bytes = rank > 0 && P.lr_ks > 1 ? align_up((int64_t)P.lr_ks * M * rank * 4, 256) : 0;
+    P.part_bytes = P.cnt_bytes = 0;
+    P.total = kPfSyncBytes + P.xp_bytes + P.c2_bytes + P.a_bytes + P.lp_bytes;
+    return P;
+  }
   P.a_bytes = rank > 0 ? align_up(M * rank * 2, 256) : 0;
   // a = x U in one launch (16-row blocks x K slices, last arrivers sum) when
   // the GEMM needs no split-K counters (those are cleared by the two-launch
@@ -1110,7 +1299,7 @@ static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, 
   const int64_t nrb = (M + 15) / 16;
   P.xu_ns = (int)((K + kLowrankRows - 1) / kLowrankRows);
   P.xu1 = rank > 0 && rank <= 128 && P.ks == 1 && nrb <= kPfSyncBytes / 4 &&
-          !getenv("GLQ_PF_XU2");
+          !env.get("GLQ_PF_XU2");
   if (P.xu1) {
     const int64_t rpad = align_up(rank, 32);
     P.lp_bytes = align_up(nrb * P.xu_ns * 16 * rpad * 4, 256);
@@ -1138,6 +1327,72 @@ int64_t pf_gemm_prefill_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t
   return pf_dense_plan(M, K, N, rank, bits).total;
 }
 
+// The dense GEMM in tile form: x in decode order, a = x U, then the tiles.
+static int pt_dense_gemm(const PfDensePlan& P, const void* x, int64_t M, int64_t K, int64_t N,
+                         const int32_t* codes, int bits, const void* scales, const void* zeros,
+                         int sym, const void* U, const void* SV, int64_t rank, const void* xU,
+                         const void* bias, void* y, void* workspace, hipStream_t s) {
+  char* w = (char*)workspace + kPfSyncBytes;
+  PfPrep q = {};
+  q.x = (const __half*)x;
+  q.xp = (__half*)w;
+  q.c2 = sym == 1 ? nullptr : (float*)(w + P.xp_bytes);
+  q.c2_ld = P.c2_ld;
+  q.bits = bits;
+  q.G = (int)(K / 128);
+  q.units = M * q.G;
+  const bool lora = SV != nullptr && rank > 0;
+  __half* abuf = (__half*)(w + P.xp_bytes + P.c2_bytes);
+  q.ncb = 1;
+  if (lora && xU == nullptr) {
+    PfLowrank& L = q.L;
+    L.x = q.x;
+    L.nmat = 1;
+    L.U[0] = (const __half*)U;
+    L.rows_total = (int)M;
+    L.K = (int)K;
+    L.rank = (int)rank;
+    L.ks = P.lr_ks;
+    L.kps = P.lr_kps;
+    L.part = (float*)((char*)abuf + P.a_bytes);
+    L.a_out = abuf;
+    L.cnt = P.lr_ks > 1 ? (unsigned*)workspace : nullptr;
+    q.n_lr = (int)((M + kLrRows - 1) / kLrRows) * P.lr_ks;
+  }
+  const int64_t grid = q.n_lr + (q.units + kPrepGroups - 1) / kPrepGroups;
+  GLQ_CHECK(grid < (1ll << 31), "too many workgroups");
+  static size_t attr = 64 * 1024;
+  const size_t lds = q.n_lr ? (size_t)kLrLds : 0;
+  int rc = set_lds_limit(pf_prep_kernel, lds, attr);
+  if (rc) return rc;
+  pf_prep_kernel<<<dim3((unsigned)grid), dim3(kPfThreads), lds, s>>>(q);
+  GLQ_LAUNCH_CHECK("pf_prep_kernel");
+  PfArgs g = {};
+  g.xp = q.xp;
+  g.c2 = q.c2;
+  g.c2_ld = q.c2_ld;
+  g.codes[0] = (const uint32_t*)codes;
+  g.scales[0] = (const __half*)scales;
+  g.zeros[0] = (const __half*)zeros;
+  g.a = lora ? (xU ? (const __half*)xU : abuf) : nullptr;
+  g.a_ld = (int)rank;
+  g.sv[0] = lora ? (const __half*)SV : nullptr;
+  g.bias = (const __half*)bias;
+  g.y = (__half*)y;
+  g.y_ld = N;
+  g.M = (int)M;
+  g.K = (int)K;
+  g.N = (int)N;
+  g.G = q.G;
+  g.kw = (int)(K * bits / 32);
+  g.rank = lora ? (int)rank : 0;
+  g.ntn = P.ntn;
+  g.max_tiles = P.ntm;
+  g.zoff = sym == 2 ? (float)(1 << (bits - 1)) : 0.f;
+  return sym == 1 ? pt_launch_tm<kPfDense, true, false>(g, bits, P.pt, s)
+                  : pt_launch_tm<kPfDense, false, true>(g, bits, P.pt, s);
+}
+
 // The prefill GEMM of glq_gemm_lora (called after its argument checks).
 int pf_dense_gemm(const void* x, int64_t M, int64_t K, int64_t N, const int32_t* codes,
                   int bits, const void* scales, const void* zeros, int sym, const void* U,
@@ -1150,6 +1405,9 @@ int pf_dense_gemm(const void* x, int64_t M, int64_t K, int64_t N, const int32_t*
             "workspace of %lld bytes needed (got %lld)", (long long)P.total,
             (long long)workspace_bytes);
   GLQ_CHECK(M * K < (1ll << 31), "M*K too large for the prefill path");
+  if (P.pt)
+    return pt_dense_gemm(P, x, M, K, N, codes, bits, scales, zeros, sym, U, SV, rank, xU, bias, y,
+                         workspace, s);
   unsigned* xcnt = (unsigned*)workspace;  // zero between calls
   char* w = (char*)workspace + (P.total ? kPfSyncBytes : 0);
   __half* abuf = P.a_bytes ? (__half*)w : nullptr;
@@ -1157,7 +1415,8 @@ int pf_dense_gemm(const void* x, int64_t M, int64_t K, int64_t N, const int32_t*
   char* w3 = w + P.a_bytes + P.lp_bytes;
   float* part = P.ks > 1 ? (float*)w3 : nullptr;
   unsigned* cnt = P.ks > 1 ? (unsigned*)(w3 + P.part_bytes) : nullptr;
-  const bool fused = P.xu1 && xU == nullptr && !getenv("GLQ_PF_XU1");
+  const PfEnv env;
+  const bool fused = P.xu1 && xU == nullptr && !env.get("GLQ_PF_XU1");
   if (fused) {
     // a = x U in the GEMM's launch (its first grid rows)
   } else if (P.xu1 && xU == nullptr) {
@@ -1225,7 +1484,7 @@ int pf_dense_gemm(const void* x, int64_t M, int64_t K, int64_t N, const int32_t*
     g.xu_cnt = xcnt;
     // GLQ_PF_SPIN_TICKS: the epilogue's wait bound (tests set 0 to take the
     // local form)
-    const char* e = getenv("GLQ_PF_SPIN_TICKS");
+    const char* e = env.get("GLQ_PF_SPIN_TICKS");
     g.xu_spin = e ? (uint64_t)strtoull(e, nullptr, 10) : 100000;  // 1 ms
   }
   return pf_launch_dense(g, bits, PfTile{P.tm, P.rt, P.deep}, sym == 1, s);
@@ -1292,22 +1551,6 @@ __device__ __forceinline__ uint32_t pf_wave_max(uint32_t v) {
   v = max(r[0], r[1]);
   const auto q = __builtin_amdgcn_permlane32_swap(v, v, false, false);
   return max(q[0], q[1]);
-}
-
-// 16 halves of a code block in the decode order of bits (perm_src): pairs
-// (c, c + 8) at 2 bits, (c, c + 4) of each 8 at 4.
-__device__ __forceinline__ void pf_permute16(int bits, u32x4 lo, u32x4 hi, u32x4& o0, u32x4& o1) {
-  const uint32_t l[4] = {lo.x, lo.y, lo.z, lo.w}, g[4] = {hi.x, hi.y, hi.z, hi.w};
-  uint32_t o[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t sel = i & 1 ? 0x07060302u : 0x05040100u;
-    if (bits == 2) o[i] = __builtin_amdgcn_perm(g[i >> 1], l[i >> 1], sel);
-    else o[i] = i < 4 ? __builtin_amdgcn_perm(l[2 + (i >> 1)], l[i >> 1], sel)
-                      : __builtin_amdgcn_perm(g[2 + ((i - 4) >> 1)], g[(i - 4) >> 1], sel);
-  }
-  o0 = u32x4{o[0], o[1], o[2], o[3]};
-  o1 = u32x4{o[4], o[5], o[6], o[7]};
 }
 
 // Rows t0 .. t0 + 15 of x in the routed experts' decode order (and in the

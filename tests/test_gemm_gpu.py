@@ -263,3 +263,49 @@ def test_one_launch_xu(gpu, monkeypatch, M, K, N, bits):
     y2 = call()
     torch.cuda.synchronize()
     assert_parity(y2, oracle_y(p), f"two-launch x U M={M}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,bits,rank,sym", [
+    (150, 14336, 520, 2, 64, False),    # 32-token tiles, a 22-row last tile, 8 rows past 2 blocks
+    (1025, 1408, 2048, 2, 40, False),   # one row over 32-token tiles, 11 groups (one a load)
+    (777, 2048, 4096, 4, 128, False),   # 64-token tiles, x U over 13 row blocks
+    (2049, 768, 2100, 4, 0, True),      # no low-rank term, symmetric, one row over
+    (400, 4096, 14336, 2, 8, True),     # symmetric 2-bit, rank 8
+], ids=str)
+def test_dense_tile_form(gpu, M, K, N, bits, rank, sym):
+    """The dense launch in tile form (chosen by size): ragged token tiles and
+    row blocks, rows whose zero-points are fractions (their sums of x come from
+    the launch before), a bias, a = x U formed there or given; the same bits
+    on repeated calls (its arrival counters are left at zero)."""
+    p = fmt.make_linear(K, N, bits=bits, group=128, rank=max(rank, 8), M=M, seed=M + N, sym=sym)
+    if not sym:
+        z = p.zeros.float()
+        frac = torch.rand(z.shape, generator=torch.Generator().manual_seed(bits)) * 0.5
+        rows = torch.arange(z.shape[0]).unsqueeze(1) % 3 == 1
+        p.zeros = torch.where(rows, z + frac, z).half()
+    d = to(p, gpu)
+    bias = (torch.randn(N, generator=torch.Generator().manual_seed(5)) * 0.1).half().to(gpu)
+    x, W = d["x"].double(), p.q.to(gpu).double()
+    s = d["scales"].double().repeat_interleave(128, dim=1)
+    W = W * s if sym else (W - d["zeros"].double().repeat_interleave(128, dim=1)) * s
+    ref = x @ W.T + bias.double()
+    kw = dict(U=d["U"], SV=d["SV"]) if rank else {}
+    if rank:
+        a = (x @ d["U"].double()).half()
+        ref = ref + a.double() @ d["SV"].double().T
+
+    def call(**k):
+        return K_.packed_dequant_matmul_fused(d["x"], d["codes"], d["scales"],
+                                              None if sym else d["zeros"], bits, 128, sym=sym,
+                                              bias=bias, **k)
+
+    y = call(**kw)
+    # fp16 rounding of y, a rounded the other way, fp32 sums of K products
+    tol = 2e-3 + 1.5e-3 * ref.abs()
+    assert bool(((y.double() - ref).abs() <= tol).all()), float((y.double() - ref).abs().max())
+    for _ in range(2):
+        assert torch.equal(call(**kw), y)
+    if rank:
+        y2 = call(SV=d["SV"], precomputed_xU=a)
+        assert bool(((y2.double() - ref).abs() <= tol).all())
