@@ -164,6 +164,29 @@ def _gemv_workspace_bytes(lib, items: int, M: int, K: int, N: int, rank: int) ->
     return n
 
 
+def _plain(*tensors) -> bool:
+    """The operator dispatch would only call the eager function: plain GPU
+    tensors and nothing that watches, transforms or differentiates the call
+    (compile and trace, dispatch and function modes, functorch, forward-mode
+    levels, a gradient to record).  The dispatch of a Python custom operator
+    costs about 7 us of host time, this check 0.5."""
+    C = torch._C
+    if (torch.compiler.is_compiling() or C._len_torch_dispatch_stack()
+            or C._len_torch_function_stack() or C._get_tracing_state() is not None
+            or C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in _PLAIN_TYPES or not t.is_cuda
+                              or (grad and t.requires_grad)):
+            return False
+    return True
+
+
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
 def packed_dequant_matmul_fused(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor,
                                 zeros: torch.Tensor | None, bits: int, groupsize: int,
                                 sym: bool = False, U: torch.Tensor | None = None,
@@ -175,9 +198,10 @@ def packed_dequant_matmul_fused(x: torch.Tensor, codes: torch.Tensor, scales: to
 
     Without `out` this is the operator glorcq_hip::packed_dequant_matmul
     (torch.library, with a fake kernel, so torch.compile traces it without a
-    graph break); with `out` (a caller's buffer, e.g. under graph capture) the
+    graph break), called directly where the dispatch would add nothing
+    (_plain); with `out` (a caller's buffer, e.g. under graph capture) the
     library is called directly.  Arguments as _packed_dequant_matmul_eager."""
-    if out is None:
+    if out is None and not _plain(x, codes, scales, zeros, U, SV, precomputed_xU, bias):
         return torch.ops.glorcq_hip.packed_dequant_matmul(
             x, codes, scales, zeros, bits, groupsize, _sym_mode(sym), U, SV, precomputed_xU, bias)
     return _packed_dequant_matmul_eager(x, codes, scales, zeros, bits, groupsize, sym, U, SV,

@@ -120,3 +120,46 @@ def test_compile_moe_block_fullgraph_equals_eager(gpu):
     got, gl = compiled(h)
     torch.cuda.synchronize()
     assert torch.equal(got, eager) and torch.equal(gl, el)
+
+
+@pytest.mark.gpu
+def test_direct_call_where_the_dispatch_adds_nothing(gpu):
+    """packed_dequant_matmul_fused calls the library directly for plain tensors
+    and goes through the operator wherever something watches or transforms the
+    call: a dispatch mode sees it, vmap and forward-mode levels and recorded
+    gradients get the operator's own answer."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from glorcq_amd import kernels as K_
+
+    p = fmt.make_linear(2048, 256, bits=2, rank=16, M=3, seed=8)
+    t = {k: getattr(p, k).to(gpu) for k in ("x", "codes", "scales", "zeros", "U", "SV")}
+
+    def call(x):
+        return K_.packed_dequant_matmul_fused(x, t["codes"], t["scales"], t["zeros"], 2, 128,
+                                              U=t["U"], SV=t["SV"])
+
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    y = call(t["x"])
+    assert K_._plain(*t.values())
+    with Watch():
+        assert torch.equal(call(t["x"]), y)
+    assert any("packed_dequant_matmul" in s for s in seen)
+    xg = t["x"].clone().requires_grad_()
+    assert not K_._plain(xg)
+    yg = call(xg)
+    assert yg.requires_grad and torch.equal(yg.detach(), y)
+    with pytest.raises(Exception):
+        yg.sum().backward()  # no gradient formula, as through the operator
+    with torch.no_grad():
+        assert K_._plain(xg) and torch.equal(call(xg), y)
+    assert torch.equal(torch.vmap(call)(torch.stack([t["x"], t["x"]])), torch.stack([y, y]))
+    with torch.autograd.forward_ad.dual_level():
+        assert not K_._plain(t["x"])
+    assert not K_._plain(p.x)  # a CPU tensor
