@@ -138,7 +138,8 @@ __device__ __forceinline__ PfK<BITS> pt_consts(__half sh, __half zh, float zoff)
 }
 
 template <int BITS, int WM, int WN, int MT, int MODE, bool SYM, bool ZF, bool SZQ>
-__device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
+__device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem, int bx, int by,
+                                        int bz) {
   constexpr bool SCALED = BITS == 2 || BITS == 4;
   static_assert(WM * WN == 4 && (SCALED || BITS == kPtTurbo || BITS == kPtHalf), "4 waves");
   static_assert(BITS != kPtHalf || MODE == kPfDense, "one matrix");
@@ -149,7 +150,7 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, h = lane >> 5;
   const int wm = wave % WM, wn = wave / WM;
-  const int ty = blockIdx.y;
+  const int ty = by;
   int e = 0, p0, rows;
   if (g.tiles) {
     if (ty >= *g.ntiles) return;  // uniform over the workgroup
@@ -160,10 +161,10 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
     p0 = ty * SL::TM;
     rows = min(SL::TM, g.M - p0);
   }
-  const int n0 = blockIdx.x * (TWO ? 32 : 64) * WN;
+  const int n0 = bx * (TWO ? 32 : 64) * WN;
   // K split z (DOWN: fp32 results of their own, summed by the combine; split 0
   // has the low-rank term)
-  const int g0 = MODE == kPfDown ? (int)blockIdx.z * g.gps : 0;
+  const int g0 = MODE == kPfDown ? bz * g.gps : 0;
 
   // ---- load addresses: element offsets from uniform bases ----
   // (buffer loads: one constant offset a lane, the group's in a scalar; they
@@ -526,7 +527,7 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
             g.y[(int64_t)(p0 + r) * g.y_ld + pt_col(g.out_bits, n)] =
                 __float2half(y[i][nt][j] + bn);
           else
-            g.yf[blockIdx.z * g.yf_ss + (int64_t)(p0 + r) * g.yf_ld + n] = y[i][nt][j];
+            g.yf[bz * g.yf_ss + (int64_t)(p0 + r) * g.yf_ld + n] = y[i][nt][j];
         }
       }
     }
@@ -535,8 +536,10 @@ __device__ __forceinline__ void pt_body(const PfArgs& g, unsigned char* smem) {
 
 template <int BITS, int WM, int WN, int MT, int MODE, bool SYM, bool ZF, bool SZQ>
 __global__ __launch_bounds__(kPfThreads, 2) void pf_tile_kernel(PfArgs g) {
+#ifdef __HIP_DEVICE_COMPILE__  // (the host pass refuses pt_body's device types)
   extern __shared__ __align__(16) unsigned char smem[];
-  pt_body<BITS, WM, WN, MT, MODE, SYM, ZF, SZQ>(g, smem);
+  pt_body<BITS, WM, WN, MT, MODE, SYM, ZF, SZQ>(g, smem, blockIdx.x, blockIdx.y, blockIdx.z);
+#endif
 }
 
 template <int BITS, int WM, int WN, int MT, int MODE, bool SYM, bool ZF, bool SZQ>
@@ -549,6 +552,44 @@ static int pt_launch_k(const PfArgs& g, hipStream_t s) {
   const dim3 grid((unsigned)g.ntn, (unsigned)g.max_tiles, (unsigned)(MODE == kPfDown ? g.ks : 1));
   pf_tile_kernel<BITS, WM, WN, MT, MODE, SYM, ZF, SZQ><<<grid, dim3(kPfThreads), lds, s>>>(g);
   GLQ_LAUNCH_CHECK("pf_tile_kernel");
+  return GLQ_OK;
+}
+
+// Two launches of 32-token tiles as one: b's nb workgroups (4-bit, the shared
+// expert), then a's (2-bit or TurboQuant, the routed experts).  Their tiles do
+// not fill the chip in whole rounds, so b's cost little beside a's: 19.5 + 11.3
+// us of the block's 155 at 32 tokens as launches of their own.
+template <int BA, int MODE, bool SZQ>
+__global__ __launch_bounds__(kPfThreads, 2) void pf_tile_pair_kernel(PfArgs a, PfArgs b, int nb) {
+#ifdef __HIP_DEVICE_COMPILE__
+  extern __shared__ __align__(16) unsigned char smem[];
+  int i = blockIdx.x;
+  if (i < nb) {
+    const int x = i % b.ntn, r = i / b.ntn;
+    pt_body<4, 1, 4, 1, MODE, false, false, SZQ>(b, smem, x, r % b.max_tiles, r / b.max_tiles);
+  } else {
+    i -= nb;
+    const int x = i % a.ntn, r = i / a.ntn;
+    pt_body<BA, 1, 4, 1, MODE, false, false, BA == kPtTurbo ? false : SZQ>(
+        a, smem, x, r % a.max_tiles, r / a.max_tiles);
+  }
+#endif
+}
+
+template <int BA, int MODE, bool SZQ>
+static int pt_launch_pair_k(const PfArgs& a, const PfArgs& b, hipStream_t s) {
+  static size_t attr = 64 * 1024;
+  using SA = PtSlot<BA, 1, 4, 1>;
+  using SB = PtSlot<4, 1, 4, 1>;
+  const size_t lds = std::max((size_t)SA::D * SA::BYTES, (size_t)SB::D * SB::BYTES);
+  int rc = set_lds_limit(pf_tile_pair_kernel<BA, MODE, SZQ>, lds, attr);
+  if (rc) return rc;
+  const int64_t nb = (int64_t)b.ntn * b.max_tiles * (MODE == kPfDown ? b.ks : 1);
+  const int64_t na = (int64_t)a.ntn * a.max_tiles * (MODE == kPfDown ? a.ks : 1);
+  GLQ_CHECK(na + nb < (1ll << 31), "too many workgroups");
+  pf_tile_pair_kernel<BA, MODE, SZQ><<<dim3((unsigned)(na + nb)), dim3(kPfThreads), lds, s>>>(
+      a, b, (int)nb);
+  GLQ_LAUNCH_CHECK("pf_tile_pair_kernel");
   return GLQ_OK;
 }
 
@@ -570,5 +611,13 @@ static int pt_launch(const PfArgs& g, int bits, hipStream_t s) {
                        : pt_launch_k<4, WM, WN, MT, MODE, SYM, ZF, true>(g, s);
   return bits == 2 ? pt_launch_k<2, WM, WN, MT, MODE, SYM, ZF, false>(g, s)
                    : pt_launch_k<4, WM, WN, MT, MODE, SYM, ZF, false>(g, s);
+}
+
+template <int BA, int MODE>
+static int pt_launch_pair(const PfArgs& a, const PfArgs& b, hipStream_t s) {
+  const int nmat = MODE == kPfGateUp ? 2 : 1;
+  if ((BA == kPtTurbo || pt_pairs(a, false, nmat)) && pt_pairs(b, false, nmat))
+    return pt_launch_pair_k<BA, MODE, true>(a, b, s);
+  return pt_launch_pair_k<BA, MODE, false>(a, b, s);
 }
 }  // namespace glq

@@ -879,19 +879,21 @@ __device__ __forceinline__ void pf_lowrank_body(const PfLowrank& L, int job, int
     }
   }
   if (L.cnt == nullptr || L.ks == 1) return;
-  // the block's last split sums them in split order (one matrix: columns
-  // [128 cb, 128 cb + nc) of its rows), pairs of columns a load
+  // the block's last split sums them in split order: its tiles' columns are
+  // [c0, c0 + 2 nc2) of a row (whole pairs), two a load
   int* flag = (int*)smem;
   __syncthreads();  // every wave is done with smem
-  if (!handoff_arrive(L.cnt + job * (int)((ctm + 3) / 4) + cb, (unsigned)L.ks, flag)) return;
-  const int nc2 = min(128, r - 128 * cb) / 2, n2 = rows * nc2;
+  const int nblk = (L.nmat * ctm + 3) / 4;
+  if (!handoff_arrive(L.cnt + job * nblk + cb, (unsigned)L.ks, flag)) return;
+  auto col0 = [&](int g) { return g >= L.nmat * ctm ? L.nmat * r : g / ctm * r + g % ctm * 32; };
+  const int c0 = col0(4 * cb), nc2 = (col0(4 * cb + 4) - c0) / 2, n2 = rows * nc2;
   for (int i0 = tid; i0 < n2; i0 += 4 * kPfThreads) {
     float s0[4] = {0.f, 0.f, 0.f, 0.f}, s1[4] = {0.f, 0.f, 0.f, 0.f};
     int64_t o[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int i = min(i0 + kPfThreads * u, n2 - 1);
-      o[u] = (int64_t)(p0 + i / nc2) * ld + 128 * cb + 2 * (i % nc2);
+      o[u] = (int64_t)(p0 + i / nc2) * ld + c0 + 2 * (i % nc2);
     }
     for (int q0 = 0; q0 < L.ks; q0 += 4) {
       unsigned long long v[4][4];
@@ -917,7 +919,7 @@ __device__ __forceinline__ void pf_lowrank_body(const PfLowrank& L, int job, int
         *(uint32_t*)(L.a_out + o[u]) = __half_as_ushort(__float2half(s0[u])) |
                                        (uint32_t)__half_as_ushort(__float2half(s1[u])) << 16;
   }
-  if (tid == 0) handoff_reset(L.cnt + job * (int)((ctm + 3) / 4) + cb);
+  if (tid == 0) handoff_reset(L.cnt + job * nblk + cb);
 }
 
 // a = fp16(x U) of the dense prefill in one launch: workgroup (row block
@@ -1106,6 +1108,17 @@ static int64_t pf_shared_sy_elems(int64_t T, int64_t H, int64_t SI, int tm) {
   return (int64_t)pt_down_split(wgs, (int)(SI / 128), gps) * T * H;
 }
 
+// K splits of the routed down of Pn pairs: its workgroups estimated from full
+// tiles and one ragged tile an expert.  (Mixtral-shaped layer, 32 tokens: 128
+// workgroups of 112 groups, 98 us unsplit.)
+static int pt_routed_split(int64_t Pn, int64_t E, int64_t H, int tm, int G, int& gps) {
+  return pt_down_split(pt_tiles_n(H, kPfDown, tm) * (Pn / tm + std::min(E, Pn)), G, gps);
+}
+
+// Arrival counters of the low-rank launches over a tile list (at most two
+// column blocks: two matrices of rank 128).
+static int pf_lrcnt(int max_tiles, int tm) { return max_tiles * ((tm + 63) / 64) * 2; }
+
 template <int MODE, bool SYM, bool ZF>
 static int pt_launch_tm(const PfArgs& g, int bits, int tm, hipStream_t s) {
   if constexpr (MODE != kPfDense)
@@ -1152,7 +1165,7 @@ static int pf_lowrank_launch(const PfLowrank& L, int n_jobs, hipStream_t s) {
   if (rc) return rc;
   pf_lowrank_kernel<<<grid, dim3(kPfThreads), kLrLds, s>>>(L);
   GLQ_LAUNCH_CHECK("pf_lowrank_kernel");
-  if (L.nmat > 0 && L.ks > 1) {
+  if (L.nmat > 0 && L.ks > 1 && !L.cnt) {
     const int64_t n = (int64_t)L.rows_total * L.nmat * L.rank;
     pf_lowrank_finalize_kernel<<<dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s>>>(
         L.part, L.ks, n, L.a_out);
@@ -1532,7 +1545,10 @@ struct PfMoe {
   int32_t* stok;           // (T * topk) token of each sorted row
   int32_t* tiles;          // (max_tiles, 3)
   int32_t* ntiles;
-  const float* ybuf;       // (T * topk, H) routed outputs per sorted row
+  unsigned* lrcnt;         // the low-rank launches' arrival counters (zeroed here)
+  int n_lrcnt;
+  const float* ybuf;       // (yks, T * topk, H) routed outputs per sorted row in K splits
+  int yks;
   const float* sy;         // (sks, T, H) shared expert output in K splits, or null
   int sks;
   const __half* syh;       // or it as fp16
@@ -1720,6 +1736,7 @@ __global__ __launch_bounds__(1024) void pf_moe_dispatch_kernel(PfMoe a) {
   __shared__ int cnt[256], off[256], cur[256], tb[256];
   const int tid = threadIdx.x, P = a.T * a.topk;
   if (tid < 256) cnt[tid] = 0;
+  for (int i = tid; i < a.n_lrcnt; i += 1024) a.lrcnt[i] = 0u;
   __syncthreads();
   constexpr int U = 8;
   for (int p0 = 0; p0 < P; p0 += 1024 * U) {
@@ -1798,14 +1815,23 @@ __global__ __launch_bounds__(256) void pf_moe_combine_kernel(PfMoe a) {
   if (i >= (int64_t)a.T * a.H) return;
   const int t = (int)(i / a.H), n = (int)(i - (int64_t)t * a.H);
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  const int64_t ss = (int64_t)a.T * a.topk * a.H;
   for (int k0 = 0; k0 < a.topk; k0 += 4) {
     float4 v[4];
     float w[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int p = t * a.topk + min(k0 + u, a.topk - 1);
-      v[u] = *(const float4*)(a.ybuf + (int64_t)a.pos[p] * a.H + n);
+      const float* yp = a.ybuf + (int64_t)a.pos[p] * a.H + n;
+      v[u] = *(const float4*)yp;
       w[u] = __half2float(a.wts[p]);
+      for (int q = 1; q < a.yks; ++q) {
+        const float4 m = *(const float4*)(yp + q * ss);
+        v[u].x += m.x;
+        v[u].y += m.y;
+        v[u].z += m.z;
+        v[u].w += m.w;
+      }
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
@@ -1847,6 +1873,8 @@ __global__ __launch_bounds__(256) void pf_moe_combine_kernel(PfMoe a) {
 // Host plan of glq_moe_prefill
 // ---------------------------------------------------------------------------
 struct PfMoePlan {
+  int yks, ygps;  // K splits of the routed down
+  int64_t off_lrcnt;
   int tm, max_tiles, ks_gu, kps_gu, ks_d, kps_d, stm;
   int64_t off_xp, off_xps, off_sel, off_wts, off_sg, off_pos, off_stok, off_tiles, off_lp,
       off_agu, off_ad, off_inter, off_y, off_sinter, off_sy, total;
@@ -1872,7 +1900,8 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
   const int64_t lrb = (Pn + kLrRows - 1) / kLrRows + std::min<int64_t>(E, Pn) / 2;
   pf_lowrank_split(H, lrb, P.ks_gu, P.kps_gu);
   pf_lowrank_split(I, lrb, P.ks_d, P.kps_d);
-  P.stm = T > 32 ? 64 : 32;
+  P.stm = T > 32 && P.tm != 32 ? 64 : 32;
+  P.yks = pt_routed_split(Pn, E, H, P.tm, (int)(I / 128), P.ygps);
   int64_t o = 0;
   auto take = [&](int64_t bytes) {
     const int64_t at = o;
@@ -1887,6 +1916,7 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
   P.off_pos = take(Pn * 4);
   P.off_stok = take(Pn * 4);
   P.off_tiles = take((int64_t)P.max_tiles * 12 + 4);
+  P.off_lrcnt = take(4 * (int64_t)pf_lrcnt(P.max_tiles, P.tm));
   const int64_t lp = rank > 0 ? std::max<int64_t>(P.ks_gu > 1 ? P.ks_gu * Pn * 2 * rank * 4 : 0,
                                                   P.ks_d > 1 ? P.ks_d * Pn * rank * 4 : 0)
                               : 0;
@@ -1894,7 +1924,7 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
   P.off_agu = take(rank > 0 ? Pn * 2 * rank * 2 : 0);
   P.off_ad = take(rank > 0 ? Pn * rank * 2 : 0);
   P.off_inter = take(Pn * I * 2);
-  P.off_y = take(Pn * H * 4);
+  P.off_y = take(P.yks * Pn * H * 4);
   P.off_sinter = take(SI > 0 ? T * SI * 2 : 0);
   P.off_sy = take(SI > 0 ? pf_shared_sy_elems(T, H, SI, P.stm) * 4 : 0);
   P.total = o;
@@ -1915,14 +1945,25 @@ static int pf_route_launch(const PfMoe& a, hipStream_t s) {
   return GLQ_OK;
 }
 
-// The shared expert over every token: xps (T, H) in its decode order -> sy
-// (sks, T, H) fp32 in K splits, through sinter (T, SI).
-static int pf_shared_launch(int64_t T, int64_t H, int64_t SI, int bits, int tm, const __half* xps,
-                            const int32_t* const codes[3], const void* const scales[3],
-                            const void* const zeros[3], __half* sinter, float* sy, int& sks,
-                            hipStream_t s) {
+// The shared expert over every token, two GEMMs in the tile form of tm tokens:
+// xps (T, H) in its decode order -> sinter (T, SI) -> sy (sks, T, H) fp32 in K
+// splits.  pair: 32-token tiles of 4-bit codes ride in the routed launches.
+struct PfShared {
+  PfArgs gu, down;
+  int bits, tm;
+  bool pair;
+};
+
+static PfShared pf_shared(int64_t T, int64_t H, int64_t SI, int bits, int tm, bool pair,
+                          const __half* xps, const int32_t* const codes[3],
+                          const void* const scales[3], const void* const zeros[3],
+                          __half* sinter, float* sy) {
+  PfShared S = {};
+  S.bits = bits;
+  S.tm = tm;
+  S.pair = pair && bits == 4 && tm == 32;
   const int ntm = (int)((T + tm - 1) / tm);
-  PfArgs g = {};
+  PfArgs& g = S.gu;
   g.xp = xps;
   for (int m = 0; m < 2; ++m) {
     g.codes[m] = (const uint32_t*)codes[m];
@@ -1936,9 +1977,7 @@ static int pf_shared_launch(int64_t T, int64_t H, int64_t SI, int bits, int tm, 
   g.ntn = pt_tiles_n(SI, kPfGateUp, tm);
   g.out_bits = bits;
   g.max_tiles = ntm;
-  int rc = pt_launch_tm<kPfGateUp, false, false>(g, bits, tm, s);
-  if (rc) return rc;
-  PfArgs d = {};
+  PfArgs& d = S.down;
   d.xp = sinter;
   d.codes[0] = (const uint32_t*)codes[2];
   d.scales[0] = (const __half*)scales[2];
@@ -1949,9 +1988,28 @@ static int pf_shared_launch(int64_t T, int64_t H, int64_t SI, int bits, int tm, 
   d.kw = (int)(SI * bits / 32);
   d.ntn = pt_tiles_n(H, kPfDown, tm);
   d.max_tiles = ntm;
-  d.ks = sks = pt_down_split((int64_t)d.ntn * ntm, d.G, d.gps);
+  d.ks = pt_down_split((int64_t)d.ntn * ntm, d.G, d.gps);
   d.yf_ss = T * H;
-  return pt_launch_tm<kPfDown, false, false>(d, bits, tm, s);
+  return S;
+}
+
+// A routed launch, with the shared expert's of the same step where it rides.
+template <int BA, int MODE>
+static int pf_routed_launch(const PfArgs& g, int tm, const PfShared* S, hipStream_t s) {
+  if (S && S->pair && tm == 32)
+    return pt_launch_pair<BA, MODE>(g, MODE == kPfGateUp ? S->gu : S->down, s);
+  if constexpr (BA == kPtTurbo)
+    return tm == 64 ? pt_launch_k<kPtTurbo, 1, 4, 2, MODE, false, false, false>(g, s)
+                    : pt_launch_k<kPtTurbo, 1, 4, 1, MODE, false, false, false>(g, s);
+  else
+    return pt_launch_tm<MODE, false, false>(g, BA, tm, s);
+}
+
+// The shared expert's launches, where they do not ride in the routed ones.
+static int pf_shared_launch(const PfShared* S, int routed_tm, hipStream_t s) {
+  if (!S || (S->pair && routed_tm == 32)) return GLQ_OK;
+  const int rc = pt_launch_tm<kPfGateUp, false, false>(S->gu, S->bits, S->tm, s);
+  return rc ? rc : pt_launch_tm<kPfDown, false, false>(S->down, S->bits, S->tm, s);
 }
 
 static int pf_moe_check(const glq_moe_params* p) {
@@ -2040,6 +2098,9 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
   a.stok = (int32_t*)(w + P.off_stok);
   a.tiles = (int32_t*)(w + P.off_tiles);
   a.ntiles = a.tiles + 3 * P.max_tiles;
+  a.lrcnt = (unsigned*)(w + P.off_lrcnt);
+  a.n_lrcnt = pf_lrcnt(P.max_tiles, P.tm);
+  a.yks = P.yks;
   a.ybuf = (const float*)(w + P.off_y);
   a.sy = SI > 0 ? (const float*)(w + P.off_sy) : nullptr;
   a.res = (const __half*)p->residual;
@@ -2054,6 +2115,15 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
   rc = pf_route_launch(a, s);
   if (rc) return rc;
 
+  PfShared sh;
+  const PfShared* shared = nullptr;
+  if (SI > 0) {
+    sh = pf_shared(T, H, SI, p->shared_bits, P.stm, p->bits == 2, a.xps, p->shared_codes,
+                   p->shared_scales, p->shared_zeros, (__half*)(w + P.off_sinter),
+                   (float*)(w + P.off_sy));
+    shared = &sh;
+    a.sks = sh.down.ks;
+  }
   // expert strides (elements)
   const int64_t kw_gu = H * p->bits / 32, kw_d = I * p->bits / 32;
   // 3. a = x U for gate and up per pair
@@ -2078,6 +2148,7 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     L.ks = P.ks_gu;
     L.kps = P.kps_gu;
     L.part = lp;
+    L.cnt = a.lrcnt;
     L.a_out = agu;
     rc = pf_lowrank_launch(L, P.max_tiles * ((P.tm + kLrRows - 1) / kLrRows), s);
     if (rc) return rc;
@@ -2108,7 +2179,8 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     g.ks = 1; g.gps = g.G;
     g.out_bits = p->bits;
     g.max_tiles = P.max_tiles;
-    rc = pt_launch_tm<kPfGateUp, false, false>(g, p->bits, P.tm, s);
+    rc = p->bits == 2 ? pf_routed_launch<2, kPfGateUp>(g, P.tm, shared, s)
+                      : pt_launch_tm<kPfGateUp, false, false>(g, 4, P.tm, s);
     if (rc) return rc;
   }
   // 5. a = inter U_down per pair
@@ -2129,6 +2201,7 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     L.ks = P.ks_d;
     L.kps = P.kps_d;
     L.part = lp;
+    L.cnt = a.lrcnt;
     L.a_out = ad;
     rc = pf_lowrank_launch(L, P.max_tiles * ((P.tm + kLrRows - 1) / kLrRows), s);
     if (rc) return rc;
@@ -2153,18 +2226,16 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     g.M = (int)Pn; g.K = (int)I; g.N = (int)H; g.G = (int)(I / 128);
     g.kw = (int)kw_d; g.rank = r;
     g.ntn = pt_tiles_n(H, kPfDown, P.tm);
-    g.ks = 1; g.gps = g.G;
+    g.ks = P.yks; g.gps = P.ygps;
+    g.yf_ss = Pn * H;
     g.max_tiles = P.max_tiles;
-    rc = pt_launch_tm<kPfDown, false, false>(g, p->bits, P.tm, s);
+    rc = p->bits == 2 ? pf_routed_launch<2, kPfDown>(g, P.tm, shared, s)
+                      : pt_launch_tm<kPfDown, false, false>(g, 4, P.tm, s);
     if (rc) return rc;
   }
-  // 7. shared expert over every token
-  if (SI > 0) {
-    rc = pf_shared_launch(T, H, SI, p->shared_bits, P.stm, a.xps, p->shared_codes,
-                          p->shared_scales, p->shared_zeros, (__half*)(w + P.off_sinter),
-                          (float*)(w + P.off_sy), a.sks, s);
-    if (rc) return rc;
-  }
+  // 7. shared expert over every token (2-bit or larger tiles)
+  rc = pf_shared_launch(shared, p->bits == 2 ? P.tm : 0, s);
+  if (rc) return rc;
   // 8. combine
   pf_moe_combine_kernel<<<dim3((unsigned)((T * H / 4 + 255) / 256)), dim3(256), 0, s>>>(a);
   GLQ_LAUNCH_CHECK("pf_moe_combine_kernel");
@@ -2181,6 +2252,8 @@ namespace glq {
 // experts again: 256 tokens through the 60-expert block took 16 steps, 2.2 ms.
 // ===========================================================================
 struct TpPlan {
+  int yks, ygps;  // K splits of the routed down
+  int64_t off_lrcnt;
   int tm, max_tiles, stm, ks_gu, kps_gu, ks_d, kps_d;
   int64_t off_xr, off_xp, off_xps, off_sel, off_wts, off_sg, off_pos, off_stok, off_tiles, off_lp,
       off_agu, off_ad, off_inter, off_tmp, off_xd, off_y, off_sinter, off_sy, total;
@@ -2192,7 +2265,8 @@ static TpPlan tp_plan(const glq_turbo_prefill_params* p) {
   TpPlan P;
   P.tm = Pn / std::max<int64_t>(E, 1) < 46 ? 32 : 64;  // as pf_moe_plan's tiles
   P.max_tiles = (int)((Pn + P.tm - 1) / P.tm + E);
-  P.stm = T > 32 ? 64 : 32;
+  P.stm = T > 32 && P.tm != 32 ? 64 : 32;
+  P.yks = pt_routed_split(Pn, E, H, P.tm, (int)(I / 128), P.ygps);
   const int64_t lrb = (Pn + kLrRows - 1) / kLrRows + std::min<int64_t>(E, Pn) / 2;
   pf_lowrank_split(H, lrb, P.ks_gu, P.kps_gu);
   pf_lowrank_split(I, lrb, P.ks_d, P.kps_d);
@@ -2211,6 +2285,7 @@ static TpPlan tp_plan(const glq_turbo_prefill_params* p) {
   P.off_pos = take(Pn * 4);
   P.off_stok = take(Pn * 4);
   P.off_tiles = take((int64_t)P.max_tiles * 12 + 4);
+  P.off_lrcnt = take(4 * (int64_t)pf_lrcnt(P.max_tiles, P.tm));
   const int64_t lp = r > 0 ? std::max<int64_t>(P.ks_gu > 1 ? P.ks_gu * Pn * 2 * r * 4 : 0,
                                                P.ks_d > 1 ? P.ks_d * Pn * r * 4 : 0)
                            : 0;
@@ -2220,7 +2295,7 @@ static TpPlan tp_plan(const glq_turbo_prefill_params* p) {
   P.off_inter = take(Pn * I * 2);
   P.off_tmp = take(p->signs[1] ? Pn * I * 2 : 0);
   P.off_xd = take(Pn * I * 2);
-  P.off_y = take(Pn * H * 4);
+  P.off_y = take(P.yks * Pn * H * 4);
   P.off_sinter = take(SI > 0 ? T * SI * 2 : 0);
   P.off_sy = take(SI > 0 ? pf_shared_sy_elems(T, H, SI, P.stm) * 4 : 0);
   P.total = o;
@@ -2285,12 +2360,6 @@ static int tp_rotate(const __half* x, int64_t rows, int64_t d, const void* Pi, _
   g.max_tiles = (int)((rows + 63) / 64);
   return pt_launch_k<kPtHalf, 2, 2, 1, kPfDense, false, false, false>(g, s);
 }
-
-template <int MODE>
-static int tp_gemm(const PfArgs& g, int tm, hipStream_t s) {
-  if (tm == 64) return pt_launch_k<kPtTurbo, 1, 4, 2, MODE, false, false, false>(g, s);
-  return pt_launch_k<kPtTurbo, 1, 4, 1, MODE, false, false, false>(g, s);
-}
 }  // namespace glq
 
 extern "C" int64_t glq_turbo_moe_prefill_workspace_bytes(const glq_turbo_prefill_params* p) {
@@ -2331,6 +2400,9 @@ extern "C" int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* wo
   a.stok = (int32_t*)(w + P.off_stok);
   a.tiles = (int32_t*)(w + P.off_tiles);
   a.ntiles = a.tiles + 3 * P.max_tiles;
+  a.lrcnt = (unsigned*)(w + P.off_lrcnt);
+  a.n_lrcnt = pf_lrcnt(P.max_tiles, P.tm);
+  a.yks = P.yks;
   a.ybuf = (const float*)(w + P.off_y);
   a.sy = SI > 0 ? (const float*)(w + P.off_sy) : nullptr;
   a.syh = (const __half*)p->shared_y;
@@ -2349,6 +2421,15 @@ extern "C" int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* wo
   // 2-3. routing and dispatch
   rc = pf_route_launch(a, s);
   if (rc) return rc;
+  PfShared sh;
+  const PfShared* shared = nullptr;
+  if (SI > 0) {
+    sh = pf_shared(T, H, SI, p->shared_bits, P.stm, true, a.xps, p->shared_codes,
+                   p->shared_scales, p->shared_zeros, hp(P.off_sinter),
+                   (float*)(w + P.off_sy));
+    shared = &sh;
+    a.sks = sh.down.ks;
+  }
   // 4. a = x U for gate and up per pair, 5. gate/up + SwiGLU -> inter
   auto lowrank = [&](const __half* x, const int32_t* arow, int m0, int nmat, int64_t K, int ks,
                      int kps, __half* out) {
@@ -2370,6 +2451,7 @@ extern "C" int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* wo
     L.ks = ks;
     L.kps = kps;
     L.part = (float*)(w + P.off_lp);
+    L.cnt = a.lrcnt;
     L.a_out = out;
     return pf_lowrank_launch(L, P.max_tiles * ((P.tm + kLrRows - 1) / kLrRows), s);
   };
@@ -2402,7 +2484,7 @@ extern "C" int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* wo
     g.rank = (int)r;
     g.ntn = pt_tiles_n(I, kPfGateUp, P.tm);
     g.max_tiles = P.max_tiles;
-    rc = tp_gemm<kPfGateUp>(g, P.tm, s);
+    rc = pf_routed_launch<kPtTurbo, kPfGateUp>(g, P.tm, shared, s);
     if (rc) return rc;
   }
   // 6. a = inter U_down per pair, 7. the down's input rotated, in decode order
@@ -2442,18 +2524,15 @@ extern "C" int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* wo
     g.M = (int)Pn; g.K = (int)I; g.N = (int)H; g.G = (int)(I / 128);
     g.rank = (int)r;
     g.ntn = pt_tiles_n(H, kPfDown, P.tm);
-    g.ks = 1; g.gps = g.G;
+    g.ks = P.yks; g.gps = P.ygps;
+    g.yf_ss = Pn * H;
     g.max_tiles = P.max_tiles;
-    rc = tp_gemm<kPfDown>(g, P.tm, s);
+    rc = pf_routed_launch<kPtTurbo, kPfDown>(g, P.tm, shared, s);
     if (rc) return rc;
   }
-  // 9. shared expert, 10. combine
-  if (SI > 0) {
-    rc = pf_shared_launch(T, H, SI, p->shared_bits, P.stm, a.xps, p->shared_codes,
-                          p->shared_scales, p->shared_zeros, hp(P.off_sinter),
-                          (float*)(w + P.off_sy), a.sks, s);
-    if (rc) return rc;
-  }
+  // 9. shared expert (2-bit or larger tiles), 10. combine
+  rc = pf_shared_launch(shared, P.tm, s);
+  if (rc) return rc;
   pf_moe_combine_kernel<<<dim3((unsigned)((T * H / 4 + 255) / 256)), dim3(256), 0, s>>>(a);
   GLQ_LAUNCH_CHECK("pf_moe_combine_kernel");
   return GLQ_OK;

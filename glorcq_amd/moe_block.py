@@ -255,12 +255,26 @@ class GraphCompatibleMoeBlock(nn.Module):
 
     MAX_TOKENS = 64  # tokens per decode step (glq_moe_decode)
 
+    def _as_prompt(self, T: int) -> bool:
+        """T tokens run as one glq_moe_prefill: more than a decode step takes,
+        and from 17 tokens where its grouped GEMMs (an expert's codes decoded
+        once for its tokens, the shared expert in the routed launches) beat
+        consecutive 16-token steps or the many-token step -- past 32 tokens,
+        or from two picks an expert (the measured crossing).  Step against
+        prompt, us, graph replays: 60 experts top-4, 20 tokens 124 / 126, 32
+        150 / 130, 64 241 / 141; 128 experts top-8, 20 120 / 142, 32 154 / 152,
+        64 299 / 155; 8 experts top-2, 17 346 / 239, 64 873 / 271."""
+        if T > self.MAX_TOKENS:
+            return True
+        return (T > 16 and (T > 32 or T * self.top_k >= 2 * self.num_experts)
+                and self.zeros_integral and self.rank % 8 == 0 and self.rank <= 128)
+
     def forward(self, hidden_states: torch.Tensor, residual: torch.Tensor | None = None):
         """(final (b, s, H) fp16, router_logits (b*s, E) fp16), as the
         reference's forward (moe_block.py:381-436); final alone when
-        return_router_logits is False.  Up to 64 tokens run as one decode step
-        (glorcq_hip::moe_decode); more (a prefill) run through
-        glorcq_hip::moe_prefill.
+        return_router_logits is False.  Up to 16 tokens run as one decode step
+        (glorcq_hip::moe_decode); a prefill, and the larger batches that
+        _as_prompt names, through glorcq_hip::moe_prefill.
         residual (the shape of hidden_states, fp16): final becomes
         fp16(residual + fp16(block output)), the decoder layer's residual add,
         inside the step's last launch."""
@@ -294,7 +308,7 @@ class GraphCompatibleMoeBlock(nn.Module):
             out = out.reshape(shape)
             return (out, lg) if self.return_router_logits else out
         codes, scales, zeros, U, cl, SV, u_slot, u_rows, sc, ss, sz = self._op_args()
-        if h.shape[0] <= self.MAX_TOKENS:
+        if not self._as_prompt(h.shape[0]):
             out, logits = torch.ops.glorcq_hip.moe_decode(
                 h, t["router_w"], t["shared_gate_w"], codes, scales, zeros, U, cl, SV, u_slot,
                 u_rows, sc, ss, sz, res, self.inter, self.top_k, self.norm_topk_prob, self.rank,

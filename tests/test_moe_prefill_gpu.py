@@ -162,3 +162,38 @@ def test_prefill_tile_edges(gpu, T, E, top_k, H, inter, bits):
     p = lora_heavy(fmt.make_moe(B=T, seed=seed, **args))
     _, out, logits = run(p, gpu)
     check(p, out, logits, str((T, E, top_k, H, inter, bits)))
+
+
+@pytest.mark.parametrize("T,E,top_k,kw", [
+    (17, 8, 2, {}),                        # from 16 tokens: two picks an expert
+    (32, 40, 4, dict(shared_inter=1152)),  # the shared expert in the routed launches, 9 groups
+    (33, 16, 1, dict(shared_bits=2)),      # past 32 tokens; 2-bit shared weights: own launches
+    (64, 4, 2, dict(inter=2304, shared_inter=0)),  # routed down in K splits (18 groups)
+], ids=str)
+def test_large_decode_batches(gpu, T, E, top_k, kw):
+    """17 to 64 tokens where they run as a prompt: against the oracle, the same
+    bits on graph replays with eager work between them (the low-rank counters
+    are cleared by every call)."""
+    args = dict(H=512, E=E, inter=640, top_k=top_k, n_clusters=3, rank=40, shared_inter=512)
+    args.update(kw)
+    seed = next(s for s in range(10, 80) if margin(fmt.make_moe(B=T, seed=s, **args)) >= 2)
+    p = lora_heavy(fmt.make_moe(B=T, seed=seed, **args))
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+    assert blk._as_prompt(T)
+    h = p.h.reshape(1, T, p.H).to(gpu)
+    out, logits = blk(h)
+    torch.cuda.synchronize()
+    check(p, out.reshape(T, p.H).cpu(), logits.cpu(), str((T, E, kw)))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        blk(h)
+    torch.cuda.current_stream().wait_stream(s)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        gout, glog = blk(h)
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(gout, out) and torch.equal(glog, logits)
+        assert torch.equal(blk(h)[0], out)
