@@ -263,10 +263,12 @@ class GraphCompatibleMoeBlock(nn.Module):
         or from two picks an expert (the measured crossing).  Step against
         prompt, us, graph replays: 60 experts top-4, 20 tokens 124 / 126, 32
         150 / 130, 64 241 / 141; 128 experts top-8, 20 120 / 142, 32 154 / 152,
-        64 299 / 155; 8 experts top-2, 17 346 / 239, 64 873 / 271."""
+        64 299 / 155; 8 experts top-2, 17 346 / 239, 64 873 / 271.  What the
+        step refuses (512 picks, hidden in 256s) it still gets to refuse."""
         if T > self.MAX_TOKENS:
             return True
         return (T > 16 and (T > 32 or T * self.top_k >= 2 * self.num_experts)
+                and T * self.top_k <= 512 and self.hidden % 256 == 0
                 and self.zeros_integral and self.rank % 8 == 0 and self.rank <= 128)
 
     def forward(self, hidden_states: torch.Tensor, residual: torch.Tensor | None = None):

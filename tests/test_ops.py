@@ -163,3 +163,20 @@ def test_direct_call_where_the_dispatch_adds_nothing(gpu):
     with torch.autograd.forward_ad.dual_level():
         assert not K_._plain(t["x"])
     assert not K_._plain(p.x)  # a CPU tensor
+
+
+@pytest.mark.parametrize("T,top_k,E,hidden,prompt", [
+    (16, 8, 8, 2048, False), (17, 2, 8, 2048, True), (17, 4, 60, 2048, False),
+    (33, 4, 60, 2048, True), (64, 8, 128, 2048, True),
+    (33, 16, 128, 2048, False), (64, 4, 60, 384, False),  # the step refuses these
+    (65, 16, 128, 384, True),
+])
+def test_moe_batches_that_run_as_a_prompt(T, top_k, E, hidden, prompt):
+    """The rule that sends a batch to glq_moe_prefill leaves what the decode
+    step refuses (more than 512 picks, a hidden width not of 256s) to it."""
+    from types import SimpleNamespace
+
+    from glorcq_amd.moe_block import GraphCompatibleMoeBlock as B
+    blk = SimpleNamespace(MAX_TOKENS=B.MAX_TOKENS, top_k=top_k, num_experts=E, hidden=hidden,
+                          zeros_integral=True, rank=64)
+    assert B._as_prompt(blk, T) is prompt
