@@ -1217,6 +1217,7 @@ constexpr int64_t kPfSyncBytes = 4096;
 //   14336, 4096, 2, 150: 118.9 / 166.7, 157.7 2048: 449.5 / 324.7, 536.7
 //   768, 2048, 2,  1024: 26.6 / 31.3, 25.3    2048:  33.2 / 34.3, 38.9
 static int pt_dense_tile(int64_t M, int64_t K, int64_t N, int bits) {
+  if (N * K * bits / 8 >= (1ll << 32)) return 0;  // its code offsets have 32 bits
   const double G = (double)(K / 128), nt = (double)((N + 255) / 256);
   const double t64 = 18 + 1.42 * G * std::max(1.0, (double)((M + 63) / 64) * nt / 256);
   const double t32 = 20 + 1.0 * G * std::max(1.0, (double)((M + 31) / 32) * nt / 256);
@@ -2339,7 +2340,8 @@ static int tp_check(const glq_turbo_prefill_params* p) {
     GLQ_CHECK((p->signs[i] != nullptr) != (p->Pi[i] != nullptr),
               "one rotation, signs or Pi, is needed for %s", i ? "down" : "gate and up");
     const int64_t d = i ? I : H;
-    GLQ_CHECK(p->Pi[i] == nullptr || al16(p->Pi[i]), "Pi must be 16-byte aligned");
+    GLQ_CHECK(p->Pi[i] == nullptr || (al16(p->Pi[i]) && d <= 32768),
+              "Pi must be 16-byte aligned, its width <= 32768 (got %lld)", (long long)d);
     GLQ_CHECK(p->signs[i] == nullptr || ((d & (d - 1)) == 0 && d <= 32768),
               "the Hadamard transform takes a power of two <= 32768 (got %lld)", (long long)d);
   }

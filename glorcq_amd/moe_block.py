@@ -767,7 +767,7 @@ def _turbo_prefill_ok(blk: GraphCompatibleMoeBlock, T: int) -> bool:
             and blk.hidden % 128 == 0 and blk.hidden <= 4096  # the decode router's limit
             and blk.inter % 128 == 0 and blk.num_experts <= 256
             and blk.top_k <= 16 and blk.rank % 8 == 0 and blk.rank <= 128
-            and blk.inter <= 1 << 16
+            and blk.inter <= 1 << 15  # Pi's offsets have 32 bits
             and T * blk.top_k * max(blk.hidden, blk.inter, blk.shared_inter) < 1 << 31)
 
 

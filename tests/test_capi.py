@@ -316,3 +316,27 @@ def test_turbo_prefill_checks_arguments(lib):
     assert lib.glq_turbo_moe_prefill(ctypes.byref(q), 1 << 12, 1 << 30, None) == 1
     q = params(hidden=384, inter=512)  # the transform takes powers of two
     assert lib.glq_turbo_moe_prefill(ctypes.byref(q), 1 << 12, 1 << 30, None) == 1
+
+
+def test_tile_form_takes_no_weights_past_32_bit_offsets(lib):
+    """Codes (or a rotation) of 4 GB and more stay with the form whose offsets
+    have 64 bits (without a low-rank term that one needs no workspace, and the
+    tile form does), or are refused."""
+    import ctypes
+
+    from glorcq_amd import _lib
+
+    # the size is the larger of the 2- and 4-bit plans'
+    assert lib.glq_gemm_workspace_bytes(64, 16384, (1 << 20) - 256, 0) > 0
+    assert lib.glq_gemm_workspace_bytes(64, 16384, 1 << 20, 0) == 0
+    q = _lib.TurboPrefillParams()
+    for k, v in dict(tokens=40, hidden=512, experts=8, inter=1 << 16, top_k=2, h=1 << 12,
+                     router_w=1 << 12, out=1 << 12).items():
+        setattr(q, k, v)
+    for i in range(3):
+        q.codes[i] = q.norms[i] = q.centroids[i] = 1 << 12
+    q.signs[0], q.Pi[1] = 1 << 12, 1 << 12
+    assert lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(q)) == -1
+    assert b"Pi" in lib.glq_last_error()
+    q.inter = 1 << 15
+    assert lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(q)) > 0
