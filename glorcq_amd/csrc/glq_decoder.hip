@@ -483,8 +483,9 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_attention_kernel(AttnAr
       float* wv = (float*)&w;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        // (a head whose scores are all -inf so far has m = -inf: no weight)
-        wv[j] = in && m[j] != -__builtin_inff() ? expf(s[i][j] - m[j]) : 0.f;
+        // (a score of -inf has no weight, also while m is -inf; a NaN score,
+        // which m passes over, gives a NaN weight)
+        wv[j] = in && s[i][j] != -__builtin_inff() ? expf(s[i][j] - m[j]) : 0.f;
         l[j] += wv[j];
       }
       if (kb < 2) *(float4*)(pw + (16 * i + li) * 8 + 4 * kb) = w;
@@ -558,7 +559,8 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_attention_kernel(AttnAr
   const int h = tid >> 5, l32 = tid & 31;
   float M = -__builtin_inff(), den = 0.f, r0 = 0.f, r1 = 0.f, r2 = 0.f, r3 = 0.f;
   auto merge = [&](float ms, float ls, float4 os) {
-    if (ms == -__builtin_inff()) return;  // no position, or none with a weight
+    // no position with a weight (scores that are all NaN leave ms = -inf, ls = NaN)
+    if (ms == -__builtin_inff() && ls == 0.f) return;
     const float Mn = fmaxf(M, ms);
     const float fo = expf(M - Mn), fn = expf(ms - Mn);  // M = -inf: fo = 0
     den = den * fo + ls * fn;

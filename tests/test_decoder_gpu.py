@@ -333,3 +333,48 @@ def test_decode_attention_splits(gpu, B, Hq, Hk, L, maxlen):
         ref = (torch.softmax(s, dim=-1) @ V).reshape(-1)
         err = (out[b].double() - ref).abs()
         assert bool((err <= 1e-3 + 2e-3 * ref.abs()).all()), float(err.max())  # fp16 rounding
+
+
+@pytest.mark.parametrize("B,Hq,Hk,L,at", [
+    (2, 8, 1, 33, (32,)),             # the one position of its wave
+    (2, 8, 1, 64, range(32)),         # a wave's whole first block
+    (1, 4, 1, 300, (0,)),             # 4 heads a group; in the first split of three
+    (1, 8, 1, 257, (256,)),           # the one position of its split
+    (1, 8, 1, 640, range(128, 256)),  # every position of a split
+    (64, 64, 8, 200, range(32, 64)),  # one workgroup a group, two blocks a wave
+])
+def test_decode_attention_nan_key(gpu, B, Hq, Hk, L, at):
+    """A NaN in a key is a NaN in its group's outputs wherever its position
+    falls (a wave's or split's only scores among them), as softmax has it; the
+    other groups and sequences, and scores of -inf, stay finite."""
+    hd = 128
+    g = torch.Generator(device=gpu).manual_seed(L)
+    q = torch.randn(B, Hq, hd, generator=g, device=gpu).half()
+    q[..., 0] = 1.0
+    kc = torch.randn(B, Hk, 1024, hd, generator=g, device=gpu).half()
+    vc = torch.randn(B, Hk, 1024, hd, generator=g, device=gpu).half()
+    ln = torch.tensor([L], dtype=torch.int32, device=gpu)
+    ws = kernels.decode_attention_workspace(q, kc)
+
+    def run():
+        out = kernels.decode_attention(q, kc, vc, ln, hd ** -0.5, workspace=ws)
+        torch.cuda.synchronize()
+        return out.reshape(B, Hk, -1)
+
+    for p in at:
+        kc[0, 0, p, 5] = float("nan")
+    out = run()
+    assert bool(out[0, 0].isnan().all())
+    out[0, 0] = 0.0
+    assert not bool(out.isnan().any())
+    # the same positions with no weight at all: a score of -inf
+    for p in at:
+        kc[0, 0, p, 5] = 0.0
+        kc[0, 0, p, 0] = float("-inf")
+    out = run()
+    keep = [p for p in range(L) if p not in set(at)]
+    K, V = kc[0, 0, keep].double(), vc[0, 0, keep].double()
+    s = q[0].double().reshape(Hk, -1, hd)[0] @ K.T * hd ** -0.5
+    ref = (torch.softmax(s, dim=-1) @ V).reshape(-1)
+    err = (out[0, 0].double() - ref).abs()
+    assert bool((err <= 1e-3 + 2e-3 * ref.abs()).all()), float(err.max())  # fp16 rounding
