@@ -392,6 +392,14 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
+// Orders LDS accesses of one wave's lanes among themselves (the hardware keeps
+// a wave's LDS accesses in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // RH: heads of a lane's sums (4 or 8, at least rep).
 template <bool XU, int RH>
 __global__ __launch_bounds__(kDecThreads, 2) void decode_attention_kernel(AttnArgs a) {
@@ -490,6 +498,7 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_attention_kernel(AttnAr
       }
       if (kb < 2) *(float4*)(pw + (16 * i + li) * 8 + 4 * kb) = w;
     }
+    wave_lds_sync();  // the wave's weights are written
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int p = 4 * i + kb;
@@ -503,6 +512,7 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_attention_kernel(AttnAr
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[h][e] = fmaf(w[h], (float)v[e], o[h][e]);
     }
+    wave_lds_sync();  // and read
   };
   {
     Block x, y;
