@@ -897,6 +897,13 @@ def moe_decode_launch(h, router_w, shared_gate_w, codes, scales, zeros, U, clust
     return out, logits
 
 
+def _scratch(device, nbytes) -> torch.Tensor:
+    """Scratch of one prompt call, from torch's allocator: the call leaves
+    nothing in it, and a captured call gets memory of its own graph, so graphs
+    captured on one stream may be replayed on several."""
+    return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
+
+
 def moe_prefill_launch(h, router_w, shared_gate_w, codes, scales, zeros, U, cluster_of, SV,
                        u_slot, u_rows, shared_codes, shared_scales, shared_zeros, residual, inter,
                        top_k, norm_topk_prob, rank, n_clusters, bits, shared_bits, shared_inter,
@@ -926,8 +933,7 @@ def moe_prefill_launch(h, router_w, shared_gate_w, codes, scales, zeros, U, clus
     n = lib.glq_moe_prefill_workspace_bytes(ctypes.byref(P))
     if n < 0:
         _lib.check(1, "glq_moe_prefill_workspace_bytes")
-    from .kernels import workspace
-    ws = workspace(h.device, max(int(n), 256))
+    ws = _scratch(h.device, n)
     _lib.check(lib.glq_moe_prefill(ctypes.byref(P), ws.data_ptr(), ws.numel(),
                                    _lib.stream_handle(h.device)), "glq_moe_prefill")
     return out, logits

@@ -90,3 +90,66 @@ def test_replaced_workspace_survives_for_captured_graph(gpu):
         torch.cuda.synchronize()
         assert torch.equal(y, eager), f"replay {i}"
         assert all(bool((t == 7).all()) for t in sentinels), f"replay {i} wrote into new memory"
+
+
+def _recorded(monkeypatch, name, ws_arg):
+    """Wraps a library entry point; the list collects its calls' workspaces as
+    (first byte, bytes)."""
+    from glorcq_amd import _lib
+
+    lib, seen = _lib.load(), []
+    real = getattr(lib, name)
+
+    def call(*a):
+        seen.append((a[ws_arg], a[ws_arg + 1]))
+        return real(*a)
+
+    monkeypatch.setattr(lib, name, call)
+    return seen
+
+
+def _two_graphs(gpu, seen, calls):
+    """Captures the calls on one stream, a graph each, checks that their
+    scratch does not overlap, and replays them on two streams at once."""
+    stream = torch.cuda.Stream()
+    graphs, outs, eager, spans = [], [], [], []
+    for call in calls:
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            eager.append(call().clone())
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        n = len(seen)
+        with torch.cuda.graph(g, stream=stream):
+            outs.append(call())
+        assert len(seen) > n, "the call under test was not reached"
+        spans.append(seen[n:])
+        graphs.append(g)
+    assert all(a + n <= b or b + m <= a for a, n in spans[0] for b, m in spans[1]), spans
+    sides = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for i in range(3):
+        for o in outs:
+            o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for s, g in zip(sides, graphs):
+            with torch.cuda.stream(s):
+                for _ in range(4):
+                    g.replay()
+        torch.cuda.synchronize()
+        for o, e in zip(outs, eager):
+            assert torch.equal(o, e), f"replay {i}"
+
+
+def test_moe_batch_graphs_of_one_stream_replay_on_two(gpu, monkeypatch):
+    """MoE batches that run as a prompt, of two sizes, captured on one stream:
+    each graph has its own scratch, so they may run side by side."""
+    from glorcq_amd import format as fmt
+    from glorcq_amd.moe_block import GraphCompatibleMoeBlock
+
+    p = fmt.make_moe(H=512, E=8, inter=640, top_k=2, n_clusters=3, rank=40, shared_inter=512,
+                     B=64, seed=3)
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+    hs = [p.h[:T].reshape(1, T, p.H).to(gpu) for T in (64, 20)]
+    assert all(blk._as_prompt(h.shape[1]) for h in hs)
+    seen = _recorded(monkeypatch, "glq_moe_prefill", 1)
+    _two_graphs(gpu, seen, [lambda h=h: blk(h)[0] for h in hs])
