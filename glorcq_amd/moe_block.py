@@ -811,8 +811,7 @@ def turbo_prefill(blk: GraphCompatibleMoeBlock, h: torch.Tensor, res: torch.Tens
     n = lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(p))
     if n < 0:
         _lib.check(1, "glq_turbo_moe_prefill_workspace_bytes")
-    from .kernels import workspace
-    ws = workspace(h.device, max(int(n), 256))
+    ws = _scratch(h.device, n)
     _lib.check(lib.glq_turbo_moe_prefill(ctypes.byref(p), ws.data_ptr(), ws.numel(),
                                          _lib.stream_handle(h.device)), "glq_turbo_moe_prefill")
     return out, logits

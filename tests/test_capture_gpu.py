@@ -153,3 +153,16 @@ def test_moe_batch_graphs_of_one_stream_replay_on_two(gpu, monkeypatch):
     assert all(blk._as_prompt(h.shape[1]) for h in hs)
     seen = _recorded(monkeypatch, "glq_moe_prefill", 1)
     _two_graphs(gpu, seen, [lambda h=h: blk(h)[0] for h in hs])
+
+
+def test_turbo_prompt_graphs_of_one_stream_replay_on_two(gpu, monkeypatch):
+    """The same for TurboQuant prompts."""
+    from glorcq_amd import format as fmt
+    from glorcq_amd.moe_block import GraphCompatibleMoeBlock
+
+    p = fmt.make_turbo_moe(H=512, E=6, inter=384, top_k=2, n_clusters=3, rank=64, B=100, seed=3,
+                           rot_gate_up="rht", rot_down="qr")
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+    hs = [p.h[:T].reshape(1, T, p.H).to(gpu) for T in (100, 17)]
+    seen = _recorded(monkeypatch, "glq_turbo_moe_prefill", 1)
+    _two_graphs(gpu, seen, [lambda h=h: blk(h)[0] for h in hs])
