@@ -27,6 +27,18 @@ int64_t pf_gemm_prefill_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t
 namespace {
 // ranks above this take the low-rank entry point before the GEMM
 constexpr int64_t kInLaunchRank = 128;
+// the counter words at the start of the workspace (kPfSyncBytes of glq_prefill.hip)
+constexpr int64_t kCounterBytes = 4096;
+
+// Bytes of the GEMM's own part of the workspace, enough for either code width
+// (the plan's token tile depends on it).  Where the low-rank entry point forms
+// x U, the GEMM has none to form, but the workspace's counter words stay free.
+int64_t prefill_ws(int64_t M, int64_t K, int64_t N, int64_t rank) {
+  const int64_t r = rank > kInLaunchRank ? 0 : rank;
+  const int64_t n = std::max(glq::pf_gemm_prefill_workspace_bytes(M, K, N, r, 2),
+                             glq::pf_gemm_prefill_workspace_bytes(M, K, N, r, 4));
+  return r == rank ? n : std::max(n, kCounterBytes);
+}
 
 int64_t lowrank_block_ws(int64_t M, int64_t K, int64_t rank) {
   const int64_t full = M / 16, tail = M % 16;
@@ -36,12 +48,10 @@ int64_t lowrank_block_ws(int64_t M, int64_t K, int64_t rank) {
 }
 }  // namespace
 
-// Enough for either code width (the plan's token tile depends on it).
 extern "C" int64_t glq_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   if (rank < 0) return -1;
-  const int64_t pf = std::max(glq::pf_gemm_prefill_workspace_bytes(M, K, N, rank, 2),
-                              glq::pf_gemm_prefill_workspace_bytes(M, K, N, rank, 4));
+  const int64_t pf = prefill_ws(M, K, N, rank);
   if (rank > kInLaunchRank) return pf + lowrank_block_ws(M, K, rank);
   return pf;
 }
@@ -82,8 +92,7 @@ extern "C" int glq_gemm_lora(const void* x, int64_t M, int64_t K, int64_t N,
   if (lora && !xU && rank > kInLaunchRank) {
     // a = fp16(x U) by the low-rank entry point (16-row blocks), past the
     // prefill workspace
-    char* xw = (char*)workspace + std::max(glq::pf_gemm_prefill_workspace_bytes(M, K, N, rank, 2),
-                                           glq::pf_gemm_prefill_workspace_bytes(M, K, N, rank, 4));
+    char* xw = (char*)workspace + prefill_ws(M, K, N, rank);
     const int64_t xneed = lowrank_block_ws(M, K, rank);
     const int64_t pbytes = xneed - align_up(M * rank * 2, 256);
     __half* abuf = (__half*)(xw + pbytes);

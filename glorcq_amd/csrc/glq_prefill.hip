@@ -1204,24 +1204,49 @@ constexpr int64_t kPfSyncBytes = 4096;
 
 // Token tile of the tile form (64 or 32, x 256 rows) for a dense launch, or 0
 // where pf_gemm_kernel's smaller tiles are the better form: estimates of the
-// three in us, from measured calls with x U (rank 64).  A workgroup of the
-// tile form takes 1.42 us a group at 64 tokens, 1 us at 32 (a CU's workgroups
-// share its rate, so from 256 tiles on time grows with the tiles) after
-// 18-20 us of the x launch, first loads and stores; pf_gemm_kernel about 470
-// TF/s after 12 us and 0.85 (2-bit) or 0.55 (4-bit) us a group of its chain.
+// three in us, with x U formed in the call (xu) or none to form.  Each form's
+// time is a start, then a cost a 128-code group for its first round of 256
+// workgroups and one for every further round (a CU's workgroups share its
+// rate, so a round begun costs nearly a whole one): 257 tiles take as long as
+// 500.  The tile form's launch before costs 7 us with x U; pf_gemm_kernel
+// forms x U in its own grid, where its epilogues wait for it.  The tile form is
+// taken where it is 5 % ahead.  Over 22 shapes (K 512 to 14336, N 512 to
+// 14336, both widths) x 20 row counts from 17 to 2048, the rule's choice is 0.6
+// (xu) and 0.1 % (none) off the best of the three in the mean, and never 3 %
+// slower than pf_gemm_kernel; over 360 further random calls 4 and 0.6 % off,
+// six of them more than 5 % slower than pf_gemm_kernel (the worst 82 against
+// 66 us: 4-bit, 8192, 1000, 336 rows).
 //   (K, N, bits, M): tile form 32 / 64, pf_gemm_kernel (us)
-//   2048, 1408, 2,  512: 34.8 / 43.5, 25.1    2048:  47.7 / 46.7, 57.5
-//   2048, 4096, 4,  512: 37.6 / 44.7, 36.6    1024:  53.0 / 47.5, 66.6
-//   4096, 14336, 2, 256: 71.8 / 65.4, 76.9    2048: 380.6 / 287.8, 426.8
-//   5632, 2048, 4,  256: 62.5 / 81.1, 43.5    1024:  69.8 / 83.8, 103.5
-//   14336, 4096, 2, 150: 118.9 / 166.7, 157.7 2048: 449.5 / 324.7, 536.7
-//   768, 2048, 2,  1024: 26.6 / 31.3, 25.3    2048:  33.2 / 34.3, 38.9
-static int pt_dense_tile(int64_t M, int64_t K, int64_t N, int bits) {
+//   with x U:                                        no x U:
+//   2048, 4096, 4,  512: 35.4 / 41.6, 35.7            26.4 / 31.8, 23.1
+//   2048, 4096, 4, 1024: 51.7 / 45.6, 63.6            41.7 / 36.1, 31.5
+//   4096, 4096, 2,  256: 48.3 / 57.7, 41.5            37.3 / 45.1, 31.8
+//   4096, 4096, 4,  640: 81.1 / 62.6, 75.6            68.2 / 50.3, 54.3
+//   4096, 4096, 4, 2048: 150.7 / 112.2, 160.7         132.9 / 94.3, 111.2
+//   768, 2048, 2,  2048: 33.3 / 33.8, 39.5            25.4 / 25.0, 16.6
+static int pt_dense_tile(int64_t M, int64_t K, int64_t N, int bits, bool xu) {
   if (N * K * bits / 8 >= (1ll << 32)) return 0;  // its code offsets have 32 bits
-  const double G = (double)(K / 128), nt = (double)((N + 255) / 256);
-  const double t64 = 18 + 1.42 * G * std::max(1.0, (double)((M + 63) / 64) * nt / 256);
-  const double t32 = 20 + 1.0 * G * std::max(1.0, (double)((M + 31) / 32) * nt / 256);
-  const double old = 12 + (bits == 2 ? 0.85 : 0.55) * G + 2e-6 * (double)M * N * K / 470;
+  const auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const double G = (double)(K / 128);
+  // us of a launch of tm x wr tiles
+  const auto us = [&](int tm, int wr, double start, double first, double more) {
+    return start + G * (first + more * (double)(up(up(M, tm) * up(N, wr), 256) - 1));
+  };
+  double t64, t32, old;
+  const bool big = up(M, 64) * up(N, 128) >= 256;  // pf_dense_plan's tiles
+  if (xu) {
+    t64 = us(64, 256, 20, 1.25, 0.87);
+    t32 = us(32, 256, 18, 0.92, 0.91);
+    old = big        ? us(64, 128, 11.7, 1.47, 0.98)
+          : M >= 256 ? us(32, 128, 14.7, 1.04, 0.28)
+                     : us(16, 64, 12.6, 0.58, 0.42);
+  } else {
+    t64 = us(64, 256, 13, 1.27, 0.87);
+    t32 = us(32, 256, 11, 0.95, 0.92);
+    old = big        ? us(64, 128, 5.6, 1.05, 0.74)
+          : M >= 256 ? us(32, 128, 4.6, 0.76, 0.36)
+                     : us(16, 64, 4.3, 0.52, 0.475);
+  }
   if (std::min(t32, t64) >= 0.95 * old) return 0;
   return t64 <= t32 ? 64 : 32;
 }
@@ -1283,7 +1308,13 @@ static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, 
   P.ks = (G + P.gps - 1) / P.gps;
   P.pt = 0;
   P.xp_bytes = P.c2_bytes = P.c2_ld = 0;
-  if (ks == 1 && !env.get("GLQ_PF_CFG")) P.pt = pt_dense_tile(M, K, N, bits);
+  if (ks == 1 && !env.get("GLQ_PF_CFG")) {
+    P.pt = pt_dense_tile(M, K, N, bits, rank > 0);
+    if (const char* e = env.get("GLQ_PF_TILE")) {  // the tile form (0: not) of 32 or 64 tokens
+      const int v = atoi(e);
+      if (v == 0 || ((v == 32 || v == 64) && N * K * bits / 8 < (1ll << 32))) P.pt = v;
+    }
+  }
   pf_lowrank_split(K, (M + kLrRows - 1) / kLrRows, P.lr_ks, P.lr_kps);
   if (P.pt) {
     // x in decode order, its group sums (whole tiles of rows), a and its

@@ -148,6 +148,36 @@ def test_split_k_variants(gpu, monkeypatch, ks, K, N, M, bits, rank):
     assert torch.equal(y, y2)  # fixed summation order: the same bits every call
 
 
+def tile_form(monkeypatch, M, K, N, rank, tile=None):
+    """The workspace of the form that a call takes differs from the other
+    form's (GLQ_PF_TILE=0): the rule, or GLQ_PF_TILE=tile, takes the tile form
+    for one of the two code widths at least."""
+    lib = _lib.load()
+    with monkeypatch.context() as m:
+        if tile is not None:
+            m.setenv("GLQ_PF_TILE", str(tile))
+        size = lib.glq_gemm_workspace_bytes(M, K, N, rank)
+        m.setenv("GLQ_PF_TILE", "0")
+        return size != lib.glq_gemm_workspace_bytes(M, K, N, rank)
+
+
+@pytest.mark.parametrize("K,N,M,rank,tile", [
+    (768, 2048, 2048, 0, False),    # no x U to form: 16.6 us in small tiles, 25.0 in the tile form
+    (1408, 2048, 1024, 0, False),   # 17.5 / 24.3
+    (2048, 4096, 512, 0, False),    # 23.1 / 26.4
+    (4096, 4096, 640, 0, True),     # 54.3 / 50.3
+    (4096, 4096, 256, 64, False),   # one round of small tiles: 41.5 / 48.3
+    (2048, 4096, 777, 64, True),    # 64.6 / 43.9
+    (4096, 4096, 2048, 64, True),   # 160.7 / 112.2
+    (4096, 4096, 2048, 0, True),    # 111.2 / 94.3
+])
+def test_dense_form_rule(monkeypatch, K, N, M, rank, tile):
+    """The tile form is taken where it is the faster one, with x U formed in the
+    call and without (us of the small tiles / the tile form; 4-bit codes, 2-bit
+    at K of 768 and 1408)."""
+    assert tile_form(monkeypatch, M, K, N, rank) is tile
+
+
 def test_gemm_requires_workspace():
     """The prefill path takes a workspace (split-K tiles, a = x U): a missing
     or short one is an argument error, raised before any launch."""
