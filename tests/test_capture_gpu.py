@@ -166,3 +166,24 @@ def test_turbo_prompt_graphs_of_one_stream_replay_on_two(gpu, monkeypatch):
     hs = [p.h[:T].reshape(1, T, p.H).to(gpu) for T in (100, 17)]
     seen = _recorded(monkeypatch, "glq_turbo_moe_prefill", 1)
     _two_graphs(gpu, seen, [lambda h=h: blk(h)[0] for h in hs])
+
+
+@pytest.mark.parametrize("given", [False, True])
+def test_prompt_linear_graphs_of_one_stream_replay_on_two(gpu, monkeypatch, given):
+    """Projections over many rows that form no x U (no low-rank term, or a
+    precomputed one), in the tile form: x in decode order and its group sums
+    are the call's own."""
+    from glorcq_amd import format as fmt
+
+    monkeypatch.setenv("GLQ_PF_TILE", "64")
+    p = fmt.make_linear(1024, 512, bits=4, group=128, rank=16, M=500, seed=5)
+    d = {k: getattr(p, k).to(gpu) for k in ("x", "codes", "scales", "zeros", "U", "SV")}
+    xu = (p.x.float() @ p.U.float()).half().to(gpu)
+
+    def call(M):
+        kw = dict(SV=d["SV"], precomputed_xU=xu[:M]) if given else {}
+        return lambda: K_.packed_dequant_matmul_fused(d["x"][:M], d["codes"], d["scales"],
+                                                      d["zeros"], 4, 128, **kw)
+
+    seen = _recorded(monkeypatch, "glq_gemm_lora", 16)
+    _two_graphs(gpu, seen, [call(500), call(333)])
