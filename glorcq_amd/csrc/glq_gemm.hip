@@ -21,7 +21,7 @@ int pf_dense_gemm(const void* x, int64_t M, int64_t K, int64_t N, const int32_t*
                   const void* SV, int64_t rank, const void* xU, const void* bias, void* y,
                   void* workspace, int64_t workspace_bytes, hipStream_t s);
 int64_t pf_gemm_prefill_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank,
-                                        int bits);
+                                        int bits, bool tile);
 }  // namespace glq
 
 namespace {
@@ -30,13 +30,12 @@ constexpr int64_t kInLaunchRank = 128;
 // the counter words at the start of the workspace (kPfSyncBytes of glq_prefill.hip)
 constexpr int64_t kCounterBytes = 4096;
 
-// Bytes of the GEMM's own part of the workspace, enough for either code width
-// (the plan's token tile depends on it).  Where the low-rank entry point forms
-// x U, the GEMM has none to form, but the workspace's counter words stay free.
-int64_t prefill_ws(int64_t M, int64_t K, int64_t N, int64_t rank) {
+// Bytes of the GEMM's own part of the workspace, with the tile form or without.
+// Where the low-rank entry point forms x U, the GEMM has none to form, but the
+// workspace's counter words stay free.
+int64_t prefill_ws(int64_t M, int64_t K, int64_t N, int64_t rank, int bits, bool tile) {
   const int64_t r = rank > kInLaunchRank ? 0 : rank;
-  const int64_t n = std::max(glq::pf_gemm_prefill_workspace_bytes(M, K, N, r, 2),
-                             glq::pf_gemm_prefill_workspace_bytes(M, K, N, r, 4));
+  const int64_t n = glq::pf_gemm_prefill_workspace_bytes(M, K, N, r, bits, tile);
   return r == rank ? n : std::max(n, kCounterBytes);
 }
 
@@ -48,10 +47,12 @@ int64_t lowrank_block_ws(int64_t M, int64_t K, int64_t rank) {
 }
 }  // namespace
 
+// Enough for either code width (the plan's token tile depends on it).
 extern "C" int64_t glq_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   if (rank < 0) return -1;
-  const int64_t pf = prefill_ws(M, K, N, rank);
+  const int64_t pf = std::max(prefill_ws(M, K, N, rank, 2, true),
+                              prefill_ws(M, K, N, rank, 4, true));
   if (rank > kInLaunchRank) return pf + lowrank_block_ws(M, K, rank);
   return pf;
 }
@@ -84,16 +85,19 @@ extern "C" int glq_gemm_lora(const void* x, int64_t M, int64_t K, int64_t N,
             "x, codes, U, SV and xU must be 16-byte aligned");
   GLQ_CHECK(workspace != nullptr && ((uintptr_t)workspace & 255) == 0,
             "a 256-byte aligned workspace of glq_gemm_workspace_bytes is required");
-  const int64_t need = glq_gemm_workspace_bytes(M, K, N, lora && !xU ? rank : 0);
-  GLQ_CHECK(workspace_bytes >= need, "workspace of %lld bytes needed (got %lld)",
-            (long long)need, (long long)workspace_bytes);
+  // the tile form's workspace where it is given, else what the call takes at
+  // least; x U of a large rank lies past it
+  const int64_t xr = lora && !xU ? rank : 0;
+  const int64_t xneed = xr > kInLaunchRank ? lowrank_block_ws(M, K, rank) : 0;
+  int64_t part = prefill_ws(M, K, N, xr, bits, true);
+  if (workspace_bytes < part + xneed) part = prefill_ws(M, K, N, xr, bits, false);
+  GLQ_CHECK(workspace_bytes >= part + xneed, "workspace of %lld bytes needed (got %lld)",
+            (long long)(part + xneed), (long long)workspace_bytes);
   hipStream_t s = (hipStream_t)stream;
   const void* a = xU;
-  if (lora && !xU && rank > kInLaunchRank) {
-    // a = fp16(x U) by the low-rank entry point (16-row blocks), past the
-    // prefill workspace
-    char* xw = (char*)workspace + prefill_ws(M, K, N, rank);
-    const int64_t xneed = lowrank_block_ws(M, K, rank);
+  if (xneed) {
+    // a = fp16(x U) by the low-rank entry point (16-row blocks)
+    char* xw = (char*)workspace + part;
     const int64_t pbytes = xneed - align_up(M * rank * 2, 256);
     __half* abuf = (__half*)(xw + pbytes);
     const int64_t full = M / 16, tail = M % 16;
@@ -110,6 +114,5 @@ extern "C" int glq_gemm_lora(const void* x, int64_t M, int64_t K, int64_t N,
     a = abuf;
   }
   return pf_dense_gemm(x, M, K, N, codes, bits, scales, zeros, sym, a ? nullptr : U,
-                       lora ? SV : nullptr, lora ? rank : 0, a, bias, y, workspace,
-                       workspace_bytes, s);
+                       lora ? SV : nullptr, lora ? rank : 0, a, bias, y, workspace, part, s);
 }

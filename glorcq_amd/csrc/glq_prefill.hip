@@ -1262,7 +1262,9 @@ struct PfEnv {
   const char* get(const char* name) const { return any ? getenv(name) : nullptr; }
 };
 
-static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, int bits) {
+// tile: the tile form may be taken.
+static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, int bits,
+                                 bool tile) {
   PfDensePlan P;
   const PfEnv env;
   // Big launches (a 64 x 128 tile per CU or more): 64-token tiles, shallow
@@ -1308,7 +1310,7 @@ static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, 
   P.ks = (G + P.gps - 1) / P.gps;
   P.pt = 0;
   P.xp_bytes = P.c2_bytes = P.c2_ld = 0;
-  if (ks == 1 && !env.get("GLQ_PF_CFG")) {
+  if (tile && ks == 1 && !env.get("GLQ_PF_CFG")) {
     P.pt = pt_dense_tile(M, K, N, bits, rank > 0);
     if (const char* e = env.get("GLQ_PF_TILE")) {  // the tile form (0: not) of 32 or 64 tokens
       const int v = atoi(e);
@@ -1365,11 +1367,12 @@ static PfDensePlan pf_dense_plan(int64_t M, int64_t K, int64_t N, int64_t rank, 
 // words (zero before the first call, left zero by every call), then a, its
 // partials, the split-K tiles (whose arrival counters the two-launch form's
 // first launch clears); none at all when the call needs no tables.
+// With the tile form allowed, or (tile false) what the call takes at least.
 int64_t pf_gemm_prefill_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank,
-                                        int bits) {
+                                        int bits, bool tile) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   if (rank < 0) return -1;
-  return pf_dense_plan(M, K, N, rank, bits).total;
+  return pf_dense_plan(M, K, N, rank, bits, tile).total;
 }
 
 // The dense GEMM in tile form: x in decode order, a = x U, then the tiles.
@@ -1445,7 +1448,10 @@ int pf_dense_gemm(const void* x, int64_t M, int64_t K, int64_t N, const int32_t*
                   void* workspace, int64_t workspace_bytes, hipStream_t s) {
   const bool lora = SV != nullptr && rank > 0;
   // a = x U needs room only when it is formed here
-  const PfDensePlan P = pf_dense_plan(M, K, N, lora && xU == nullptr ? rank : 0, bits);
+  const int64_t xr = lora && xU == nullptr ? rank : 0;
+  PfDensePlan P = pf_dense_plan(M, K, N, xr, bits, true);
+  // a workspace too small for the tile form takes the other one
+  if (P.pt && workspace_bytes < P.total) P = pf_dense_plan(M, K, N, xr, bits, false);
   GLQ_CHECK(P.total == 0 || (workspace != nullptr && workspace_bytes >= P.total),
             "workspace of %lld bytes needed (got %lld)", (long long)P.total,
             (long long)workspace_bytes);

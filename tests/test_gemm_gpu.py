@@ -192,6 +192,44 @@ def test_gemm_requires_workspace():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rank,given", [(0, False), (64, False), (192, False), (64, True)])
+def test_small_workspace_takes_the_small_tiles(gpu, monkeypatch, rank, given):
+    """A workspace that holds the small tiles' tables and not the tile form's
+    (none at all where no x U is formed) is taken, by the small tiles; a
+    shorter one is refused."""
+    lib = _lib.load()
+    M, K, N = 300, 1024, 520
+    p = fmt.make_linear(K, N, bits=4, rank=max(rank, 8), M=M, seed=rank)
+    d = to(p, gpu)
+    xu = (p.x.float() @ p.U.float()).half().to(gpu)
+    r = 0 if given else rank
+    monkeypatch.setenv("GLQ_PF_TILE", "0")
+    least = lib.glq_gemm_workspace_bytes(M, K, N, r)
+    monkeypatch.setenv("GLQ_PF_TILE", "64")
+    full = lib.glq_gemm_workspace_bytes(M, K, N, r)
+    assert least < full
+
+    def call(nbytes):
+        ws = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=gpu)
+        y = torch.empty(M, N, dtype=torch.float16, device=gpu)
+        rc = lib.glq_gemm_lora(d["x"].data_ptr(), M, K, N, d["codes"].data_ptr(), 4,
+                               d["scales"].data_ptr(), d["zeros"].data_ptr(), 128, 0,
+                               None if given or not rank else d["U"].data_ptr(),
+                               d["SV"].data_ptr() if rank else None, rank,
+                               xu.data_ptr() if given else None, None, y.data_ptr(),
+                               ws.data_ptr(), nbytes, _lib.stream_handle(gpu))
+        torch.cuda.synchronize()
+        return rc, y
+
+    for nbytes in (least, full - 256, full):
+        rc, y = call(nbytes)
+        _lib.check(rc, "glq_gemm_lora")
+        assert_parity(y, oracle_y(p, lora=rank > 0), f"{nbytes} of {least}, {full} bytes")
+    if least:
+        assert call(least - 256)[0] == 1 and b"workspace" in lib.glq_last_error()
+
+
+@pytest.mark.gpu
 def test_config1_down_m512(gpu):
     """The config-1 down projection (1408 -> 2048) at the prefill size M=512."""
     p = fmt.make_linear(1408, 2048, bits=2, group=128, rank=64, M=512, seed=1408 + 512)
