@@ -458,8 +458,9 @@ def _turbo_derived(t: dict) -> None:
         Pi = t[f"Pi_{proj}"]
         t[f"Pi_{proj}_c"] = None if Pi is None else Pi.to(torch.float16).contiguous()
     # glq_turbo_moe_prefill's shared GEMMs take integer zero-points; checked
-    # once here
-    sw = _turbo_shared_weights(t)
+    # once here, for weights of the block's own (a shared expert of modules runs
+    # as its modules, whose weights may be loaded again)
+    sw = _turbo_shared_weights(t) if "shared_q" in t else None
     t["shared_zeros_integral"] = sw is not None and all(
         bool(torch.equal(z, z.round())) for z in sw[2])
     if t["rank"] > 0:
@@ -773,8 +774,9 @@ def _turbo_prefill_ok(blk: GraphCompatibleMoeBlock, T: int) -> bool:
 
 def turbo_prefill(blk: GraphCompatibleMoeBlock, h: torch.Tensor, res: torch.Tensor | None):
     """A prompt through a TurboQuant block (glq_turbo_moe_prefill): (out (T, H)
-    fp16, router logits (T, E) fp16).  A shared expert whose weights its
-    grouped GEMMs do not take runs as its own projections first."""
+    fp16, router logits (T, E) fp16).  A shared expert of modules, or of
+    weights that its grouped GEMMs do not take, runs as its own projections
+    first."""
     lib = _lib.load()
     t = blk.t
     T, H = h.shape
@@ -798,8 +800,8 @@ def turbo_prefill(blk: GraphCompatibleMoeBlock, h: torch.Tensor, res: torch.Tens
         p.Pi[i] = None if t[f"signs_{proj}"] is not None else _lib.ptr(t[f"Pi_{proj}_c"])
     shared = None
     if blk.shared_inter > 0:
-        sw = _turbo_shared_weights(t)
-        if sw is not None and t["shared_zeros_integral"] and blk.shared_inter % 128 == 0:
+        if t["shared_zeros_integral"] and blk.shared_inter % 128 == 0:
+            sw = _turbo_shared_weights(t)
             p.shared_inter, p.shared_bits = blk.shared_inter, 4
             for i in range(3):
                 p.shared_codes[i] = sw[0][i].data_ptr()

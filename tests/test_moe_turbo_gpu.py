@@ -16,6 +16,7 @@ import torch
 import torch.nn as nn
 
 from glorcq_amd import format as fmt
+from glorcq_amd import moe_block
 from glorcq_amd.moe_block import GraphCompatibleMoeBlock
 from oracle import glorcq_oracle as O
 from test_moe_gpu import check_routing, margin
@@ -287,3 +288,37 @@ def test_turbo_prompt(gpu, T, H, inter, rot_gu, rot_down, rank, shared):
         assert not blk.t["shared_zeros_integral"]
         out, _ = run(blk, p, gpu)
         assert bar(out, O.moe_forward(p))
+
+
+def test_turbo_prompt_runs_the_shared_modules(gpu):
+    """A shared expert of modules runs as those modules in a prompt too: their
+    forward hooks fire, and weights loaded again (zero-points that are not
+    integers) are the ones used."""
+    from glorcq_amd.quantized_linear import GLoRCQLinear
+
+    p = problem(20, 6, shared_inter=512, E=16)
+    assert margin(p) >= 2
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+
+    def load(m, q):
+        qi = torch.from_numpy(O.unpack_codes(q.codes[0].numpy(), q.bits, q.K))
+        m.load_gptq({"qweight_int": qi, "scales": q.scales[0], "zeros": q.zeros[0],
+                     "bits": q.bits, "groupsize": q.group, "sym": False}, device=gpu)
+        return m
+
+    mods = tuple(load(GLoRCQLinear(p.shared[s].K, p.shared[s].N), p.shared[s]) for s in fmt.PROJS)
+    del blk.t["shared_q"]  # as a block stacked from modules has them
+    blk.t["shared_mods"] = mods
+    moe_block._turbo_derived(blk.t)
+    seen = []
+    for m in mods:
+        m.register_forward_hook(lambda m, a, y: seen.append(m))
+    out, _ = run(blk, p, gpu)
+    assert set(seen) == set(mods)
+    first = O.moe_forward(p)
+    assert bar(out, first)
+    for s, m in zip(fmt.PROJS, mods):
+        p.shared[s].zeros = (p.shared[s].zeros.float() + 0.25).half()
+        load(m, p.shared[s])
+    out, _ = run(blk, p, gpu)
+    assert bar(out, O.moe_forward(p)) and not bar(out, first)
