@@ -168,13 +168,14 @@ def _plain(*tensors) -> bool:
     """The operator dispatch would only call the eager function: plain GPU
     tensors and nothing that watches, transforms or differentiates the call
     (compile and trace, dispatch and function modes, functorch, forward-mode
-    levels, a gradient to record).  The dispatch of a Python custom operator
-    costs about 7 us of host time, this check 0.5."""
+    levels, a profiler, a gradient to record).  The dispatch of a Python custom
+    operator costs about 7 us of host time, this check 0.5."""
     C = torch._C
     if (torch.compiler.is_compiling() or C._len_torch_dispatch_stack()
             or C._len_torch_function_stack() or C._get_tracing_state() is not None
             or C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0):
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch.autograd.profiler._is_profiler_enabled):
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:

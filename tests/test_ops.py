@@ -180,3 +180,20 @@ def test_moe_batches_that_run_as_a_prompt(T, top_k, E, hidden, prompt):
     blk = SimpleNamespace(MAX_TOKENS=B.MAX_TOKENS, top_k=top_k, num_experts=E, hidden=hidden,
                           zeros_integral=True, rank=64)
     assert B._as_prompt(blk, T) is prompt
+
+
+@pytest.mark.gpu
+def test_profiler_sees_the_operator(gpu):
+    """With a profiler active the call goes through the operator, so that it is
+    recorded under its name."""
+    from glorcq_amd import kernels as K_
+
+    p = fmt.make_linear(2048, 256, bits=2, rank=16, M=3, seed=8)
+    t = {k: getattr(p, k).to(gpu) for k in ("x", "codes", "scales", "zeros", "U", "SV")}
+    assert K_._plain(*t.values())
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        assert not K_._plain(*t.values())
+        K_.packed_dequant_matmul_fused(t["x"], t["codes"], t["scales"], t["zeros"], 2, 128,
+                                       U=t["U"], SV=t["SV"])
+    assert K_._plain(*t.values())
+    assert "glorcq_hip::packed_dequant_matmul" in {e.key for e in prof.key_averages()}
