@@ -164,28 +164,34 @@ def _gemv_workspace_bytes(lib, items: int, M: int, K: int, N: int, rank: int) ->
     return n
 
 
-def _plain(*tensors) -> bool:
+# (looked up once: the check below is on the path of every fused linear)
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_tracing_state = torch._C._get_tracing_state
+_functorch_level = torch._C._functorch.peek_interpreter_stack
+_forward_ad, _profiler = torch.autograd.forward_ad, torch.autograd.profiler
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _plain(x, *rest) -> bool:
     """The operator dispatch would only call the eager function: plain GPU
     tensors and nothing that watches, transforms or differentiates the call
     (compile and trace, dispatch and function modes, functorch, forward-mode
-    levels, a profiler, a gradient to record).  The dispatch of a Python custom
-    operator costs about 7 us of host time, this check 0.5."""
-    C = torch._C
-    if (torch.compiler.is_compiling() or C._len_torch_dispatch_stack()
-            or C._len_torch_function_stack() or C._get_tracing_state() is not None
-            or C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0
-            or torch.autograd.profiler._is_profiler_enabled):
+    levels, a profiler, a gradient to record), nothing that the dispatch
+    resolves or refuses first (lazily negated tensors, names).  The dispatch of
+    a Python custom operator costs about 7 us of host time, this check 0.5."""
+    if (torch.compiler.is_compiling() or type(x) not in _PLAIN_TYPES or not x.is_cuda
+            or _dispatch_modes() or _function_modes()
+            or _tracing_state() is not None or _functorch_level() is not None
+            or _forward_ad._current_level >= 0 or _profiler._is_profiler_enabled
+            or x.has_names()):
         return False
     grad = torch.is_grad_enabled()
-    for t in tensors:
-        if t is not None and (type(t) not in _PLAIN_TYPES or not t.is_cuda
+    for t in (x, *rest):
+        if t is not None and (type(t) not in _PLAIN_TYPES or t.is_neg()
                               or (grad and t.requires_grad)):
             return False
     return True
-
-
-_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def packed_dequant_matmul_fused(x: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor,
@@ -202,7 +208,8 @@ def packed_dequant_matmul_fused(x: torch.Tensor, codes: torch.Tensor, scales: to
     graph break), called directly where the dispatch would add nothing
     (_plain); with `out` (a caller's buffer, e.g. under graph capture) the
     library is called directly.  Arguments as _packed_dequant_matmul_eager."""
-    if out is None and not _plain(x, codes, scales, zeros, U, SV, precomputed_xU, bias):
+    if out is None and not (type(bits) is int and type(groupsize) is int and
+                            _plain(x, codes, scales, zeros, U, SV, precomputed_xU, bias)):
         return torch.ops.glorcq_hip.packed_dequant_matmul(
             x, codes, scales, zeros, bits, groupsize, _sym_mode(sym), U, SV, precomputed_xU, bias)
     return _packed_dequant_matmul_eager(x, codes, scales, zeros, bits, groupsize, sym, U, SV,

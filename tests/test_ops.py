@@ -197,3 +197,25 @@ def test_profiler_sees_the_operator(gpu):
                                        U=t["U"], SV=t["SV"])
     assert K_._plain(*t.values())
     assert "glorcq_hip::packed_dequant_matmul" in {e.key for e in prof.key_averages()}
+
+
+@pytest.mark.gpu
+def test_what_the_dispatch_resolves_or_refuses_first(gpu):
+    """A lazily negated activation gives its own values' result, and names and
+    sizes that are not integers are refused, as by the operator."""
+    from glorcq_amd import kernels as K_
+
+    p = fmt.make_linear(2048, 256, bits=2, rank=16, M=3, seed=8)
+    t = {k: getattr(p, k).to(gpu) for k in ("x", "codes", "scales", "zeros", "U", "SV")}
+
+    def call(x, bits=2, group=128, **kw):
+        return K_.packed_dequant_matmul_fused(x, t["codes"], t["scales"], t["zeros"], bits, group,
+                                              U=t["U"], SV=kw.get("SV", t["SV"]))
+
+    neg = torch._neg_view(t["x"])  # as conj().imag is
+    assert neg.is_neg() and torch.equal(call(neg), call((-t["x"]).contiguous()))
+    assert torch.equal(call(t["x"], SV=torch._neg_view(t["SV"])), call(t["x"], SV=-t["SV"]))
+    for bad in (lambda: call(t["x"].rename("a", "b")), lambda: call(t["x"], bits=2.0),
+                lambda: call(t["x"], group=128.0)):
+        with pytest.raises(RuntimeError):
+            bad()
