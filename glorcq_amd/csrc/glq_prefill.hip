@@ -718,6 +718,7 @@ struct PfLowrank {
   int64_t u_cs;            // elements between clusters
   const int32_t* cluster[2];  // (E,) cluster of expert e per matrix (null: 0)
   const int32_t* uslot[2];    // cluster -> row of U[m] (a cross-layer pool), or null
+  int ncl[2], urows[2];       // clusters of matrix m, rows of U[m]: ids are clamped (0: not)
   const int32_t* tiles;    // tile list of the GEMM (null: dense)
   const int32_t* ntiles;
   int tile_rows;           // rows per tile of the list
@@ -764,7 +765,9 @@ __device__ __forceinline__ void pf_lowrank_body(const PfLowrank& L, int job, int
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     int c = (m < L.nmat && L.cluster[m]) ? L.cluster[m][e] : 0;
+    if (L.ncl[m] > 0) c = min(max(c, 0), L.ncl[m] - 1);
     if (m < L.nmat && L.uslot[m]) c = L.uslot[m][c];
+    if (L.urows[m] > 0) c = min(max(c, 0), L.urows[m] - 1);
     U[m] = m < L.nmat ? L.U[m] + (int64_t)c * L.u_cs : nullptr;
   }
   // A: instruction q of the wave loads rows 4 (4 wave + q) .. + 3
@@ -2071,8 +2074,11 @@ static int pf_moe_check(const glq_moe_params* p) {
   const bool lora = r > 0 && p->SV[0] != nullptr;
   if (lora) {
     GLQ_CHECK(r % 8 == 0 && r <= 128, "rank=%lld must be a multiple of 8, <= 128", (long long)r);
-    for (int s = 0; s < 3; ++s)
+    for (int s = 0; s < 3; ++s) {
       GLQ_CHECK(p->U[s] && p->cluster_of[s] && p->SV[s], "U, cluster_of and SV are needed with a rank");
+      GLQ_CHECK(p->u_rows[s] >= 0 && p->u_rows[s] < (1ll << 24) && p->n_clusters < (1ll << 24),
+                "u_rows or n_clusters out of range");
+    }
   }
   GLQ_CHECK(p->h && p->router_w && p->out, "null h, router_w or out");
   for (int s = 0; s < 3; ++s) {
@@ -2175,6 +2181,8 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
       L.U[m] = (const __half*)p->U[m];
       L.cluster[m] = p->cluster_of[m];
       L.uslot[m] = p->u_slot[m];
+      L.ncl[m] = (int)p->n_clusters;
+      L.urows[m] = (int)(p->u_rows[m] > 0 ? p->u_rows[m] : p->n_clusters);
     }
     L.u_cs = H * r;
     L.tiles = a.tiles;
@@ -2229,6 +2237,7 @@ extern "C" int glq_moe_prefill(const glq_moe_params* p, void* workspace, int64_t
     L.nmat = 1;
     L.U[0] = (const __half*)p->U[2];
     L.cluster[0] = p->cluster_of[2];
+    L.urows[0] = (int)(p->u_rows[2] > 0 ? p->u_rows[2] : p->n_clusters);
     L.u_cs = I * r;
     L.tiles = a.tiles;
     L.ntiles = a.ntiles;

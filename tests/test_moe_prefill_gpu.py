@@ -197,3 +197,31 @@ def test_large_decode_batches(gpu, T, E, top_k, kw):
         torch.cuda.synchronize()
         assert torch.equal(gout, out) and torch.equal(glog, logits)
         assert torch.equal(blk(h)[0], out)
+
+
+@pytest.mark.parametrize("T", [8, 20, 65])
+@pytest.mark.parametrize("pool", [False, True])
+def test_cluster_ids_are_clamped(gpu, T, pool):
+    """Cluster ids past the U pool read its last row (negative ones its first),
+    in a decode step, in a batch that runs as a prompt and in a prompt; also
+    through the rows of a cross-layer pool."""
+    p = lora_heavy(fmt.make_moe(H=512, E=6, inter=256, top_k=2, n_clusters=3, rank=16,
+                                shared_inter=0, B=T, seed=4))
+    ids = torch.tensor([0, 7, -2, 2, 1, 3])
+    outs = []
+    for cl in (ids, ids.clamp(0, 2)):
+        p.cluster_of = {proj: cl for proj in fmt.PROJS}
+        blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+        if pool:  # rows 4, 1, 2 of five hold the clusters; down's ids are rows
+            slot = torch.tensor([4, 1, 2], dtype=torch.int32, device=gpu)
+            for proj in fmt.PROJS:
+                U = blk.t[f"U_{proj}"]
+                big = torch.full((5, *U.shape[1:]), float("nan"), dtype=U.dtype, device=gpu)
+                big[slot.long()] = U
+                blk.t[f"U_{proj}"], blk.t[f"urows_{proj}"] = big, 5
+            blk.t["uslot_gate"] = blk.t["uslot_up"] = slot
+            blk.t["cluster_down"] = slot[ids.clamp(0, 2).to(gpu)].contiguous()
+        outs.append(blk(p.h.reshape(1, T, p.H).to(gpu))[0])
+    torch.cuda.synchronize()
+    assert not bool(outs[0].isnan().any()) and torch.equal(*outs)
+    check(p, outs[1].reshape(T, p.H).cpu(), blk(p.h.reshape(1, T, p.H).to(gpu))[1].cpu(), str(T))
