@@ -64,6 +64,7 @@ class TurboPrefillParams(ctypes.Structure):
         ("signs", _vp * 2), ("Pi", _vp * 2),
         *[(n, _vp * 3) for n in ("shared_codes", "shared_scales", "shared_zeros")],
         *[(n, _vp) for n in ("shared_y", "residual", "out", "router_logits")],
+        ("u_rows", _i64 * 3),
     ]
 
 

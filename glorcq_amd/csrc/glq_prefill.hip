@@ -2377,6 +2377,7 @@ static int tp_check(const glq_turbo_prefill_params* p) {
     if (p->rank > 0)
       GLQ_CHECK(p->U[i] && p->cluster_of[i] && p->SV[i] && al16(p->U[i]) && al16(p->SV[i]),
                 "U, cluster_of and SV (16-byte aligned) are needed with a rank");
+    GLQ_CHECK(p->u_rows[i] >= 0 && p->u_rows[i] < (1ll << 24), "u_rows out of range (proj %d)", i);
     if (SI > 0)
       GLQ_CHECK(p->shared_codes[i] && p->shared_scales[i] && p->shared_zeros[i] &&
                     al16(p->shared_codes[i]),
@@ -2488,6 +2489,7 @@ extern "C" int glq_turbo_moe_prefill(const glq_turbo_prefill_params* p, void* wo
     for (int m = 0; m < nmat; ++m) {
       L.U[m] = (const __half*)p->U[m0 + m];
       L.cluster[m] = p->cluster_of[m0 + m];
+      L.urows[m] = (int)p->u_rows[m0 + m];
     }
     L.u_cs = K * r;
     L.tiles = a.tiles;

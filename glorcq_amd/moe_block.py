@@ -819,6 +819,7 @@ def turbo_prefill(blk: GraphCompatibleMoeBlock, h: torch.Tensor, res: torch.Tens
             p.U[i] = t[f"U_{proj}"].data_ptr()
             p.cluster_of[i] = t[f"cluster_{proj}"].data_ptr()
             p.SV[i] = t[f"SV_{proj}"].data_ptr()
+            p.u_rows[i] = t[f"U_{proj}"].shape[0]
     for i, proj in enumerate(("gate", "down")):
         p.signs[i] = _lib.ptr(t[f"signs_{proj}"])
         p.Pi[i] = None if t[f"signs_{proj}"] is not None else _lib.ptr(t[f"Pi_{proj}_c"])

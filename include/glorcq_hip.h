@@ -539,9 +539,10 @@ int glq_turbo_moe_gemv(int64_t picks, int64_t x_div, const void* x_rot, int64_t 
  * 704-740, on TurboQuant layers; the decode step's routing and combine).
  * Projections in the order gate, up, down: codes (experts, N, K/16) words,
  * norms (experts, N), centroids (4,), SV (experts, N, rank), U (rows, K,
- * rank) at row cluster_of[expert].  Rotations [0] of gate and up's input,
- * [1] of down's: signs (fp32, a power-of-two width) or Pi (width, width)
- * fp16 rows, x_rot = fp16(x Pi^T).  The shared expert: 2- or 4-bit group-128
+ * rank) at row cluster_of[expert], clamped into [0, u_rows) (u_rows 0: as it
+ * is).  Rotations [0] of gate and up's input, [1] of down's: signs (fp32, a
+ * power-of-two width) or Pi (width, width) fp16 rows, x_rot = fp16(x Pi^T).
+ * The shared expert: 2- or 4-bit group-128
  * weights with integer zero-points (shared_inter > 0), or its output
  * shared_y (tokens, hidden), or none.  residual may be NULL.  hidden, inter
  * and shared_inter are multiples of 128, rank of 8 (<= 128; 0: none).
@@ -567,6 +568,7 @@ typedef struct glq_turbo_prefill_params {
   const void* residual;
   void* out;
   void* router_logits;
+  int64_t u_rows[3];
 } glq_turbo_prefill_params;
 
 int64_t glq_turbo_moe_prefill_workspace_bytes(const glq_turbo_prefill_params* p);

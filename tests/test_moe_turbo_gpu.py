@@ -322,3 +322,17 @@ def test_turbo_prompt_runs_the_shared_modules(gpu):
         load(m, p.shared[s])
     out, _ = run(blk, p, gpu)
     assert bar(out, O.moe_forward(p)) and not bar(out, first)
+
+
+@pytest.mark.parametrize("B", [8, 20])
+def test_turbo_cluster_ids_are_clamped(gpu, B):
+    """Cluster ids past U's rows read the last one (negative ones the first),
+    in a step and in a prompt."""
+    p = problem(B, 6)
+    ids = torch.arange(p.E) % 6 - 1  # -1 .. 4 of 4 clusters
+    outs = []
+    for cl in (ids, ids.clamp(0, 3)):
+        p.cluster_of = {proj: cl for proj in fmt.PROJS}
+        outs.append(run(GraphCompatibleMoeBlock.from_problem(p, gpu), p, gpu)[0])
+    assert torch.equal(*outs)
+    assert bar(outs[0], O.moe_forward(p))
