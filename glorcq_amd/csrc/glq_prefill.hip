@@ -2069,6 +2069,7 @@ static int pf_moe_check(const glq_moe_params* p) {
   const int64_t SI = p->shared_inter;
   GLQ_CHECK(SI >= 0 && SI % 128 == 0 && SI <= (1 << 17), "shared_inter=%lld must be a multiple of 128",
             (long long)SI);
+  GLQ_CHECK(T * SI < (1ll << 31), "tokens x shared_inter too large");  // 32-bit row offsets
   if (SI > 0) GLQ_CHECK(p->shared_bits == 2 || p->shared_bits == 4, "shared_bits must be 2 or 4");
   const int64_t r = p->rank;
   const bool lora = r > 0 && p->SV[0] != nullptr;

@@ -340,3 +340,24 @@ def test_tile_form_takes_no_weights_past_32_bit_offsets(lib):
     assert b"Pi" in lib.glq_last_error()
     q.inter = 1 << 15
     assert lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(q)) > 0
+
+
+def test_moe_prefill_refuses_rows_past_32_bit_offsets(lib):
+    """The shared expert's down launch reads its (tokens, shared_inter) input
+    through 32-bit byte offsets: 2^31 elements and more are refused."""
+    import ctypes
+
+    from glorcq_amd import _lib
+
+    q = _lib.MoeParams()
+    for k, v in dict(hidden=512, experts=4, inter=128, top_k=1, bits=2, shared_bits=4, group=128,
+                     h=1 << 12, router_w=1 << 12, out=1 << 12, shared_inter=1 << 15).items():
+        setattr(q, k, v)
+    for i in range(3):
+        for f in ("codes", "scales", "zeros", "shared_codes", "shared_scales", "shared_zeros"):
+            getattr(q, f)[i] = 1 << 12
+    q.tokens = (1 << 16) - 1
+    assert lib.glq_moe_prefill_workspace_bytes(ctypes.byref(q)) > 0
+    q.tokens = 1 << 16
+    assert lib.glq_moe_prefill_workspace_bytes(ctypes.byref(q)) == -1
+    assert b"shared_inter" in lib.glq_last_error()
