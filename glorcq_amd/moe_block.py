@@ -481,6 +481,8 @@ def _turbo_derived(t: dict) -> None:
     for proj in ("gate", "down"):
         Pi = t[f"Pi_{proj}"]
         t[f"Pi_{proj}_c"] = None if Pi is None else Pi.to(torch.float16).contiguous()
+    if t["Pi_gate_c"] is not None and t["Pi_gate_c"].data_ptr() % 16:  # 16-byte loads
+        t["Pi_gate_c"] = t["Pi_gate_c"].clone()
     # glq_turbo_moe_prefill's shared GEMMs take integer zero-points; checked
     # once here, for weights of the block's own (a shared expert of modules runs
     # as its modules, whose weights may be loaded again)
@@ -785,10 +787,11 @@ def turbo_step(blk: GraphCompatibleMoeBlock, h: torch.Tensor, res: torch.Tensor 
 
 def _turbo_prefill_ok(blk: GraphCompatibleMoeBlock, T: int) -> bool:
     """More than one step's tokens go through glq_turbo_moe_prefill when it
-    takes the block: gate and up rotated alike, widths of whole 128-code
-    groups, a rank that is a multiple of 8 (at most 128)."""
+    takes the block and the prompt: gate and up rotated alike, widths of whole
+    128-code groups, a rank that is a multiple of 8 (at most 128), its limits on
+    tokens and offsets.  Others run as steps."""
     t = blk.t
-    return (T > TURBO_MAX_TOKENS and not os.environ.get("GLQ_TURBO_SEQ") and t["same_rot_gu"]
+    return (TURBO_MAX_TOKENS < T <= 1 << 20 and not os.environ.get("GLQ_TURBO_SEQ") and t["same_rot_gu"]
             and blk.hidden % 128 == 0 and blk.hidden <= 4096  # the decode router's limit
             and blk.inter % 128 == 0 and blk.num_experts <= 256
             and blk.top_k <= 16 and blk.rank % 8 == 0 and blk.rank <= 128

@@ -361,3 +361,34 @@ def test_moe_prefill_refuses_rows_past_32_bit_offsets(lib):
     q.tokens = 1 << 16
     assert lib.glq_moe_prefill_workspace_bytes(ctypes.byref(q)) == -1
     assert b"shared_inter" in lib.glq_last_error()
+
+
+@pytest.mark.parametrize("T,kw,prompt", [
+    (16, {}, False), (17, {}, True),
+    (1 << 20, {}, True), ((1 << 20) + 1, {}, False),  # more than the entry point takes: steps
+    (100, dict(inter=200), False), (100, dict(rank=136), False), (100, dict(hidden=8192), False),
+    (1 << 20, dict(top_k=16), False),  # 32-bit row offsets
+])
+def test_turbo_prompts_that_run_as_one(lib, T, kw, prompt):
+    """What the rule sends to glq_turbo_moe_prefill the entry point takes; the
+    rest runs as 16-token steps."""
+    import ctypes
+    from types import SimpleNamespace
+
+    from glorcq_amd import _lib
+    from glorcq_amd.moe_block import _turbo_prefill_ok
+
+    size = {**dict(hidden=256, inter=128, num_experts=16, top_k=2, rank=16, shared_inter=0), **kw}
+    blk = SimpleNamespace(t={"same_rot_gu": True}, **size)
+    assert _turbo_prefill_ok(blk, T) is prompt
+    if not prompt:
+        return
+    q = _lib.TurboPrefillParams()
+    q.tokens, q.hidden, q.experts, q.inter = T, size["hidden"], 16, size["inter"]
+    q.top_k, q.rank = size["top_k"], size["rank"]
+    q.h = q.router_w = q.out = 1 << 12
+    for i in range(3):
+        for f in ("codes", "norms", "centroids", "U", "cluster_of", "SV"):
+            getattr(q, f)[i] = 1 << 12
+    q.signs[0], q.Pi[1] = 1 << 12, 1 << 12
+    assert lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(q)) > 0

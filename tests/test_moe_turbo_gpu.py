@@ -336,3 +336,19 @@ def test_turbo_cluster_ids_are_clamped(gpu, B):
         outs.append(run(GraphCompatibleMoeBlock.from_problem(p, gpu), p, gpu)[0])
     assert torch.equal(*outs)
     assert bar(outs[0], O.moe_forward(p))
+
+
+def test_turbo_prompt_takes_an_unaligned_rotation(gpu):
+    """gate and up's Pi may lie anywhere (the steps multiply by it through the
+    library); the prompt's 16-byte loads read an aligned copy."""
+    p = fmt.make_turbo_moe(H=256, E=6, inter=256, top_k=2, n_clusters=3, rank=16, B=20, seed=3,
+                           rot_gate_up="qr", rot_down="qr")
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+    want, _ = run(blk, p, gpu)
+    Pi = blk.t["Pi_gate"]
+    off = torch.cat([Pi.flatten()[:1], Pi.flatten()])[1:].reshape(Pi.shape)
+    assert off.is_contiguous() and off.data_ptr() % 16
+    blk.t["Pi_gate"] = blk.t["Pi_up"] = off
+    moe_block._turbo_derived(blk.t)
+    got, _ = run(blk, p, gpu)
+    assert torch.equal(got, want)
