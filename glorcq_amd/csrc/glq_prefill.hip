@@ -383,7 +383,8 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
   const int n0 = tn * WGR;
   const int g0 = sp * g.gps, g1 = min(g0 + g.gps, g.G);
 
-  // ---- per-lane load addresses (offsets in elements; uniform bases) ----
+  // ---- per-lane load addresses: offsets in elements from uniform bases (the
+  // workgroup's first weight row: weights of 4 GB and more come here) ----
   // A: this lane's XI slot rows
   int aoff[XI];
 #pragma unroll
@@ -398,9 +399,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
   const __half* zb[NMAT];
 #pragma unroll
   for (int m = 0; m < NMAT; ++m) {
-    cb[m] = g.codes[m] + e * g.codes_es;
-    sb[m] = g.scales[m] + e * g.sz_es;
-    zb[m] = SYM ? sb[m] : g.zeros[m] + e * g.sz_es;
+    cb[m] = g.codes[m] + e * g.codes_es + (int64_t)n0 * g.kw;
+    sb[m] = g.scales[m] + e * g.sz_es + (int64_t)n0 * g.G;
+    zb[m] = SYM ? sb[m] : g.zeros[m] + e * g.sz_es + (int64_t)n0 * g.G;
   }
   // codes: instruction q covers bytes q*1024 + 16*lane of the wave's region
   // (lanes past the wave's code bytes re-load its first ones into the padding)
@@ -411,7 +412,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
     const int rt = o / (16 * SL::CB), row = (o % (16 * SL::CB)) / SL::CB;
     const int piece = (o % SL::CB) / 16;
     const int n = min(pf_row<RT, MODE>(n0, wave, rt, row), g.N - 1);
-    coff[q] = n * g.kw + 4 * piece;
+    coff[q] = (n - n0) * g.kw + 4 * piece;
     cmat[q] = MODE == kPfGateUp ? rt / (RT / 2) : 0;
   }
   // scales / zero-points: lane -> (row tile lane/16, row lane%16)
@@ -419,7 +420,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
   {
     const int rt = min(lane >> 4, RT - 1);
     const int n = min(pf_row<RT, MODE>(n0, wave, rt, lane & 15), g.N - 1);
-    soff = n * g.G;
+    soff = (n - n0) * g.G;
     smat = MODE == kPfGateUp ? rt / (RT / 2) : 0;
   }
   auto issue = [&](int grp, unsigned char* slot) {

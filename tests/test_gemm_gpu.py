@@ -377,3 +377,27 @@ def test_dense_tile_form(gpu, M, K, N, bits, rank, sym):
     if rank:
         y2 = call(SV=d["SV"], precomputed_xU=a)
         assert bool(((y2.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+def test_codes_past_8_gb(gpu):
+    """Rows of a weight whose codes lie past 2^31 words (4-bit, 16384 x 2^20 and
+    512 more: 8.6 GB) against the same rows as a weight of their own: fp16
+    roundings of equal fp32 sums (another tile may sum in another order)."""
+    K, n, N, M = 16384, 512, (1 << 20) + 512, 17
+    g = torch.Generator(device=gpu).manual_seed(3)
+    codes = torch.zeros(N, K // 8, dtype=torch.int32, device=gpu)
+    scales = torch.ones(N, K // 128, dtype=torch.float16, device=gpu)
+    zeros = torch.full_like(scales, 8.0)
+    codes[-n:] = torch.randint(-(2**31), 2**31, (n, K // 8), generator=g, device=gpu,
+                               dtype=torch.int64).int()
+    scales[-n:] = (torch.rand(n, K // 128, generator=g, device=gpu) * 0.02).half()
+    x = torch.randn(M, K, generator=g, device=gpu).half()
+    y = K_.packed_dequant_matmul_fused(x, codes, scales, zeros, 4, 128)[:, -n:].clone()
+    own = [t[-n:].clone() for t in (codes, scales, zeros)]
+    del codes, scales, zeros
+    torch.cuda.empty_cache()
+    ref = K_.packed_dequant_matmul_fused(x, *own, 4, 128)
+    err = (y.float() - ref.float()).abs()
+    assert bool((err <= 1e-3 + 1e-3 * ref.float().abs()).all()), float(err.max())
+    assert float(ref.float().abs().max()) > 1.0
