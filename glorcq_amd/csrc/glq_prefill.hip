@@ -1930,9 +1930,11 @@ static PfMoePlan pf_moe_plan(int64_t T, int64_t H, int64_t E, int64_t I, int64_t
   // Token tile by the mean tokens an expert gets: 128 tokens where most experts
   // fill one such tile and overflow a 64-token one, 64 above, 32 where most
   // of a 64-token tile would be empty.  Whole blocks at 32 / 64 / 128: 19
-  // tokens an expert 293 / 336 / 458 us, 47: 382 / 363 / 421, 50: 361 / 385 /
-  // 393, 94: 594 / 577 / 566, 128: 716 / 649 / 671, 250: 1183 / 1036 / 1053.
-  P.tm = avg < 46 ? 32 : (avg >= 80 && avg < 112 ? 128 : 64);
+  // tokens an expert 293 / 336 / 458 us, 47: 382 / 363 / 421.  128 against 64
+  // over five blocks (experts, top-k: 60, 4; 128, 8; 8, 2; 32, 4; 64, 6): at 80
+  // tokens 0.978 to 0.995 of the time, 88 0.97 to 1.01, 96 0.984 to 1.003;
+  // 100 0.97 to 1.04, 104 0.99 to 1.02, 112 1.00 to 1.03, 128 0.99 to 1.08.
+  P.tm = avg < 46 ? 32 : (avg >= 80 && avg < 98 ? 128 : 64);
   if (const char* e = getenv("GLQ_PF_MOE_TM")) {
     const int v = atoi(e);
     P.tm = v >= 128 ? 128 : (v >= 64 ? 64 : 32);

@@ -392,3 +392,32 @@ def test_turbo_prompts_that_run_as_one(lib, T, kw, prompt):
             getattr(q, f)[i] = 1 << 12
     q.signs[0], q.Pi[1] = 1 << 12, 1 << 12
     assert lib.glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(q)) > 0
+
+
+@pytest.mark.parametrize("mean,tile", [(20, 32), (45, 32), (46, 64), (79, 64), (80, 128),
+                                       (97, 128), (98, 64), (200, 64)])
+def test_moe_prefill_token_tile(lib, monkeypatch, mean, tile):
+    """The routed token tile by the mean tokens an expert gets: 32 below 46,
+    128 from 80 to 97, else 64 (by the workspace's size, in which two of the
+    tiles may agree)."""
+    import ctypes
+
+    from glorcq_amd import _lib
+
+    q = _lib.MoeParams()
+    for k, v in dict(tokens=32 * mean, hidden=512, experts=256, inter=512, top_k=8, bits=2,
+                     group=128, h=1 << 12, router_w=1 << 12, out=1 << 12).items():
+        setattr(q, k, v)
+    for i in range(3):
+        for f in ("codes", "scales", "zeros"):
+            getattr(q, f)[i] = 1 << 12
+
+    def size():
+        return lib.glq_moe_prefill_workspace_bytes(ctypes.byref(q))
+
+    monkeypatch.delenv("GLQ_PF_MOE_TM", raising=False)
+    mine, forced = size(), {}
+    for tm in (32, 64, 128):
+        monkeypatch.setenv("GLQ_PF_MOE_TM", str(tm))
+        forced[tm] = size()
+    assert mine == forced[tile] and len(set(forced.values())) >= 2
