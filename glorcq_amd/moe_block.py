@@ -89,7 +89,6 @@ class GraphCompatibleMoeBlock(nn.Module):
         zkeys += [f"szeros_{p}" for p in PROJS if f"szeros_{p}" in stacked]
         self.zeros_integral = self.kind == "gptq" and all(
             bool(torch.equal(stacked[k], stacked[k].round())) for k in zkeys)
-        self._step_max = self._step_limit() if self.kind == "gptq" else 0
 
     # ---- construction ----
     @staticmethod
@@ -234,7 +233,6 @@ class GraphCompatibleMoeBlock(nn.Module):
                 t["cluster_down"] = slot[t["cluster_down"].long()].contiguous()
             else:
                 t[f"uslot_{proj}"] = slot
-        self._step_max = self._step_limit()
 
     # ---- the step ----
     def _op_args(self):
@@ -257,27 +255,6 @@ class GraphCompatibleMoeBlock(nn.Module):
 
     MAX_TOKENS = 64  # tokens per decode step (glq_moe_decode)
 
-    def _step_limit(self) -> int:
-        """The largest batch of 17 to MAX_TOKENS tokens that the decode step
-        takes (its limits on picks, widths, LDS and alignment), or 16: a larger
-        one is the step's to refuse, also where a prompt could run it."""
-        if not _lib.available():
-            return self.MAX_TOKENS
-        lib, rw = _lib.load(), self.t["router_w"]
-        P = _moe_params(rw, rw, self.t["shared_gate_w"], *self._op_args(), None, rw, None,
-                        self.inter, self.top_k, self.norm_topk_prob, self.rank, self.n_clusters,
-                        self.bits, self.shared_bits, self.shared_inter)
-        lo, hi = 16, self.MAX_TOKENS  # what is taken and what might be: every limit grows with T
-        mid = hi
-        while lo < hi:
-            P.tokens = mid
-            if lib.glq_moe_workspace_bytes(ctypes.byref(P)) >= 0:
-                lo = mid
-            else:
-                hi = mid - 1
-            mid = (lo + hi + 1) // 2
-        return lo
-
     def _as_prompt(self, T: int) -> bool:
         """T tokens run as one glq_moe_prefill: more than a decode step takes,
         and from 17 tokens where its grouped GEMMs (an expert's codes decoded
@@ -286,8 +263,8 @@ class GraphCompatibleMoeBlock(nn.Module):
         or from two picks an expert (the measured crossing).  Step against
         prompt, us, graph replays: 60 experts top-4, 20 tokens 124 / 126, 32
         150 / 130, 64 241 / 141; 128 experts top-8, 20 120 / 142, 32 154 / 152,
-        64 299 / 155; 8 experts top-2, 17 346 / 239, 64 873 / 271.  (Batches
-        past _step_max stay the step's to refuse.)"""
+        64 299 / 155; 8 experts top-2, 17 346 / 239, 64 873 / 271.  What the
+        step refuses (512 picks, hidden in 256s) it still gets to refuse."""
         if T > self.MAX_TOKENS:
             return True
         return (T > 16 and (T > 32 or T * self.top_k >= 2 * self.num_experts)
@@ -333,8 +310,7 @@ class GraphCompatibleMoeBlock(nn.Module):
             out = out.reshape(shape)
             return (out, lg) if self.return_router_logits else out
         codes, scales, zeros, U, cl, SV, u_slot, u_rows, sc, ss, sz = self._op_args()
-        n = h.shape[0]
-        if not self._as_prompt(n) or self._step_max < n <= self.MAX_TOKENS:
+        if not self._as_prompt(h.shape[0]):
             out, logits = torch.ops.glorcq_hip.moe_decode(
                 h, t["router_w"], t["shared_gate_w"], codes, scales, zeros, U, cl, SV, u_slot,
                 u_rows, sc, ss, sz, res, self.inter, self.top_k, self.norm_topk_prob, self.rank,

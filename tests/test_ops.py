@@ -219,36 +219,3 @@ def test_what_the_dispatch_resolves_or_refuses_first(gpu):
                 lambda: call(t["x"], group=128.0)):
         with pytest.raises(RuntimeError):
             bad()
-
-
-@pytest.mark.parametrize("kw,limit", [
-    (dict(H=512, top_k=2), 64),
-    (dict(H=512, top_k=12, E=12), 42),   # 512 picks
-    (dict(H=384, top_k=2), 16),          # hidden in 256s
-    (dict(H=5376, top_k=2), 16),         # the router's LDS budget
-    (dict(H=512, top_k=2, unaligned="scodes_down"), 16),
-])
-def test_moe_step_limit(kw, limit):
-    """A block knows the largest batch that the decode step takes, whatever it
-    is refused for."""
-    kw = dict(kw)
-    unaligned = kw.pop("unaligned", None)
-    p = fmt.make_moe(**{**dict(E=4, inter=128, n_clusters=2, rank=16, shared_inter=128), **kw})
-    blk = GraphCompatibleMoeBlock.from_problem(p, "cpu")
-    if unaligned:
-        c = blk.t[unaligned]
-        blk.t[unaligned] = torch.cat([c.flatten()[:1], c.flatten()])[1:].reshape(c.shape)
-    assert blk._step_limit() == limit
-
-
-@pytest.mark.gpu
-def test_moe_batches_past_the_step_limit_are_refused(gpu):
-    """Batches of 17 to 64 tokens that a prompt could run and the step refuses
-    (a hidden width past its LDS budget) are refused; a prompt of 65 runs."""
-    p = fmt.make_moe(H=5376, E=4, inter=128, top_k=2, n_clusters=2, rank=16, shared_inter=0, B=65)
-    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
-    h = p.h.reshape(1, 65, p.H).to(gpu)
-    for T in (16, 17, 40, 64):
-        with pytest.raises(RuntimeError, match="LDS budget"):
-            blk(h[:, :T])
-    assert blk(h)[0].shape == h.shape
