@@ -256,27 +256,49 @@ class GraphCompatibleMoeBlock(nn.Module):
     MAX_TOKENS = 64  # tokens per decode step (glq_moe_decode)
 
     def _as_prompt(self, T: int) -> bool:
-        """T tokens run as one glq_moe_prefill: more than a decode step takes,
-        and from 17 tokens where its grouped GEMMs (an expert's codes decoded
-        once for its tokens, the shared expert in the routed launches) beat
-        consecutive 16-token steps or the many-token step -- past 32 tokens,
-        or from two picks an expert (the measured crossing).  Step against
-        prompt, us, graph replays: 60 experts top-4, 20 tokens 124 / 126, 32
-        150 / 130, 64 241 / 141; 128 experts top-8, 20 120 / 142, 32 154 / 152,
-        64 299 / 155; 8 experts top-2, 17 346 / 239, 64 873 / 271.  What the
-        step refuses (512 picks, hidden in 256s) it still gets to refuse."""
+        """T tokens may run as one glq_moe_prefill: more than a decode step
+        takes, and from 17 tokens where its grouped GEMMs (an expert's codes
+        decoded once for its tokens, the shared expert in the routed launches)
+        can beat consecutive 16-token steps or the many-token step -- past 32
+        tokens, or from two picks an expert (the measured crossing; whether
+        they do is _prompt_pays').  Step against prompt, us, graph replays: 60
+        experts top-4, 20 tokens 124 / 126, 32 150 / 130, 64 241 / 141; 128
+        experts top-8, 20 120 / 142, 32 154 / 152, 64 299 / 155; 8 experts top-2,
+        17 346 / 239, 64 873 / 271.  More than 512 picks and hidden widths not of
+        256s, which the step refuses, are left to it."""
         if T > self.MAX_TOKENS:
             return True
         return (T > 16 and (T > 32 or T * self.top_k >= 2 * self.num_experts)
                 and T * self.top_k <= 512 and self.hidden % 256 == 0
                 and self.zeros_integral and self.rank % 8 == 0 and self.rank <= 128)
 
+    def _prompt_pays(self, T: int) -> bool:
+        """A batch that may run as a prompt is the faster for it: a prompt's
+        eight launches cost more than a step's three to five, and 20 us again
+        where the shared expert needs launches of its own (4-bit experts, 2-bit
+        shared weights); it gains on the picks' products (an estimate in us,
+        linear in their number and size, fitted to 1400 measured pairs: hidden
+        512 to 4096, inter 512 to 14336, 2 to 128 experts, 17 to 48 tokens).
+        Step against prompt, us: 2-bit 2048 x 768, 4 experts top-1, 17 tokens
+        44 / 58; 4-bit 1024 x 1024 and shared 2048, 16 experts top-2, 17 58 / 73,
+        20 of 2-bit 70 / 56; 4-bit 512 x 512 and shared 1024, 8 experts top-4, 48
+        56 / 69.  The estimate's choice is 0.5 % off the better of the two in the
+        mean, and in 1 % of the pairs more than 3 % slower than the step (17 %
+        without it, up to 1.8 x)."""
+        picks, H, I, S = T * self.top_k, self.hidden, self.inter, self.shared_inter
+        gain = 88e-9 * picks * H * I + 0.12 * picks + 2e-6 * S * H
+        apart = S > 0 and not (self.bits == 2 and self.shared_bits == 4)
+        if T > 32:  # (the many-token step also reads every code for few tokens)
+            gain += 0.5e-6 * self.num_experts * H * I * self.bits / 8
+            return gain > (30 if apart else 9)
+        return gain > (31 if apart else 13)
+
     def forward(self, hidden_states: torch.Tensor, residual: torch.Tensor | None = None):
         """(final (b, s, H) fp16, router_logits (b*s, E) fp16), as the
         reference's forward (moe_block.py:381-436); final alone when
         return_router_logits is False.  Up to 16 tokens run as one decode step
         (glorcq_hip::moe_decode); a prefill, and the larger batches that
-        _as_prompt names, through glorcq_hip::moe_prefill.
+        _as_prompt and _prompt_pays name, through glorcq_hip::moe_prefill.
         residual (the shape of hidden_states, fp16): final becomes
         fp16(residual + fp16(block output)), the decoder layer's residual add,
         inside the step's last launch."""
@@ -310,7 +332,8 @@ class GraphCompatibleMoeBlock(nn.Module):
             out = out.reshape(shape)
             return (out, lg) if self.return_router_logits else out
         codes, scales, zeros, U, cl, SV, u_slot, u_rows, sc, ss, sz = self._op_args()
-        if not self._as_prompt(h.shape[0]):
+        n = h.shape[0]
+        if not self._as_prompt(n) or (n <= self.MAX_TOKENS and not self._prompt_pays(n)):
             out, logits = torch.ops.glorcq_hip.moe_decode(
                 h, t["router_w"], t["shared_gate_w"], codes, scales, zeros, U, cl, SV, u_slot,
                 u_rows, sc, ss, sz, res, self.inter, self.top_k, self.norm_topk_prob, self.rank,

@@ -151,6 +151,7 @@ def test_moe_batch_graphs_of_one_stream_replay_on_two(gpu, monkeypatch):
     blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
     hs = [p.h[:T].reshape(1, T, p.H).to(gpu) for T in (64, 20)]
     assert all(blk._as_prompt(h.shape[1]) for h in hs)
+    blk._prompt_pays = lambda T: True
     seen = _recorded(monkeypatch, "glq_moe_prefill", 1)
     _two_graphs(gpu, seen, [lambda h=h: blk(h)[0] for h in hs])
 

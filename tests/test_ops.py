@@ -219,3 +219,25 @@ def test_what_the_dispatch_resolves_or_refuses_first(gpu):
                 lambda: call(t["x"], group=128.0)):
         with pytest.raises(RuntimeError):
             bad()
+
+
+@pytest.mark.parametrize("block,T,pays", [
+    # hidden, inter, experts, top_k, shared inter, bits, shared bits: step / prompt us
+    ((2048, 1408, 60, 4, 5632, 2, 4), 32, True),    # 139 / 116
+    ((2048, 768, 128, 8, 0, 2, 4), 32, True),       # 138 / 134
+    ((4096, 14336, 8, 2, 0, 2, 4), 17, True),       # 437 / 240
+    ((2048, 512, 256, 1, 0, 2, 4), 33, True),       # 195 / 96
+    ((2048, 768, 4, 1, 0, 2, 4), 17, False),        # 44 / 58
+    ((2048, 768, 2, 1, 1536, 4, 4), 17, False),     # 45 / 82
+    ((2048, 768, 2, 1, 1536, 4, 4), 48, False),     # 72 / 94
+    ((1024, 1024, 16, 2, 2048, 4, 4), 17, False),   # 58 / 73
+    ((512, 512, 8, 2, 512, 2, 4), 20, False),       # 36 / 44
+])
+def test_moe_batches_that_a_prompt_serves_faster(block, T, pays):
+    from types import SimpleNamespace
+
+    from glorcq_amd.moe_block import GraphCompatibleMoeBlock as B
+    H, inter, E, k, S, bits, sbits = block
+    blk = SimpleNamespace(hidden=H, inter=inter, num_experts=E, top_k=k, shared_inter=S,
+                          bits=bits, shared_bits=sbits)
+    assert B._prompt_pays(blk, T) is pays
