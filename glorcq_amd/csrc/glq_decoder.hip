@@ -332,9 +332,8 @@ __global__ __launch_bounds__(kDecThreads) void qk_norm_rope_kernel(QkArgs a) {
 //  * A wave takes 32-position blocks w, w + 4, ... of its workgroup's range
 //    with the next block's 16 KB in flight; online softmax a block.
 //  * The L positions are split evenly on the device over at most nsplit
-//    workgroups a group (whole 128-position steps), so every L uses them all;
-//    the ones past L leave at once and are not counted.  nsplit gives about
-//    two workgroups a CU (the kernel's occupancy): one round of them.
+//    workgroups a group (whole 128-position steps); the ones past L leave at
+//    once and are not counted (attention_split has nsplit).
 // The last workgroup of (b, g) to arrive (an arrival counter, data handed
 // over coherently) merges the splits in order -- M = max m_s, out = sum o_s
 // e^(m_s - M) / sum l_s e^(m_s - M) -- and zeroes the counter for the next
@@ -342,8 +341,7 @@ __global__ __launch_bounds__(kDecThreads) void qk_norm_rope_kernel(QkArgs a) {
 //
 // 16 sequences x 4000 positions, 32 / 4 heads (131 MB): with 128 positions a
 // workgroup staged in LDS and each head's scores and sums read from there,
-// 85 us (1.5 TB/s); this form 38 us (3.4 TB/s), and 4.8 TB/s at 16 x 8000,
-// 64 / 8 heads (108 us).
+// 85 us (1.5 TB/s); this form 30 us (4.4 TB/s).
 // ---------------------------------------------------------------------------
 constexpr int kAttnChunk = 128;   // positions of a workgroup's step
 constexpr int kAttnMaxRep = 8;
@@ -406,7 +404,7 @@ __global__ __launch_bounds__(kDecThreads, 2) void decode_attention_kernel(AttnAr
   extern __shared__ __align__(16) unsigned char smem[];
   float* obuf = (float*)smem + kAttnWts;  // [wave][head][m, l, o[128]]
   int* flag = (int*)(obuf + kAttnOut);
-  const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
+  const int g = blockIdx.x, b = blockIdx.y, split = blockIdx.z, tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rep = a.Hq / a.Hk;
   const int L = min(max(*a.len, 1), a.max_len);
@@ -824,6 +822,19 @@ extern "C" int glq_decode_attention_xu(const void* q, const void* k_cache, const
                           stream);
 }
 
+// Position splits of `groups` KV groups over `steps` 128-position steps: one
+// workgroup a CU, since a CU's second one shares its rate and brings another
+// partial to merge, and a launch a little past 256 of them waits for those few.
+// From 129 to 170 groups one split would leave CUs idle and three fill both
+// places of each.  us at one / two workgroups a CU: 16 groups x 2100 positions
+// 17.3 / 22.0, 64 x 4000 30.0 / 34.9, 8 x 8000 23.7 / 43.3, 192 x 4000 69.6 /
+// 88.0, 256 x 1500 35.6 / 43.8; 160 x 4000 one split 77.3, three 67.1.
+static int attention_split(int64_t groups, int64_t steps) {
+  int64_t n = std::max<int64_t>(1, 256 / groups);
+  if (n == 1 && groups < 171 && groups > 128) n = 3;
+  return (int)std::min({steps, (int64_t)glq::kAttnMaxSplit, n});
+}
+
 static int attention_launch(const void* q, const void* k_cache, const void* v_cache,
                             int64_t tokens, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
                             int64_t max_len, const int32_t* len, float scale, int64_t* advance,
@@ -852,11 +863,9 @@ static int attention_launch(const void* q, const void* k_cache, const void* v_ca
   a.q = (const __half*)q; a.k_cache = (const __half*)k_cache; a.v_cache = (const __half*)v_cache;
   a.len = len; a.advance = advance; a.out = (__half*)out;
   a.B = (int)tokens; a.Hq = (int)q_heads; a.Hk = (int)kv_heads; a.max_len = (int)max_len;
-  // about two workgroups a CU, whole steps, a bounded merge (the workspace
-  // holds a partial for every step of the cache)
+  // (the workspace holds a partial for every step of the cache)
   const int64_t steps = (max_len + kAttnChunk - 1) / kAttnChunk;
-  a.nsplit = (int)std::max<int64_t>(
-      1, std::min({steps, (int64_t)kAttnMaxSplit, 512 / (tokens * kv_heads)}));
+  a.nsplit = attention_split(tokens * kv_heads, steps);
   a.scale = scale;
   a.part = (float*)workspace;
   a.count = (unsigned*)((char*)workspace +
@@ -865,7 +874,9 @@ static int attention_launch(const void* q, const void* k_cache, const void* v_ca
   a.xpart = parts;
   a.rank = (int)rank;
   a.rpad = (int)align_up(rank, 32);
-  const dim3 grid((unsigned)a.nsplit, (unsigned)kv_heads, (unsigned)tokens);
+  // splits last: the ones past the length are the grid's end, so that the others
+  // spread evenly over the XCDs
+  const dim3 grid((unsigned)kv_heads, (unsigned)tokens, (unsigned)a.nsplit);
   const bool few = q_heads / kv_heads <= 4;
   auto kern = U ? (few ? decode_attention_kernel<true, 4> : decode_attention_kernel<true, 8>)
                 : (few ? decode_attention_kernel<false, 4> : decode_attention_kernel<false, 8>);

@@ -305,9 +305,11 @@ def test_fused_layers_match_framework_layers(gpu, monkeypatch, B, producer):
 
 @pytest.mark.parametrize("B,Hq,Hk,L,maxlen", [
     (130, 32, 4, 300, 320),   # one workgroup a group: three steps, the last ragged
-    (64, 32, 4, 257, 600),    # two splits of two steps, the second of one position
+    (32, 32, 4, 257, 600),    # two splits of two steps, the second of one position
+    (20, 64, 8, 700, 720),    # 160 groups: three splits of two steps
+    (32, 64, 8, 300, 600),    # 256 groups: one split each
     (8, 16, 4, 1000, 1032),   # 4 heads a group, one step a split
-    (16, 64, 8, 1153, 2000),  # 4 splits of three steps, one position over
+    (8, 64, 8, 1153, 2000),   # 4 splits of three steps, one position over
     (2, 6, 1, 127, 9000),     # one split of a long cache
 ])
 def test_decode_attention_splits(gpu, B, Hq, Hk, L, maxlen):
