@@ -284,8 +284,12 @@ class GraphCompatibleMoeBlock(nn.Module):
         20 of 2-bit 70 / 56; 4-bit 512 x 512 and shared 1024, 8 experts top-4, 48
         56 / 69.  The estimate's choice is 0.5 % off the better of the two in the
         mean, and in 1 % of the pairs more than 3 % slower than the step (17 %
-        without it, up to 1.8 x)."""
+        without it, up to 1.8 x).  Past 2048 columns, where the step nears its
+        LDS limits and refuses some blocks, a prompt is never more than 8 %
+        slower and always taken."""
         picks, H, I, S = T * self.top_k, self.hidden, self.inter, self.shared_inter
+        if H > 2048:
+            return True
         gain = 88e-9 * picks * H * I + 0.12 * picks + 2e-6 * S * H
         apart = S > 0 and not (self.bits == 2 and self.shared_bits == 4)
         if T > 32:  # (the many-token step also reads every code for few tokens)

@@ -232,6 +232,7 @@ def test_what_the_dispatch_resolves_or_refuses_first(gpu):
     ((2048, 768, 2, 1, 1536, 4, 4), 48, False),     # 72 / 94
     ((1024, 1024, 16, 2, 2048, 4, 4), 17, False),   # 58 / 73
     ((512, 512, 8, 2, 512, 2, 4), 20, False),       # 36 / 44
+    ((5376, 128, 4, 2, 0, 2, 4), 17, True),         # the step refuses it (LDS)
 ])
 def test_moe_batches_that_a_prompt_serves_faster(block, T, pays):
     from types import SimpleNamespace
@@ -241,3 +242,18 @@ def test_moe_batches_that_a_prompt_serves_faster(block, T, pays):
     blk = SimpleNamespace(hidden=H, inter=inter, num_experts=E, top_k=k, shared_inter=S,
                           bits=bits, shared_bits=sbits)
     assert B._prompt_pays(blk, T) is pays
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,inter,S", [(5376, 128, 0), (4096, 256, 256), (2048, 128, 128)])
+def test_moe_batches_of_wide_blocks_run(gpu, H, inter, S):
+    """Batches of 17 to 64 tokens run whether or not the step takes the block's
+    width."""
+    p = fmt.make_moe(H=H, E=4, inter=inter, top_k=2, n_clusters=2, rank=16, shared_inter=S, B=65)
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+    h = p.h.reshape(1, 65, p.H).to(gpu)
+    ref = blk(h)[0]
+    for T in (17, 33, 64):
+        # (fp16 roundings of x U, the SwiGLU product and the output, sums in another order)
+        err = (blk(h[:, :T])[0].float() - ref[:, :T].float()).abs()
+        assert bool((err <= 2e-3 + 1e-2 * ref[:, :T].float().abs()).all()), float(err.max())
