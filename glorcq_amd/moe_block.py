@@ -794,7 +794,7 @@ def _turbo_prefill_ok(blk: GraphCompatibleMoeBlock, T: int) -> bool:
     128-code groups, a rank that is a multiple of 8 (at most 128), its limits on
     tokens and offsets.  Others run as steps."""
     t = blk.t
-    return (TURBO_MAX_TOKENS < T <= 1 << 20 and not os.environ.get("GLQ_TURBO_SEQ") and t["same_rot_gu"]
+    return (TURBO_MAX_TOKENS < T <= 1 << 20 and t["same_rot_gu"]
             and blk.hidden % 128 == 0 and blk.hidden <= 4096  # the decode router's limit
             and blk.inter % 128 == 0 and blk.num_experts <= 256
             and blk.top_k <= 16 and blk.rank % 8 == 0 and blk.rank <= 128
