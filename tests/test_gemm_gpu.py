@@ -334,18 +334,23 @@ def test_one_launch_xu(gpu, monkeypatch, M, K, N, bits):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,K,N,bits,rank,sym", [
-    (150, 14336, 520, 2, 64, False),    # 32-token tiles, a 22-row last tile, 8 rows past 2 blocks
-    (1025, 1408, 2048, 2, 40, False),   # one row over 32-token tiles, 11 groups (one a load)
-    (777, 2048, 4096, 4, 128, False),   # 64-token tiles, x U over 13 row blocks
-    (2049, 768, 2100, 4, 0, True),      # no low-rank term, symmetric, one row over
-    (400, 4096, 14336, 2, 8, True),     # symmetric 2-bit, rank 8
+@pytest.mark.parametrize("M,K,N,bits,rank,sym,tile", [
+    # a 22-row last tile, 8 rows past 2 row blocks, fractional zero-points
+    (150, 14336, 520, 2, 64, False, 32),
+    (150, 14336, 520, 4, 64, False, 64),
+    (1025, 1408, 2048, 2, 40, False, 32),  # one row over, 11 groups (one a load)
+    (777, 2048, 4096, 4, 128, False, 64),  # x U over 13 row blocks
+    (2049, 768, 2100, 4, 0, True, 64),     # no low-rank term, symmetric, one row over
+    (400, 4096, 14336, 2, 8, True, 64),    # symmetric 2-bit, rank 8
+    (17, 128, 40, 2, 8, False, 32),        # one group, one row block
 ], ids=str)
-def test_dense_tile_form(gpu, M, K, N, bits, rank, sym):
-    """The dense launch in tile form (chosen by size): ragged token tiles and
-    row blocks, rows whose zero-points are fractions (their sums of x come from
+def test_dense_tile_form(gpu, monkeypatch, M, K, N, bits, rank, sym, tile):
+    """The dense launch in tile form (GLQ_PF_TILE): ragged token tiles and row
+    blocks, rows whose zero-points are fractions (their sums of x come from
     the launch before), a bias, a = x U formed there or given; the same bits
     on repeated calls (its arrival counters are left at zero)."""
+    assert tile_form(monkeypatch, M, K, N, rank, tile)
+    monkeypatch.setenv("GLQ_PF_TILE", str(tile))
     p = fmt.make_linear(K, N, bits=bits, group=128, rank=max(rank, 8), M=M, seed=M + N, sym=sym)
     if not sym:
         z = p.zeros.float()

@@ -36,7 +36,7 @@ def check(p, out, logits, what):
 
 def test_config3_prefill_512(gpu):
     """BASELINE config 3's prefill: a Mixtral-8x7B-shaped layer over 512 tokens
-    (about 128 tokens per expert: 128-token tiles), LoRA factors x3."""
+    (about 128 tokens per expert: 64-token tiles), LoRA factors x3."""
     p = lora_heavy(fmt.make_mixtral_layer(B=512, seed=42), f=3.0)
     assert margin(p) >= 2
     print("config 3 prefill T=512", flush=True)
@@ -144,7 +144,7 @@ def test_non_integer_shared_zeros_use_decode_steps(gpu):
 
 
 @pytest.mark.parametrize("T,E,top_k,H,inter,bits", [
-    (65, 8, 2, 512, 1024, 2),    # 16 tokens an expert: 32-token tiles, scale quads
+    (65, 8, 2, 512, 1024, 2),    # 16 tokens an expert: 32-token tiles, scale pairs
     (65, 1, 1, 128, 128, 2),     # one expert, one group, one row block
     (129, 4, 2, 512, 640, 4),    # 64 an expert (64-token tiles), 8 and 5 groups, 4-bit
     (160, 4, 2, 1280, 512, 2),   # 80 an expert (128-token tiles), 10 and 4 groups
@@ -152,7 +152,7 @@ def test_non_integer_shared_zeros_use_decode_steps(gpu):
 ], ids=str)
 def test_prefill_tile_edges(gpu, T, E, top_k, H, inter, bits):
     """The tile form's token tiles (by the mean tokens an expert gets) at their
-    edges: ragged last tiles, groups loaded one and four at a time, row blocks
+    edges: ragged last tiles, groups loaded one and two at a time, row blocks
     past the projection's rows."""
     args = dict(H=H, E=E, inter=inter, top_k=top_k, n_clusters=2, rank=24, shared_inter=256,
                 bits=bits)

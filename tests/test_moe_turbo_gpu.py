@@ -352,3 +352,42 @@ def test_turbo_prompt_takes_an_unaligned_rotation(gpu):
     moe_block._turbo_derived(blk.t)
     got, _ = run(blk, p, gpu)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("T,inter,shared", [
+    (40, 1408, 0),     # 11 groups in two splits
+    (40, 2048, 512),   # 16 groups in four, the shared expert in the launches
+    (100, 1536, 0),    # 12 groups in three
+], ids=str)
+def test_turbo_prompt_down_in_splits(gpu, T, inter, shared):
+    """The routed down over K splits: each starts at its own group of codes,
+    the row norms scale every split's sum, the low-rank term comes once, the
+    combine adds them."""
+    import ctypes
+
+    from glorcq_amd import _lib
+
+    kw = dict(H=512, E=6, inter=inter, top_k=2, n_clusters=3, rank=40, shared_inter=shared,
+              rot_gate_up="rht", rot_down="qr")
+    # the fp32 results are the workspace's largest part: more than one split's
+    q = _lib.TurboPrefillParams()
+    q.tokens, q.hidden, q.experts, q.inter, q.top_k = T, 512, 6, inter, 2
+    q.h = q.router_w = q.out = 1 << 12
+    for i in range(3):
+        q.codes[i] = q.norms[i] = q.centroids[i] = 1 << 12
+    q.signs[0], q.Pi[1] = 1 << 12, 1 << 12
+    picks = 2 * T
+    rest = 2 * T * 512 * 2 + 2 * picks * inter * 2 + (1 << 15)
+    splits = (_lib.load().glq_turbo_moe_prefill_workspace_bytes(ctypes.byref(q)) - rest) \
+        / (picks * 512 * 4)
+    assert splits > 1
+    seed = next(s for s in range(3, 60)
+                if margin(fmt.make_turbo_moe(B=T, seed=s, **kw)) >= 2)
+    p = lora_heavy(fmt.make_turbo_moe(B=T, seed=seed, **kw), 10.0)
+    blk = GraphCompatibleMoeBlock.from_problem(p, gpu)
+    res = (torch.randn(1, T, 512, generator=torch.Generator().manual_seed(T)) * 0.5).half()
+    out, logits = blk(p.h.reshape(1, T, 512).to(gpu), residual=res.to(gpu))
+    torch.cuda.synchronize()
+    check_routing(p, logits.cpu())
+    ref = O.moe_forward(p).half().double() + res.reshape(T, 512).double()
+    assert bar(out.reshape(T, 512).cpu(), ref)
