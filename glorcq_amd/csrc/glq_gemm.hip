@@ -1,11 +1,12 @@
-// Prefill entry point glq_gemm_lora: argument checks, then the grouped
-// dequant-to-fp16 MFMA GEMM of glq_prefill.hip in its dense form (one
-// "expert", token rows in order):
-//   launch 1  pf_lowrank_kernel   a = fp16(x U), only when U is given (rank
-//   (+ finalize)                  <= 128; larger ranks take
-//                                 glq_lowrank_xu_batched first)
-//   launch 2  pf_gemm_kernel      y = fp16(x W^T + a SV^T + bias) over tiles
-//                                 sized to the problem, x read as given
+// Prefill entry point glq_gemm_lora: argument checks, the workspace's layout,
+// then the grouped dequant-to-fp16 MFMA GEMM of glq_prefill.hip in its dense
+// form, y = fp16(x W^T + a SV^T + bias), a = fp16(x U):
+//   small tiles  pf_gemm_kernel, one launch: x read as given, a formed by the
+//                launch's first grid rows (pf_xu_job)
+//   tile form    pf_prep_kernel (x in decode order, its group sums, a), then
+//                pf_tile_kernel
+// pt_dense_tile picks the form; ranks past 128 have a formed by
+// glq_lowrank_xu_batched first.
 // Reference: gptq_dequant_gemm_kernel (inference/kernels/gptq_matmul.cu:
 // 111-213, used for B > 4) and the LoRA tail of GLoRCQLinear.forward
 // (inference/quantized_linear.py:338-349).

@@ -1,6 +1,6 @@
 // Prefill GEMM tiles of 64 tokens x 64 weight rows a wave (pf_tile_kernel):
-// the form of the grouped and dense prefill GEMMs for launches that fill the
-// chip (glq_prefill.hip picks it by size; the smaller tiles of pf_gemm_kernel
+// the form of every grouped prefill GEMM and of the dense ones that it runs
+// faster (pt_dense_tile in glq_prefill.hip; the smaller tiles of pf_gemm_kernel
 // take the rest).
 //
 // What bounds this contraction is neither memory nor the matrix cores alone:

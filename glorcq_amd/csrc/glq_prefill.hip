@@ -7,10 +7,11 @@
 // inference/moe_block.py:704-740: each active expert's projections on its
 // gathered tokens).
 //
-// The MoE block's projections run in the tile form of glq_pf_tile.h.
-// pf_gemm_kernel<BITS, TM, RT, MODE, SYM, ZF, DEEP> takes the dense projection:
-// a workgroup of 4 waves owns TM token rows x (4 * 16 RT) weight rows and a
-// range of K.
+// The MoE block's projections, and dense ones where it is the faster form
+// (pt_dense_tile), run in the tile form of glq_pf_tile.h.
+// pf_gemm_kernel<BITS, TM, RT, SYM, ZF, DEEP> takes the other dense ones: a
+// workgroup of 4 waves owns TM token rows x (4 * 16 RT) weight rows and a range
+// of K.
 //  * Per 128-code group one LDS slot receives, by direct global->LDS loads,
 //    the TM rows of A (16-byte piece c of slot row r at c ^ (r % 16), so 16
 //    lanes reading one piece of 16 rows hit 16 distinct bank groups), each
@@ -19,31 +20,30 @@
 //    group (vmcnt), one barrier makes them everyone's and frees the oldest
 //    slot for the next issue.  DEEP rings give half the CU's LDS to one
 //    workgroup (for small launches); others take 2 or 3 slots.
-//  * A: the dense form reads the caller's x in natural order and builds each
-//    MFMA operand in the decode's order with v_perm (pf_nat_a); the MoE forms
-//    read rows that their producers already wrote in decode order
-//    (glq_gemv_core.h perm_src), gathered through an index list.
+//  * A: the caller's x in natural order; each MFMA operand is built in the
+//    decode's order with v_perm (pf_nat_a).
 //  * B: codes decode into exact fp16 MFMA operands q - zi (zi the
 //    zero-point's nearest integer): one v_and_or per code pair lands q under
 //    an exponent chosen per bit position (exactly 2^e + q), one packed fp16
 //    add removes 2^e + zi.  Each group's fp32 MFMA sum is scaled once,
 //    y += s (acc - zf c2), zf = z - zi and c2 the group's sum of x (only for
-//    non-integer zero-points: an MFMA of A against ones in the dense form),
+//    non-integer zero-points: an MFMA of A against ones),
 //    so W = s (q - z) enters exactly, as in the reference's fp32 kernel.
 //    Lane group kb of a wave holds code words 2kb, 2kb+1 (2-bit) or
 //    4kb..4kb+3 (4-bit) of a group; k-step t uses slice t of them.
 //  * v_mfma_f32_16x16x32_f16 with A = 16 token rows, B = 16 weight rows: each
 //    A operand feeds RT MFMAs and each decoded B operand TM/16.
-//  * Split K (ks > 1, the MoE launches): each (tile, split) workgroup writes
-//    an fp32 partial tile; the last of a tile's splits to arrive (a per-tile
-//    counter, left zero again) sums the partials in split order and runs the
-//    epilogue, so the result does not depend on arrival order.
-//  * Epilogues: DENSE y = fp16(acc + a SV^T + bias); GATE/UP inter =
-//    fp16(fp16(silu(fp16 g)) * fp16 u) with each projection's own a SV^T,
-//    stored in the down projection's decode order; DOWN fp32 y + a SV^T.
+//  * Split K (ks > 1; no plan takes it by itself, GLQ_PF_KS asks for it): each
+//    (tile, split) workgroup writes an fp32 partial tile; the last of a tile's
+//    splits to arrive (a per-tile counter, left zero again) sums the partials
+//    in split order and runs the epilogue, so the result does not depend on
+//    arrival order.
+//  * Epilogue: y = fp16(acc + a SV^T + bias).
 //
-// pf_lowrank_kernel: a = x U for the low-rank term (fp32 accumulation, one
-// fp16 rounding), 16 rows per workgroup with U staged in LDS.
+// pf_lowrank_body: a = x U for the low-rank term (fp32 accumulation, one fp16
+// rounding), 64 rows per workgroup with U staged transposed in LDS: the MoE
+// prompts' launches (pf_lowrank_kernel) and the dense tile form's
+// (pf_prep_kernel).
 #include <unistd.h>
 
 #include <algorithm>
@@ -63,8 +63,8 @@ enum PfMode { kPfDense = 0, kPfGateUp = 1, kPfDown = 2 };
 constexpr int kPfThreads = 256;  // 4 waves
 
 struct PfArgs {
-  const __half* xp;          // A rows in decode order, K halves each
-  const int32_t* arow;       // A row of sorted row p (null: p)
+  const __half* xp;          // A rows, K halves each: in decode order (tile form) or natural
+  const int32_t* arow;       // tile form: A row of sorted row p (null: p)
   const uint32_t* codes[2];  // matrix m: (E, N, kw) words
   const __half* scales[2];   // (E, N, G)
   const __half* zeros[2];    // (E, N, G) (unused with SYM)
@@ -81,11 +81,11 @@ struct PfArgs {
   int64_t y_ld;
   float* yf;                 // DOWN: (rows, N) fp32
   int64_t yf_ld, yf_ss;      // and elements between its K splits (tile form)
-  const float* c2;           // ZF: per (group, row) sum of x, (G, c2_ld) fp32
+  const float* c2;           // tile form, ZF: per (group, row) sum of x, (G, c2_ld) fp32
   int64_t c2_ld;
-  float* part;               // split-K partial tiles (ks, tiles, TM, ntn*WGROWS) fp32, or null
+  float* part;               // pf_gemm_kernel: split-K partial tiles (ks, tiles, TM, ntn*WGR) fp32
   unsigned* cnt;             // split-K arrival counters (tiles * ntn), zero between launches
-  const int32_t* tiles;      // (max_tiles, 3): expert, first sorted row, rows; null: dense
+  const int32_t* tiles;      // tile form: (max_tiles, 3): expert, first sorted row, rows; null: dense
   const int32_t* ntiles;     // device count of valid tiles
   int M, K, N, G, kw, rank;
   int ntn;                   // weight-row tiles of a workgroup along N
@@ -315,13 +315,10 @@ __device__ __forceinline__ f16x8 pf_nat_a(const unsigned char* row, int kb, int 
 
 // Weight row of row tile rt of a wave (see the file comment); may be >= N
 // (clamp for loads).
-template <int RT, int MODE>
+template <int RT>
 __device__ __forceinline__ int pf_row(int n0, int wave, int rt, int li) {
-  if constexpr (MODE == kPfGateUp) return n0 + wave * (8 * RT) + (rt % (RT / 2)) * 16 + li;
-  else return n0 + wave * (16 * RT) + rt * 16 + li;
+  return n0 + wave * (16 * RT) + rt * 16 + li;
 }
-template <int RT, int MODE>
-constexpr int pf_wg_rows() { return MODE == kPfGateUp ? 4 * 8 * RT : 4 * 16 * RT; }
 
 // LDS slot of one group: A (TM token rows x 256 B, swizzled pieces), then per
 // wave its RT row tiles' codes (16 rows x CB bytes each, padded to whole
@@ -348,15 +345,13 @@ struct PfSlot {
                                 : (2 * 3 * BYTES <= 160 * 1024 ? 3 : 2);
 };
 
-template <int BITS, int TM, int RT, int MODE, bool SYM, bool ZF, bool DEEP>
+template <int BITS, int TM, int RT, bool SYM, bool ZF, bool DEEP>
 __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
   extern __shared__ __align__(16) unsigned char smem[];
   using SL = PfSlot<BITS, TM, RT, DEEP>;
   constexpr int TT = TM / 16;
   constexpr int XI = TM / 16;  // A load instructions per wave per group (4 rows each)
-  constexpr int WGR = pf_wg_rows<RT, MODE>();
-  constexpr int NMAT = MODE == kPfGateUp ? 2 : 1;
-  constexpr bool NAT = MODE == kPfDense;  // A rows in natural order (the caller's x)
+  constexpr int WGR = 4 * 16 * RT;
   constexpr int D = SL::D;
   constexpr int NI = XI + SL::NC + 1 + (SYM ? 0 : 1);  // loads per lane per group
   const int tid = threadIdx.x, lane = tid & 63;
@@ -369,16 +364,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
     return;
   }
   const int ty = blockIdx.y - g.xu_rows;
-  int e = 0, p0, rows;
-  if (g.tiles) {
-    if (ty >= *g.ntiles) return;  // uniform over the workgroup
-    e = g.tiles[3 * ty];
-    p0 = g.tiles[3 * ty + 1];
-    rows = g.tiles[3 * ty + 2];
-  } else {
-    p0 = ty * TM;
-    rows = min(TM, g.M - p0);
-  }
+  const int p0 = ty * TM, rows = min(TM, g.M - p0);
   const int tn = blockIdx.x % g.ntn, sp = blockIdx.x / g.ntn;
   const int n0 = tn * WGR;
   const int g0 = sp * g.gps, g1 = min(g0 + g.gps, g.G);
@@ -390,59 +376,40 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
 #pragma unroll
   for (int q = 0; q < XI; ++q) {
     const int r = (wave * XI + q) * 4 + (lane >> 4);
-    const int p = p0 + min(r, rows - 1);
-    const int ar = g.arow ? g.arow[p] : p;
-    aoff[q] = ar * g.K + (((lane & 15) ^ (r & 15)) << 3);
+    aoff[q] = (p0 + min(r, rows - 1)) * g.K + (((lane & 15) ^ (r & 15)) << 3);
   }
-  const uint32_t* cb[NMAT];
-  const __half* sb[NMAT];
-  const __half* zb[NMAT];
-#pragma unroll
-  for (int m = 0; m < NMAT; ++m) {
-    cb[m] = g.codes[m] + e * g.codes_es + (int64_t)n0 * g.kw;
-    sb[m] = g.scales[m] + e * g.sz_es + (int64_t)n0 * g.G;
-    zb[m] = SYM ? sb[m] : g.zeros[m] + e * g.sz_es + (int64_t)n0 * g.G;
-  }
+  const uint32_t* cb = g.codes[0] + (int64_t)n0 * g.kw;
+  const __half* sb = g.scales[0] + (int64_t)n0 * g.G;
+  const __half* zb = SYM ? sb : g.zeros[0] + (int64_t)n0 * g.G;
   // codes: instruction q covers bytes q*1024 + 16*lane of the wave's region
   // (lanes past the wave's code bytes re-load its first ones into the padding)
-  int coff[SL::NC], cmat[SL::NC];
+  int coff[SL::NC];
 #pragma unroll
   for (int q = 0; q < SL::NC; ++q) {
     const int o = (q * 1024 + 16 * lane) % SL::CW;
     const int rt = o / (16 * SL::CB), row = (o % (16 * SL::CB)) / SL::CB;
     const int piece = (o % SL::CB) / 16;
-    const int n = min(pf_row<RT, MODE>(n0, wave, rt, row), g.N - 1);
+    const int n = min(pf_row<RT>(n0, wave, rt, row), g.N - 1);
     coff[q] = (n - n0) * g.kw + 4 * piece;
-    cmat[q] = MODE == kPfGateUp ? rt / (RT / 2) : 0;
   }
   // scales / zero-points: lane -> (row tile lane/16, row lane%16)
-  int soff, smat;
-  {
-    const int rt = min(lane >> 4, RT - 1);
-    const int n = min(pf_row<RT, MODE>(n0, wave, rt, lane & 15), g.N - 1);
-    soff = (n - n0) * g.G;
-    smat = MODE == kPfGateUp ? rt / (RT / 2) : 0;
-  }
+  const int soff =
+      (min(pf_row<RT>(n0, wave, min(lane >> 4, RT - 1), lane & 15), g.N - 1) - n0) * g.G;
   auto issue = [&](int grp, unsigned char* slot) {
 #pragma unroll
     for (int q = 0; q < XI; ++q)
       __builtin_amdgcn_global_load_lds((const void*)(g.xp + aoff[q] + grp * 128),
                                        (lds_void*)(slot + SL::A + (wave * XI + q) * 1024), 16, 0, 0);
 #pragma unroll
-    for (int q = 0; q < SL::NC; ++q) {
-      const uint32_t* base = NMAT == 2 && cmat[q] ? cb[NMAT - 1] : cb[0];
-      __builtin_amdgcn_global_load_lds((const void*)(base + coff[q] + grp * (SL::CB / 4)),
+    for (int q = 0; q < SL::NC; ++q)
+      __builtin_amdgcn_global_load_lds((const void*)(cb + coff[q] + grp * (SL::CB / 4)),
                                        (lds_void*)(slot + SL::C + wave * SL::CR + q * 1024),
                                        16, 0, 0);
-    }
-    const __half* sbase = NMAT == 2 && smat ? sb[NMAT - 1] : sb[0];
-    __builtin_amdgcn_global_load_lds((const void*)(sbase + soff + grp),
+    __builtin_amdgcn_global_load_lds((const void*)(sb + soff + grp),
                                      (lds_void*)(slot + SL::S + wave * 256), 2, 0, 0);
-    if constexpr (!SYM) {
-      const __half* zbase = NMAT == 2 && smat ? zb[NMAT - 1] : zb[0];
-      __builtin_amdgcn_global_load_lds((const void*)(zbase + soff + grp),
+    if constexpr (!SYM)
+      __builtin_amdgcn_global_load_lds((const void*)(zb + soff + grp),
                                        (lds_void*)(slot + SL::Z + wave * 256), 2, 0, 0);
-    }
   };
 
   f32x4 y[TT][RT];
@@ -484,10 +451,8 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
       kc[rt] = pf_consts<BITS, SYM>(sh, zh, g.zoff);
     }
     // the group's sum of x (q - zi), fp32
-    auto a_op = [&](int i, int t) -> f16x8 {
-      const unsigned char* row = sl + SL::A + (16 * i + li) * 256;
-      if constexpr (NAT) return pf_nat_a<BITS>(row, kb, t, li);
-      else return *(const f16x8*)(row + (((4 * kb + t) ^ li) << 4));
+    auto a_op = [&](int i, int t) {
+      return pf_nat_a<BITS>(sl + SL::A + (16 * i + li) * 256, kb, t, li);
     };
     f32x4 acc[TT][RT];
 #pragma unroll
@@ -504,11 +469,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
       }
     }
     // y += s (acc - zf c2): c2 = the group's sum of x per token, needed only
-    // for non-integer zero-points (zf != 0); natural-order A forms it here
-    // (an MFMA against ones, when any row of the wave has zf != 0), the
-    // decode-order A of the MoE forms reads it from g.c2
+    // for non-integer zero-points (zf != 0): an MFMA against ones when any row
+    // of the wave has one
     f32x4 c2v[TT];
-    if constexpr (ZF && NAT) {
+    if constexpr (ZF) {
       bool any = false;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) any |= kc[rt].zf != 0.f;
@@ -530,18 +494,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
         const float zf = kc[rt].zf;
 #pragma unroll
         for (int i = 0; i < TT; ++i) {
-          float4 c2;
-          if constexpr (NAT) {
-            c2 = float4{c2v[i][0], c2v[i][1], c2v[i][2], c2v[i][3]};
-          } else {
-            // rows past the tile's last are read (the layout has whole
-            // tiles) and never stored
-            c2 = *(const float4*)(g.c2 + (int64_t)grp * g.c2_ld + p0 + 16 * i + 4 * kb);
-          }
-          y[i][rt][0] = fmaf(s, acc[i][rt][0] - zf * c2.x, y[i][rt][0]);
-          y[i][rt][1] = fmaf(s, acc[i][rt][1] - zf * c2.y, y[i][rt][1]);
-          y[i][rt][2] = fmaf(s, acc[i][rt][2] - zf * c2.z, y[i][rt][2]);
-          y[i][rt][3] = fmaf(s, acc[i][rt][3] - zf * c2.w, y[i][rt][3]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            y[i][rt][j] = fmaf(s, acc[i][rt][j] - zf * c2v[i][j], y[i][rt][j]);
         }
       } else {
 #pragma unroll
@@ -552,7 +507,6 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
     }
   }
   wait_vmcnt<0>();  // the tail's loads land before the workgroup's LDS goes away
-
 
   // ---- split K: partial tiles, the last split of a tile reduces ----
   if (g.ks > 1) {
@@ -596,70 +550,42 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(PfArgs g) {
   // ---- low-rank term: y += a SV^T (a: token rows, SV: weight rows) ----
   if (g.xu_rows && g.rank > 0) pf_xu_wait(g, p0, rows, smem, &xflag);
   if (g.a != nullptr && g.rank > 0) {
-    constexpr int RM = RT / NMAT;  // row tiles per matrix
     for (int j0 = 0; j0 < g.rank; j0 += 32) {
       const int jk = j0 + 8 * kb;
       const bool jv = jk < g.rank;
+      f16x8 bv[RT];
 #pragma unroll
-      for (int m = 0; m < NMAT; ++m) {
-        f16x8 bv[RM];
+      for (int rt = 0; rt < RT; ++rt) {
+        const int n = min(pf_row<RT>(n0, wave, rt, li), g.N - 1);
+        bv[rt] = jv ? *(const f16x8*)(g.sv[0] + (int64_t)n * g.rank + jk) : f16x8{};
+      }
 #pragma unroll
-        for (int q = 0; q < RM; ++q) {
-          const int rt = m * RM + q;
-          const int n = min(pf_row<RT, MODE>(n0, wave, rt, li), g.N - 1);
-          bv[q] = jv ? *(const f16x8*)(g.sv[m] + e * g.sv_es + (int64_t)n * g.rank + jk)
-                     : f16x8{};
+      for (int i = 0; i < TT; ++i) {
+        const int p = p0 + min(16 * i + li, rows - 1);
+        f16x8 av = f16x8{};
+        if (jv) {
+          const __half* ap = g.a + (int64_t)p * g.a_ld + jk;
+          av = g.xu_rows ? pf_load8_coh(ap) : *(const f16x8*)ap;
         }
 #pragma unroll
-        for (int i = 0; i < TT; ++i) {
-          const int p = p0 + min(16 * i + li, rows - 1);
-          f16x8 av = f16x8{};
-          if (jv) {
-            const __half* ap = g.a + (int64_t)p * g.a_ld + m * g.rank + jk;
-            av = g.xu_rows ? pf_load8_coh(ap) : *(const f16x8*)ap;
-          }
-#pragma unroll
-          for (int q = 0; q < RM; ++q) y[i][m * RM + q] = mfma_16x16x32(av, bv[q], y[i][m * RM + q]);
-        }
+        for (int rt = 0; rt < RT; ++rt) y[i][rt] = mfma_16x16x32(av, bv[rt], y[i][rt]);
       }
     }
   }
 
   // ---- stores: lane holds tokens 16i + 4kb + j of weight row li ----
-  if constexpr (MODE == kPfGateUp) {
-    constexpr int H2 = RT / 2;
 #pragma unroll
-    for (int rt = 0; rt < H2; ++rt) {
-      const int n = pf_row<RT, MODE>(n0, wave, rt, li);
-      if (n >= g.N) continue;
-      const int col = (n & ~15) + perm_pos_rt(g.out_bits, n & 15);
+  for (int rt = 0; rt < RT; ++rt) {
+    const int n = pf_row<RT>(n0, wave, rt, li);
+    if (n >= g.N) continue;
+    const float bn = g.bias ? __half2float(g.bias[n]) : 0.f;
 #pragma unroll
-      for (int i = 0; i < TT; ++i)
+    for (int i = 0; i < TT; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int r = 16 * i + 4 * kb + j;
-          if (r < rows)
-            g.y[(int64_t)(p0 + r) * g.y_ld + col] = swiglu_fp16(y[i][rt][j], y[i][rt + H2][j]);
-        }
-    }
-  } else {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int n = pf_row<RT, MODE>(n0, wave, rt, li);
-      if (n >= g.N) continue;
-      const float bn = (MODE == kPfDense && g.bias) ? __half2float(g.bias[n]) : 0.f;
-#pragma unroll
-      for (int i = 0; i < TT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int r = 16 * i + 4 * kb + j;
-          if (r >= rows) continue;
-          if constexpr (MODE == kPfDense)
-            g.y[(int64_t)(p0 + r) * g.y_ld + n] = __float2half(y[i][rt][j] + bn);
-          else
-            g.yf[(int64_t)(p0 + r) * g.yf_ld + n] = y[i][rt][j];
-        }
-    }
+      for (int j = 0; j < 4; ++j) {
+        const int r = 16 * i + 4 * kb + j;
+        if (r < rows) g.y[(int64_t)(p0 + r) * g.y_ld + n] = __float2half(y[i][rt][j] + bn);
+      }
   }
   if (g.xu_rows && g.rank > 0) {  // the workgroup has read a of its rows' blocks
     __syncthreads();
@@ -1033,16 +959,16 @@ __global__ __launch_bounds__(kPfThreads) void pf_prep_kernel(PfPrep p) {
 // Host side shared by the dense GEMM and the MoE prefill
 // ---------------------------------------------------------------------------
 
-template <int BITS, int TM, int RT, int MODE, bool SYM, bool ZF, bool DEEP = false>
+template <int BITS, int TM, int RT, bool SYM, bool ZF, bool DEEP = false>
 static int pf_launch_k(const PfArgs& g, hipStream_t s) {
   static size_t attr = 64 * 1024;
   using SL = PfSlot<BITS, TM, RT, DEEP>;
   size_t lds = (size_t)SL::D * SL::BYTES;
   if (g.xu_rows) lds = std::max(lds, kXuJobLds);  // the x U jobs and the epilogue's local form
-  int rc = set_lds_limit(pf_gemm_kernel<BITS, TM, RT, MODE, SYM, ZF, DEEP>, lds, attr);
+  int rc = set_lds_limit(pf_gemm_kernel<BITS, TM, RT, SYM, ZF, DEEP>, lds, attr);
   if (rc) return rc;
   const dim3 grid((unsigned)(g.ntn * g.ks), (unsigned)(g.max_tiles + g.xu_rows));
-  pf_gemm_kernel<BITS, TM, RT, MODE, SYM, ZF, DEEP><<<grid, dim3(kPfThreads), lds, s>>>(g);
+  pf_gemm_kernel<BITS, TM, RT, SYM, ZF, DEEP><<<grid, dim3(kPfThreads), lds, s>>>(g);
   GLQ_LAUNCH_CHECK("pf_gemm_kernel");
   return GLQ_OK;
 }
@@ -1057,18 +983,18 @@ template <int BITS, bool SYM, bool ZF>
 static int pf_launch_dense_bits(const PfArgs& g, PfTile t, hipStream_t s) {
   if (t.deep) {
     if (t.tm == 16) {
-      if (t.rt == 1) return pf_launch_k<BITS, 16, 1, kPfDense, SYM, ZF, true>(g, s);
-      return pf_launch_k<BITS, 16, 2, kPfDense, SYM, ZF, true>(g, s);
+      if (t.rt == 1) return pf_launch_k<BITS, 16, 1, SYM, ZF, true>(g, s);
+      return pf_launch_k<BITS, 16, 2, SYM, ZF, true>(g, s);
     }
     if (t.tm == 32) {
-      if (t.rt == 1) return pf_launch_k<BITS, 32, 1, kPfDense, SYM, ZF, true>(g, s);
-      return pf_launch_k<BITS, 32, 2, kPfDense, SYM, ZF, true>(g, s);
+      if (t.rt == 1) return pf_launch_k<BITS, 32, 1, SYM, ZF, true>(g, s);
+      return pf_launch_k<BITS, 32, 2, SYM, ZF, true>(g, s);
     }
-    return pf_launch_k<BITS, 64, 2, kPfDense, SYM, ZF, true>(g, s);
+    return pf_launch_k<BITS, 64, 2, SYM, ZF, true>(g, s);
   }
-  if (t.tm == 128) return pf_launch_k<BITS, 128, 2, kPfDense, SYM, ZF>(g, s);
-  if (t.tm == 64) return pf_launch_k<BITS, 64, 2, kPfDense, SYM, ZF>(g, s);
-  return pf_launch_k<BITS, 32, 4, kPfDense, SYM, ZF>(g, s);
+  if (t.tm == 128) return pf_launch_k<BITS, 128, 2, SYM, ZF>(g, s);
+  if (t.tm == 64) return pf_launch_k<BITS, 64, 2, SYM, ZF>(g, s);
+  return pf_launch_k<BITS, 32, 4, SYM, ZF>(g, s);
 }
 
 static int pf_launch_dense(const PfArgs& g, int bits, PfTile t, bool sym, hipStream_t s) {
@@ -1561,11 +1487,12 @@ namespace glq {
 //   2. pf_moe_dispatch_kernel  per-expert counts and positions: the pairs
 //                              (token, pick) sorted by expert, and the list of
 //                              TM-row tiles (expert, first row, rows)
-//   3. pf_lowrank_kernel (+ finalize)  a = x U_c(e) for gate and up per pair
-//   4. pf_gemm_kernel GATE/UP  inter = SwiGLU per pair (down's decode order)
-//   5. pf_lowrank_kernel (+ finalize)  a = inter U_down,c(e) per pair
-//   6. pf_gemm_kernel DOWN     y per pair (fp32)
-//   7. shared expert (dense GATE/UP, DOWN over all tokens), when present
+//   3. pf_lowrank_kernel       a = x U_c(e) for gate and up per pair
+//   4. tile form GATE/UP       inter = SwiGLU per pair (down's decode order)
+//   5. pf_lowrank_kernel       a = inter U_down,c(e) per pair
+//   6. tile form DOWN          y per pair (fp32, in K splits)
+//   7. shared expert (GATE/UP, DOWN over all tokens), when present: riding in 4
+//      and 6 as a pair launch, or two launches of its own
 //   8. pf_moe_combine_kernel   out = fp16(sum_k w_k y_k + sg fp16(shared))
 //                              (+ residual)
 // Rows within an expert come in the order of an atomic counter, but every
