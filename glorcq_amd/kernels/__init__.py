@@ -288,10 +288,10 @@ def _packed_dequant_matmul_eager(x: torch.Tensor, codes: torch.Tensor, scales: t
         r = rank if precomputed_xU is None else 0
         nbytes = lib.glq_gemm_workspace_bytes(M, K, N, r)
         # (the arrival counters are x U's: without it the call leaves nothing in
-        # its workspace, and takes one of its own, so that captured calls of one
-        # stream may be replayed on several)
-        ws = (gemm_workspace(x.device, nbytes) if r else
-              torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=x.device))
+        # its workspace, and takes one of its own where it needs any, so that
+        # captured calls of one stream may be replayed on several)
+        ws = (torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes and not r else
+              gemm_workspace(x.device, nbytes))
         rc = lib.glq_gemm_lora(
             x.data_ptr(), M, K, N, codes.data_ptr(), bits, scales.data_ptr(), _lib.ptr(zeros),
             groupsize, _sym_mode(sym), _lib.ptr(U if precomputed_xU is None else None),
