@@ -237,7 +237,8 @@ def _packed_dequant_matmul_eager(x: torch.Tensor, codes: torch.Tensor, scales: t
     _require(x, "x", torch.float16)
     _require(codes, "codes", torch.int32)
     _require(scales, "scales", torch.float16)
-    asym = _sym_mode(sym) != SYM_SIGNED
+    mode = _sym_mode(sym)
+    asym = mode != SYM_SIGNED
     if asym:
         if zeros is None:
             raise RuntimeError("zeros required for asymmetric codes")
@@ -294,7 +295,7 @@ def _packed_dequant_matmul_eager(x: torch.Tensor, codes: torch.Tensor, scales: t
               gemm_workspace(x.device, nbytes))
         rc = lib.glq_gemm_lora(
             x.data_ptr(), M, K, N, codes.data_ptr(), bits, scales.data_ptr(), _lib.ptr(zeros),
-            groupsize, _sym_mode(sym), _lib.ptr(U if precomputed_xU is None else None),
+            groupsize, mode, _lib.ptr(U if precomputed_xU is None else None),
             _lib.ptr(SV), rank, _lib.ptr(precomputed_xU), _lib.ptr(bias), out.data_ptr(),
             ws.data_ptr(), ws.numel(), stream)
         _lib.check(rc, "glq_gemm_lora")
@@ -307,7 +308,7 @@ def _packed_dequant_matmul_eager(x: torch.Tensor, codes: torch.Tensor, scales: t
         xu = None if precomputed_xU is None else precomputed_xU[m0:m1]
         rc = lib.glq_gemv_lora(
             x[m0:m1].data_ptr(), mb, K, N, codes.data_ptr(), bits, scales.data_ptr(),
-            _lib.ptr(zeros), groupsize, _sym_mode(sym),
+            _lib.ptr(zeros), groupsize, mode,
             _lib.ptr(U if precomputed_xU is None else None), _lib.ptr(SV), rank,
             _lib.ptr(xu), _lib.ptr(bias), out[m0:m1].data_ptr(),
             ws.data_ptr(), ws.numel(), stream)
