@@ -228,12 +228,14 @@ int glq_lowrank_xu_routed(int64_t picks, const void* x, int64_t K, const void* U
  * reference's gptq_dequant_gemm_kernel path (inference/kernels/gptq_matmul.cu:
  * 111-213, taken for B > 4) and the LoRA tail of GLoRCQLinear.forward
  * (inference/quantized_linear.py:338-349).  Group 128.  Codes decode into
- * exact fp16 operands (q - zero-point's integer part) of
- * v_mfma_f32_16x16x32_f16, each group's fp32 sum scaled once (any zero-point,
- * symmetric or not); a = fp16(x U) comes from xU or from a low-rank launch
- * before the GEMM (rank <= 128: one launch whose 16-row blocks' K slices
- * hand their partial sums to the block's last arriving slice).
- * The workspace (glq_gemm_workspace_bytes, 256-byte aligned) is required.
+ * exact fp16 operands (q - zero-point's integer part) of MFMAs, each group's
+ * fp32 sum scaled once (any zero-point, symmetric or not); a = fp16(x U) comes
+ * from xU, from the GEMM's own launch or the one before it (rank <= 128), or
+ * from the low-rank entry point.  Two forms by size: small tiles, and wide
+ * ones over x put in order by a launch before.
+ * The workspace (glq_gemm_workspace_bytes, 256-byte aligned) is required; one
+ * that holds only what the small tiles need (4096 bytes of counters, a and its
+ * partials; nothing without a U) is taken, by those.
  * When U is given (no xU) its first 4096 bytes are arrival counters: they
  * must be zero before the workspace's first use with glq_gemm_lora (allocate
  * it zero-filled) and every call leaves them zero; do not share the buffer

@@ -242,7 +242,7 @@ def test_config1_down_m512(gpu):
 @pytest.mark.gpu
 @pytest.mark.parametrize("bits", [2, 4])
 def test_large_prefill_tiles(gpu, bits):
-    """M = 1024 over K = 4096 (128-token tiles for 2-bit, one K split)."""
+    """M = 1024 over K = 4096, by the form that the size takes."""
     p = fmt.make_linear(4096, 1024, bits=bits, group=128, rank=64, M=1024, seed=77 + bits)
     d = to(p, gpu)
     y = K_.packed_dequant_matmul_fused(d["x"], d["codes"], d["scales"], d["zeros"], bits, 128,
